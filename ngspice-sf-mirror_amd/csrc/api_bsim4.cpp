@@ -16,6 +16,8 @@
 #include "ngmi_internal.h"
 #include "bsim4_setup.h"
 #include "bsim4_eval.h"
+#include "bsim4_dev.h"
+#include "set_table.h"
 
 namespace ngmi {
 int launch_bsim4_eval(const B4Tab &tab, const B4Ckt &ck, const double *vterm,
@@ -52,26 +54,147 @@ struct ngmi_bsim4_set {
     std::vector<double> rows;                 /* n x B4F__COUNT, after finalize */
     std::vector<int> code;
     int icols = 0, mcols = 0;
-    double *d_itab = nullptr, *d_mtab = nullptr;
-    int *d_model_of = nullptr, *d_code = nullptr;
+    SetRecords recs;
+    std::vector<void *> dev;                  /* device buffers */
     size_t dev_bytes = 0;
     B4Tab tab{};
     bool final_ = false;
 
     void release()
     {
-        (void)hipFree(d_itab);
-        (void)hipFree(d_mtab);
-        (void)hipFree(d_model_of);
-        (void)hipFree(d_code);
-        d_itab = d_mtab = nullptr;
-        d_model_of = d_code = nullptr;
+        for (void *p : dev) (void)hipFree(p);
+        dev.clear();
+        dev_bytes = 0;
+    }
+    template <class T>
+    int upload(const std::vector<T> &v, const T **out)
+    {
+        const size_t bytes = std::max<size_t>(v.size(), 1) * sizeof(T);
+        void *p = nullptr;
+        NGMI_HIP(hipMalloc(&p, bytes));
+        dev.push_back(p);
+        dev_bytes += bytes;
+        if (!v.empty()) NGMI_HIP(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+        *out = static_cast<const T *>(p);
+        return NGMI_OK;
     }
 };
 
 namespace ngmi {
+
 const B4Tab *set_table(const ngmi_bsim4_set *s) { return s && s->final_ ? &s->tab : nullptr; }
+
+const SetRecords *set_records(const ngmi_bsim4_set *s) { return s && s->final_ ? &s->recs : nullptr; }
+
+void set_tiles(const ngmi_bsim4_set *s, const std::vector<int> &at, std::vector<double> &tiles)
+{
+    const size_t ntile = (at.size() + B4_TILE - 1) / B4_TILE;
+    const int nc = B4_NC_GEOM;
+    tiles.assign(ntile * B4_TILE * (size_t)nc, 0.0);
+    for (size_t i = 0; i < at.size(); i++) {
+        if (at[i] < 0) continue;
+        const double *row = &s->rows[(size_t)at[i] * B4F__COUNT];
+        double *t = &tiles[(i / B4_TILE) * B4_TILE * nc + i % B4_TILE];
+        for (int c = 0; c < nc; c++) t[(size_t)c * B4_TILE] = row[B4_IFIELDS[c]];
+    }
 }
+
+/* the set's records: instances of one model card that differ only in the
+ * per-instance fields share one, equal ones of several cards too */
+static void build_records(const std::vector<double> &rows, const std::vector<int> &model_of, int nm,
+                          const std::vector<char> &perinst, SetRecords &R)
+{
+    const size_t n = model_of.size();
+    const int F = B4F__COUNT;
+    R = SetRecords();
+    std::vector<int> extra;   /* fields that vary within a card beyond the per-instance list */
+    for (int f = 0; f < F; f++) {
+        if (!perinst[f]) continue;
+        if (B4_ICOL[f] < B4_NC_LD) R.nc = std::max(R.nc, B4_NC_LD);
+        else if (B4_ICOL[f] < B4_NC_GEOM) R.nc = B4_NC_GEOM;
+        else extra.push_back(f);
+    }
+    /* a card, or a card at one set of extra values, is a candidate; equal
+     * candidates (in the fields read from records) are one record */
+    auto hash = [](uint64_t h, uint64_t v) { return (h ^ v) * 0x9E3779B97F4A7C15ull + (h >> 29); };
+    auto bits = [](double v) { uint64_t u; std::memcpy(&u, &v, 8); return u; };
+    std::unordered_multimap<uint64_t, size_t> cand;      /* hash -> first instance of a candidate */
+    std::unordered_multimap<uint64_t, int> by_content;   /* hash -> record */
+    std::vector<int> cand_rec(n, -1), of_model(nm, -1);
+    std::vector<size_t> rec_inst;
+    R.rec_of.assign(n, -1);
+    auto record_of = [&](size_t k) {
+        const double *row = &rows[k * F];
+        uint64_t h = 1;
+        for (int f = 0; f < F; f++)
+            if (B4_ICOL[f] >= R.nc) h = hash(h, bits(row[f]));
+        const auto rg = by_content.equal_range(h);
+        for (auto it = rg.first; it != rg.second; ++it) {
+            const double *o = &rows[rec_inst[it->second] * F];
+            bool same = true;
+            for (int f = 0; f < F && same; f++)
+                if (B4_ICOL[f] >= R.nc) same = bits(row[f]) == bits(o[f]);
+            if (same) return it->second;
+        }
+        const int r = (int)rec_inst.size();
+        rec_inst.push_back(k);
+        by_content.emplace(h, r);
+        return r;
+    };
+    /* more records than this are no cheaper to read than columns */
+    const size_t most = std::max<size_t>(4096, n / 8);
+    for (size_t k = 0; k < n; k++) {
+        int r = -1;
+        if (extra.empty()) {
+            int &m = of_model[model_of[k]];
+            if (m < 0) m = record_of(k);
+            r = m;
+        } else {
+            const double *row = &rows[k * F];
+            uint64_t h = hash(2, (uint64_t)model_of[k]);
+            for (int f : extra) h = hash(h, bits(row[f]));
+            const auto rg = cand.equal_range(h);
+            for (auto it = rg.first; it != rg.second && r < 0; ++it) {
+                const double *o = &rows[it->second * F];
+                bool same = model_of[it->second] == model_of[k];
+                for (int f : extra) same = same && bits(row[f]) == bits(o[f]);
+                if (same) r = cand_rec[it->second];
+            }
+            if (r < 0) {
+                r = cand_rec[k] = record_of(k);
+                cand.emplace(h, k);
+            }
+        }
+        if (rec_inst.size() > most) {
+            R.rec_of.clear();
+            return;
+        }
+        R.rec_of[k] = r;
+    }
+    R.rec.resize(rec_inst.size() * F);
+    for (size_t r = 0; r < rec_inst.size(); r++)
+        std::copy(&rows[rec_inst[r] * F], &rows[rec_inst[r] * F] + F, &R.rec[r * F]);
+    R.ok = true;
+}
+
+/* items (tile, record) over the tiles of `at`'s records: a tile is listed
+ * once for each record among its lanes */
+static void build_items(const std::vector<int> &rec_of, std::vector<int> &items)
+{
+    for (size_t t = 0; t * B4_TILE < rec_of.size(); t++) {
+        const size_t b = t * B4_TILE, e = std::min(rec_of.size(), b + B4_TILE), i0 = items.size();
+        for (size_t k = b; k < e; k++) {
+            bool seen = false;
+            for (size_t q = i0; q < items.size() && !seen; q += 2) seen = items[q + 1] == rec_of[k];
+            if (!seen) {
+                items.push_back((int)t);
+                items.push_back(rec_of[k]);
+            }
+        }
+    }
+}
+
+}  // namespace ngmi
 
 extern "C" {
 
@@ -178,9 +301,13 @@ int ngmi_bsim4_set_add(ngmi_bsim4_set *s, ngmi_bsim4_model *const *models, int n
     return first;
 }
 
-int ngmi_bsim4_set_finalize(ngmi_bsim4_set *s)
+}  // extern "C"
+
+namespace ngmi {
+
+/* resolves every instance and splits the columns; no device work */
+static int set_resolve(ngmi_bsim4_set *s)
 {
-    if (!s) return NGMI_E_PANIC;
     const size_t n = s->inst.size();
     const int F = B4F__COUNT;
     const int nm = (int)s->models.size();
@@ -233,6 +360,27 @@ int ngmi_bsim4_set_finalize(ngmi_bsim4_set *s)
     s->code.assign(F, 0);
     s->icols = s->mcols = 0;
     for (int f = 0; f < F; f++) s->code[f] = perinst[f] ? s->icols++ : ~(s->mcols++);
+    build_records(s->rows, s->model_of, nm, perinst, s->recs);
+    /* one selector word for the whole set lets the kernels compile the
+     * selectors as constants */
+    s->tab = B4Tab{};
+    s->tab.flags = n ? (int)s->rows[B4F_flags] : -1;
+    for (size_t k = 1; k < n && s->tab.flags >= 0; k++)
+        if ((int)s->rows[k * F + B4F_flags] != s->tab.flags) s->tab.flags = -1;
+    s->tab.n = (int64_t)n;
+    s->tab.nm = nm;
+    s->tab.mcols = s->mcols;
+    s->final_ = true;
+    return NGMI_OK;
+}
+
+int set_upload_columns(ngmi_bsim4_set *s)
+{
+    const size_t n = s->inst.size();
+    const int F = B4F__COUNT, nm = (int)s->models.size();
+    std::vector<size_t> firstOf(nm, (size_t)-1);
+    for (size_t k = 0; k < n; k++)
+        if (firstOf[s->model_of[k]] == (size_t)-1) firstOf[s->model_of[k]] = k;
     std::vector<double> itab((size_t)s->icols * n), mtab((size_t)s->mcols * std::max(nm, 1));
     for (int f = 0; f < F; f++) {
         if (s->code[f] >= 0) {
@@ -242,34 +390,55 @@ int ngmi_bsim4_set_finalize(ngmi_bsim4_set *s)
             /* model-major: one card's per-model values are contiguous, so
              * the few cards a workgroup reads stay in its L1 */
             for (int m = 0; m < nm; m++)
-                mtab[(size_t)m * s->mcols + (~s->code[f])] = s->rows[firstOf[m] * F + f];
+                if (firstOf[m] != (size_t)-1) mtab[(size_t)m * s->mcols + (~s->code[f])] = s->rows[firstOf[m] * F + f];
         }
     }
-    /* one selector word for the whole set lets the kernels compile the
-     * selectors as constants */
-    s->tab.flags = n ? (int)s->rows[B4F_flags] : -1;
-    for (size_t k = 1; k < n && s->tab.flags >= 0; k++)
-        if ((int)s->rows[k * F + B4F_flags] != s->tab.flags) s->tab.flags = -1;
-    s->release();
-    const size_t bi = std::max<size_t>(itab.size(), 1) * sizeof(double);
-    const size_t bm = std::max<size_t>(mtab.size(), 1) * sizeof(double);
-    const size_t bo = std::max<size_t>(n, 1) * sizeof(int);
-    NGMI_HIP(hipMalloc(&s->d_itab, bi));
-    NGMI_HIP(hipMalloc(&s->d_mtab, bm));
-    NGMI_HIP(hipMalloc(&s->d_model_of, bo));
-    NGMI_HIP(hipMalloc(&s->d_code, F * sizeof(int)));
-    if (!itab.empty()) NGMI_HIP(hipMemcpy(s->d_itab, itab.data(), itab.size() * 8, hipMemcpyHostToDevice));
-    if (!mtab.empty()) NGMI_HIP(hipMemcpy(s->d_mtab, mtab.data(), mtab.size() * 8, hipMemcpyHostToDevice));
-    if (n) NGMI_HIP(hipMemcpy(s->d_model_of, s->model_of.data(), n * sizeof(int), hipMemcpyHostToDevice));
-    NGMI_HIP(hipMemcpy(s->d_code, s->code.data(), F * sizeof(int), hipMemcpyHostToDevice));
-    s->dev_bytes = bi + bm + bo + F * sizeof(int);
-    s->tab.itab = s->d_itab;
-    s->tab.mtab = s->d_mtab;
-    s->tab.model_of = s->d_model_of;
-    s->tab.n = (int64_t)n;
-    s->tab.nm = nm;
-    s->tab.mcols = s->mcols;
-    s->tab.code = s->d_code;
+    s->tab.mode = B4T_COLUMNS;
+    int rc;
+    if ((rc = s->upload(itab, &s->tab.itab)) || (rc = s->upload(mtab, &s->tab.mtab)) ||
+        (rc = s->upload(s->model_of, &s->tab.model_of)) || (rc = s->upload(s->code, &s->tab.code)))
+        return rc;
+    return NGMI_OK;
+}
+
+int set_finalize_host(ngmi_bsim4_set *s)
+{
+    if (!s) return NGMI_E_PANIC;
+    const int rc = set_resolve(s);
+    if (rc == NGMI_OK) s->release();
+    return rc;
+}
+
+}  // namespace ngmi
+
+extern "C" {
+
+int ngmi_bsim4_set_finalize(ngmi_bsim4_set *s)
+{
+    int rc = set_finalize_host(s);
+    if (rc) return rc;
+    s->final_ = false;   /* until its tables are on the device */
+    const SetRecords &R = s->recs;
+    if (!R.ok) {
+        if ((rc = set_upload_columns(s))) return rc;
+        s->final_ = true;
+        return NGMI_OK;
+    }
+    std::vector<int> items, at(s->inst.size());
+    for (size_t k = 0; k < at.size(); k++) at[k] = (int)k;
+    build_items(R.rec_of, items);
+    const size_t ntile = (at.size() + B4_TILE - 1) / B4_TILE, nit = items.size() / 2;
+    /* scalar records run a tile once per record in it: worth it up to a
+     * third more workgroups, or while they all fit two to a SIMD (one of
+     * 1024 SIMDs each) */
+    s->tab.mode = nit <= std::max(ntile + ntile / 3, (size_t)2048) ? B4T_UNIFORM : B4T_LANES;
+    s->tab.nc = R.nc;
+    s->tab.nitems = (int)nit;
+    std::vector<double> tiles;
+    set_tiles(s, at, tiles);
+    if ((rc = s->upload(R.rec, &s->tab.rec)) || (rc = s->upload(tiles, &s->tab.itile)) ||
+        (rc = s->upload(R.rec_of, &s->tab.rec_of)) || (rc = s->upload(items, &s->tab.items)))
+        return rc;
     s->final_ = true;
     return NGMI_OK;
 }

@@ -148,23 +148,24 @@ NGMI_HD double dev_fetlim(double vnew, double vold, double vto)
     return vnew;
 }
 
-/* NIintegrate (niinteg.c:18-80) on charge state qcap; returns ceq */
+/* NIintegrate (niinteg.c:18-80) on charge state qcap, whose values at
+ * levels 0 and 1 are q0 and q1; stores and returns the current */
 template <class S>
-NGMI_HD double b4_integrate(S &st, const B4Ckt &ck, int qcap)
+NGMI_HD double b4_integrate(S &st, const B4Ckt &ck, int qcap, double q0, double q1)
 {
     const int ccap = qcap + 1;
     double c;
     if (ck.method == 1) {
-        if (ck.order == 1) c = ck.ag[0] * st.s(0, qcap) + ck.ag[1] * st.s(1, qcap);
-        else c = -st.s(1, ccap) * ck.ag[1] + ck.ag[0] * (st.s(0, qcap) - st.s(1, qcap));
+        if (ck.order == 1) c = ck.ag[0] * q0 + ck.ag[1] * q1;
+        else c = -st.s(1, ccap) * ck.ag[1] + ck.ag[0] * (q0 - q1);
     } else {
         c = 0;
         for (int k = ck.order; k >= 2; k--) c += ck.ag[k] * st.s(k, qcap);
-        c += ck.ag[1] * st.s(1, qcap);
-        c += ck.ag[0] * st.s(0, qcap);
+        c += ck.ag[1] * q1;
+        c += ck.ag[0] * q0;
     }
     st.set(0, ccap, c);
-    return c - ck.ag[0] * st.s(0, qcap);
+    return c;
 }
 
 /* junction diode DC model for one side (b4ld.c:700-860) */
@@ -347,37 +348,34 @@ NGMI_HD int b4_load(const P &prm, S &st, C &ca, const B4Ckt &ck, const double *v
     } else if ((mode & (M_INITJCT | M_INITFIX)) && PR(off) != 0.0) {
         vds = vgs = vbs = 0.0;
     } else {
-        const double s0vds = st.s(0, B4X_vds), s0vgs = st.s(0, B4X_vgs), s0vbs = st.s(0, B4X_vbs);
-        const double s0vbd = st.s(0, B4X_vbd);
         double delvbd, delvgd, delvds, delvgs, delvbs, vgdo;
+        double r0vds, r0vgs, r0vbs, r0vbd;   /* level 0, the limiting reference */
         const int from1 = mode & (M_INITPRED | M_GUESSED);
         if (from1) {
             /* b4ld.c:322-372: state0 takes state1, and in INITPRED the
              * voltages extrapolate */
             const double s1vds = st.s(1, B4X_vds), s1vgs = st.s(1, B4X_vgs), s1vbs = st.s(1, B4X_vbs);
-            const double s1vdbs = st.s(1, B4X_vdbs);
-            st.set(0, B4X_vds, s1vds);
-            st.set(0, B4X_vgs, s1vgs);
-            st.set(0, B4X_vbs, s1vbs);
-            st.set(0, B4X_vbd, s1vbs - s1vds);
-            st.set(0, B4X_vdbs, s1vdbs);
-            st.set(0, B4X_vdbd, s1vdbs - s1vds);
             if (mode & M_INITPRED) {
                 const double xf = ck.xfact;
                 vds = (1.0 + xf) * s1vds - (xf * st.s(2, B4X_vds));
                 vgs = (1.0 + xf) * s1vgs - (xf * st.s(2, B4X_vgs));
                 vbs = (1.0 + xf) * s1vbs - (xf * st.s(2, B4X_vbs));
             }
+            r0vds = s1vds;
+            r0vgs = s1vgs;
+            r0vbs = s1vbs;
+            r0vbd = s1vbs - s1vds;
+        } else {
+            r0vds = st.s(0, B4X_vds);
+            r0vgs = st.s(0, B4X_vgs);
+            r0vbs = st.s(0, B4X_vbs);
+            r0vbd = st.s(0, B4X_vbd);
         }
         if (!(mode & M_INITPRED)) {
             vds = type * (vnode[0] - vnode[2]);
             vgs = type * (vnode[1] - vnode[2]);
             vbs = type * (vnode[3] - vnode[2]);
         }
-        const double r0vds = from1 ? st.s(0, B4X_vds) : s0vds;
-        const double r0vgs = from1 ? st.s(0, B4X_vgs) : s0vgs;
-        const double r0vbs = from1 ? st.s(0, B4X_vbs) : s0vbs;
-        const double r0vbd = from1 ? st.s(0, B4X_vbd) : s0vbd;
         vgdo = r0vgs - r0vds;
         vbd = vbs - vds;
         vgd = vgs - vds;
@@ -1949,9 +1947,8 @@ NGMI_HD int b4_load(const P &prm, S &st, C &ca, const B4Ckt &ck, const double *v
     }
 
     /* ---- junction C-V (b4ld.c:3944-4063) */
-    double capbs = 0.0, capbd = 0.0;
+    double capbs = 0.0, capbd = 0.0, qbs = 0.0, qbd = 0.0;
     if (ChargeComputationNeeded) {
-        double qbs, qbd;
         b4_jcv(vbs_jct, PR(czbs), PR(czbssw), PR(czbsswg), PR(MJS), PR(MJSWS), PR(MJSWGS),
                PR(PhiBS), PR(PhiBSWS), PR(PhiBSWGS), qbs, capbs);
         b4_jcv(vbd_jct, PR(czbd), PR(czbdsw), PR(czbdswg), PR(MJD), PR(MJSWD), PR(MJSWGD),
@@ -2066,26 +2063,36 @@ NGMI_HD int b4_load(const P &prm, S &st, C &ca, const B4Ckt &ck, const double *v
             gcbsb = (cbdb - capbs) * ag0;
             gcbbb = -(gcbgb + gcbdb + gcbsb);
         }
+        const double sqd = qdrn - qbd, sqb = qbulk + qbd + qbs;
         st.set(0, B4X_qg, qgate);
-        st.set(0, B4X_qd, qdrn - st.s(0, B4X_qbd));
-        st.set(0, B4X_qs, qsrc - st.s(0, B4X_qbs));
-        st.set(0, B4X_qb, qbulk + st.s(0, B4X_qbd) + st.s(0, B4X_qbs));
+        st.set(0, B4X_qd, sqd);
+        st.set(0, B4X_qs, qsrc - qbs);
+        st.set(0, B4X_qb, sqb);
         if (!(mode & M_INITSMSIG) && !(mode & M_DCTRANCURVE)) {
+            /* the charges at level 1: in INITTRAN level 0's, stored there */
+            double q1b, q1g, q1d;
             if (mode & M_INITTRAN) {
-                st.set(1, B4X_qb, st.s(0, B4X_qb));
-                st.set(1, B4X_qg, st.s(0, B4X_qg));
-                st.set(1, B4X_qd, st.s(0, B4X_qd));
+                q1b = sqb;
+                q1g = qgate;
+                q1d = sqd;
+                st.set(1, B4X_qb, q1b);
+                st.set(1, B4X_qg, q1g);
+                st.set(1, B4X_qd, q1d);
+            } else {
+                q1b = st.s(1, B4X_qb);
+                q1g = st.s(1, B4X_qg);
+                q1d = st.s(1, B4X_qd);
             }
-            b4_integrate(st, ck, B4X_qb);
-            b4_integrate(st, ck, B4X_qg);
-            b4_integrate(st, ck, B4X_qd);
-            ceqqg = st.s(0, B4X_cqg) - gcggb * vgb + gcgdb * vbd + gcgsb * vbs;
-            ceqqd = st.s(0, B4X_cqd) - gcdgb * vgb + gcddb * vbd + gcdsb * vbs;
-            ceqqb = st.s(0, B4X_cqb) - gcbgb * vgb + gcbdb * vbd + gcbsb * vbs;
+            const double cqb = b4_integrate(st, ck, B4X_qb, sqb, q1b);
+            const double cqg = b4_integrate(st, ck, B4X_qg, qgate, q1g);
+            const double cqd = b4_integrate(st, ck, B4X_qd, sqd, q1d);
+            ceqqg = cqg - gcggb * vgb + gcgdb * vbd + gcgsb * vbs;
+            ceqqd = cqd - gcdgb * vgb + gcddb * vbd + gcdsb * vbs;
+            ceqqb = cqb - gcbgb * vgb + gcbdb * vbd + gcbsb * vbs;
             if (mode & M_INITTRAN) {
-                st.set(1, B4X_cqb, st.s(0, B4X_cqb));
-                st.set(1, B4X_cqg, st.s(0, B4X_cqg));
-                st.set(1, B4X_cqd, st.s(0, B4X_cqd));
+                st.set(1, B4X_cqb, cqb);
+                st.set(1, B4X_cqg, cqg);
+                st.set(1, B4X_cqd, cqd);
             }
         } else {
             gcggb = gcgdb = gcgsb = gcgbb = gcdgb = gcddb = gcdsb = gcdbb = 0.0;

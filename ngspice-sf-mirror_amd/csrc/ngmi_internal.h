@@ -45,15 +45,22 @@ int waves_for(int knob, int64_t instances);
     } while (0)
 
 /*
- * Device view of a BSIM4 evaluation table.  Each field is either a
- * per-instance column (itab[col * n + i]) or, when every instance of a
- * model card has the same value, a per-model column (mtab[m * mcols +
- * col], model-major so that one card's values share cache lines).
- * code[f] = col for a per-instance field and ~col for a per-model one; the
- * code array lives in device memory and is read with a scalar load next to
- * each use (a kernel-argument copy would pin ~190 SGPRs for the whole
- * kernel).
+ * Device view of a BSIM4 evaluation table.
+ *
+ * Record form (mode B4T_UNIFORM, B4T_LANES; see bsim4_dev.h): rec holds
+ * complete field rows, rec_of[i] the record of instance i, itile the
+ * per-instance columns in tiles of 64 instances, of which the first nc vary
+ * within a record.
+ *
+ * Column form (B4T_COLUMNS), for sets whose instances share no records:
+ * each field is either a per-instance column (itab[col * n + i]) or, when
+ * every instance of a model card has the same value, a per-model column
+ * (mtab[m * mcols + col], model-major so that one card's values share cache
+ * lines).  code[f] = col for a per-instance field and ~col for a per-model
+ * one, read with a scalar load next to each use.
  */
+enum : int { B4T_COLUMNS = 0, B4T_UNIFORM = 1, B4T_LANES = 2 };
+
 struct B4Tab {
     const double *itab;
     const double *mtab;
@@ -63,6 +70,11 @@ struct B4Tab {
     int mcols;       /* per-model columns (row stride of mtab) */
     const int *code;
     int flags;       /* the selector word when every instance shares it, else -1 */
+    int mode, nc;
+    const double *rec, *itile;
+    const int *rec_of;
+    const int *items;   /* B4T_UNIFORM: (tile, record) pairs */
+    int nitems;
 };
 
 }  // namespace ngmi

@@ -32,9 +32,8 @@
 #include "tran_types.h"
 
 namespace ngmi {
-int launch_tran_pass(const B4Tab *tab0, const TranDev *D0, int c_begin, int c_end, const B4Tab *tabs,
-                     const TranDev *Ds, const int2 *mos_blk, int n_mos_blk, const int2 *step_blk,
-                     int n_step_blk, size_t lds_bytes, hipStream_t s, hipEvent_t *ev);
+int launch_tran_pass(const MosLaunch &M, const TranDev *D0, int c_begin, int c_end, const TranDev *Ds,
+                     const int2 *step_blk, int n_step_blk, size_t lds_bytes, hipStream_t s, hipEvent_t *ev);
 int set_tran_lds_limit(size_t bytes);
 int launch_zero_int(int *p, hipStream_t s);
 int launch_guess_apply(const TranDev &D, const float *y, const int64_t *dest, const double2 *base,
@@ -43,7 +42,6 @@ int mlp_forward_rows(ngmi_mlp *n, const float *X, float *y, int maxRows, const i
                      hipStream_t s);
 int mlp_guess_rows(const ngmi_mlp *n, const float *X, int *count, int maxRows, const int64_t *dest,
                    const double2 *base, double *x, float *yout, unsigned long long *rows_total, hipStream_t s);
-const B4Tab *set_table(const ngmi_bsim4_set *s);
 }
 
 using namespace ngmi;
@@ -70,6 +68,8 @@ constexpr int64_t PV_POOL_BYTES = 512ll << 20;
 constexpr int64_t PV_SLOT_MAX_BYTES = 1ll << 30;
 
 #include "circuit_types.h"
+#include "set_table.h"
+#include "bsim4_dev.h"
 
 /* circuits of one topology inside a batch: shared symbolic analysis and
  * BSIM4 table, per-circuit device arrays */
@@ -77,6 +77,10 @@ struct TopoGroup {
     int C = 0, N = 0, NN = 0, NM = 0, NCAP = 0, NRES = 0, NVS = 0;
     std::vector<int> ids;               /* batch index of each circuit of the group */
     ngmi_bsim4_set *set = nullptr;
+    /* padded MOSFET storage, where the circuits' records allow it: the
+     * MOSFET at each place of a circuit (-1: a hole) */
+    bool can_pad = false;
+    std::vector<int> place;
     TranDev D{};
     size_t lds = 0;
     std::vector<int> probe;
@@ -100,8 +104,10 @@ struct ngmi_batch {
     /* one fused launch per pass: group descriptors and block -> group maps */
     TranDev *dD = nullptr;
     B4Tab *dTab = nullptr;
-    int2 *mos_blk = nullptr, *step_blk = nullptr;
-    int n_mos_blk = 0, n_step_blk = 0;
+    int4 *mos_blk = nullptr;
+    int2 *step_blk = nullptr;
+    int n_step_blk = 0;
+    MosLaunch mos;
     size_t lds = 0;
     int *done_count = nullptr;
     /* kernel timing of the last run (events on the launch stream) */
@@ -811,10 +817,9 @@ int analyze(const ngmi_circuit &c0, Plan &P)
     return NGMI_OK;
 }
 
-/* one topology group of a batch: symbolic analysis, BSIM4 table and the
- * device arrays of its circuits */
-int build_group(ngmi_batch *b, TopoGroup *G, const std::vector<const ngmi_circuit *> &ckts,
-                const int *probe, int nprobe)
+/* a topology group's sizes, its BSIM4 instances and their places in padded
+ * storage */
+int build_set(TopoGroup *G, const std::vector<const ngmi_circuit *> &ckts)
 {
     auto fail = [](const char *what) {
         if (what) set_error("%s", what);
@@ -830,13 +835,6 @@ int build_group(ngmi_batch *b, TopoGroup *G, const std::vector<const ngmi_circui
     G->NCAP = (int)c0.caps.size();
     G->NRES = (int)c0.res.size();
     const int N = G->N, NN = G->NN, NM = G->NM, NCAP = G->NCAP, NRES = G->NRES, NVS = G->NVS;
-
-    Plan P;
-    if (analyze(c0, P) != NGMI_OK) return fail(nullptr);
-    G->ic_nodes_host = P.ic_nodes;
-    G->nbr_host = P.nbr;
-    G->nslots = P.nslots; G->nterms = P.nterms;
-    G->nlev_f = P.nlev_f; G->nlev_fw = P.nlev_fw; G->nlev_bw = P.nlev_bw;
 
     /* ---- BSIM4 instances, circuit-major */
     G->set = ngmi_bsim4_set_new();
@@ -870,7 +868,47 @@ int build_group(ngmi_batch *b, TopoGroup *G, const std::vector<const ngmi_circui
             if (rc < 0) return fail(nullptr);
         }
     }
-    if (ngmi_bsim4_set_finalize(G->set) != NGMI_OK) return fail(nullptr);
+    if (set_finalize_host(G->set) != NGMI_OK) return NGMI_E_UNSUPP;
+    /* places of padded storage: circuit 0's MOSFETs by record, each record's
+     * part rounded up to whole tiles; usable when every circuit's tiles have
+     * one record too */
+    const SetRecords &R = *set_records(G->set);
+    if (!R.ok) return NGMI_OK;
+    std::vector<int> order(NM);
+    for (int j = 0; j < NM; j++) order[j] = j;
+    std::stable_sort(order.begin(), order.end(), [&](int p, int q) { return R.rec_of[p] < R.rec_of[q]; });
+    for (int j = 0; j < NM; j++) {
+        if (j > 0 && R.rec_of[order[j]] != R.rec_of[order[j - 1]])
+            while (G->place.size() % MOS_TILE) G->place.push_back(-1);
+        G->place.push_back(order[j]);
+    }
+    while (G->place.size() % MOS_TILE) G->place.push_back(-1);
+    for (int c = 0; c < C; c++)
+        for (size_t t = 0; t < G->place.size(); t += MOS_TILE)
+            for (size_t q = t; q < t + MOS_TILE && G->place[q] >= 0; q++)
+                if (R.rec_of[(size_t)c * NM + G->place[q]] != R.rec_of[(size_t)c * NM + G->place[t]]) return NGMI_OK;
+    G->can_pad = true;
+    return NGMI_OK;
+}
+
+/* the rest of a group: the symbolic plan of its topology and the device
+ * arrays of its circuits, MOSFETs stored as b->mos says */
+int build_group(ngmi_batch *b, TopoGroup *G, const std::vector<const ngmi_circuit *> &ckts,
+                const int *probe, int nprobe)
+{
+    auto fail = [](const char *what) {
+        if (what) set_error("%s", what);
+        return NGMI_E_UNSUPP;
+    };
+    const ngmi_circuit &c0 = *ckts[0];
+    const int C = G->C, N = G->N, NN = G->NN, NM = G->NM, NCAP = G->NCAP, NRES = G->NRES, NVS = G->NVS;
+
+    Plan P;
+    if (analyze(c0, P) != NGMI_OK) return fail(nullptr);
+    G->ic_nodes_host = P.ic_nodes;
+    G->nbr_host = P.nbr;
+    G->nslots = P.nslots; G->nterms = P.nterms;
+    G->nlev_f = P.nlev_f; G->nlev_fw = P.nlev_fw; G->nlev_bw = P.nlev_bw;
 
     /* ---- per-circuit element values */
     std::vector<double> cap_c((size_t)C * NCAP), res_g((size_t)C * NRES), vs_par((size_t)C * NVS * VSP);
@@ -895,10 +933,15 @@ int build_group(ngmi_batch *b, TopoGroup *G, const std::vector<const ngmi_circui
         }
         for (int u = 1; u <= NN; u++) ic_val[(size_t)c * (NN + 1) + u] = ck.ic[u];
     }
-    std::vector<int> mos_nodes(4 * (size_t)NM), cap_nodes(2 * (size_t)NCAP), res_nodes(2 * (size_t)NRES),
+    const bool padded = b->mos.mode == B4T_UNIFORM;
+    std::vector<int> at(NM);   /* MOSFET at each place */
+    for (int j = 0; j < NM; j++) at[j] = j;
+    if (padded) at = G->place;
+    const int NS = (int)at.size();
+    std::vector<int> mos_nodes(4 * (size_t)NS, -1), cap_nodes(2 * (size_t)NCAP), res_nodes(2 * (size_t)NRES),
         vs_nodes(3 * (size_t)NVS), ic_nodes(NN + 1);
-    for (int j = 0; j < NM; j++)
-        for (int r = 0; r < 4; r++) mos_nodes[(size_t)r * NM + j] = c0.mos[j].node[r];
+    for (int j = 0; j < NS; j++)
+        for (int r = 0; r < 4 && at[j] >= 0; r++) mos_nodes[(size_t)r * NS + j] = c0.mos[at[j]].node[r];
     for (int k = 0; k < NCAP; k++) {
         cap_nodes[k] = (int)c0.caps[k][0];
         cap_nodes[NCAP + k] = (int)c0.caps[k][1];
@@ -920,6 +963,7 @@ int build_group(ngmi_batch *b, TopoGroup *G, const std::vector<const ngmi_circui
     
     TranDev &D = G->D;
     D.C = C; D.N = N; D.NN = NN; D.NM = NM; D.NCAP = NCAP; D.NRES = NRES; D.NVS = NVS;
+    D.NS = NS; D.W = padded ? NS / MOS_TILE : 0; D.NV = padded ? D.W : NM;
     D.nslots = P.nslots; D.nlev_f = G->nlev_f; D.nlev_fw = G->nlev_fw; D.nlev_bw = G->nlev_bw;
     D.n_aleaf = P.n_aleaf; D.n_acomb = P.n_acomb; D.n_rleaf = P.n_rleaf; D.n_rcomb = P.n_rcomb;
     D.n_apart = P.n_apart; D.n_rpart = P.n_rpart; D.n_icrow = P.n_icrow;
@@ -971,15 +1015,40 @@ int build_group(ngmi_batch *b, TopoGroup *G, const std::vector<const ngmi_circui
     UP(P.bw_term, bw_term, uint32_t, up);
     UP(P.perm, perm_unknown, int, ip);
     UP(P.unk_pos, unk_pos, int, ip);
-    UP(P.mos_pos, mos_pos, int, ip);
+    auto by_place = [&](const std::vector<int> &v, int rows) {
+        std::vector<int> o((size_t)rows * NS, -1);
+        for (int k = 0; k < rows; k++)
+            for (int j = 0; j < NS; j++)
+                if (at[j] >= 0) o[(size_t)k * NS + j] = v[(size_t)k * NM + at[j]];
+        return o;
+    };
+    const std::vector<int> mos_pos = by_place(P.mos_pos, B4S__COUNT), rmos_pos = by_place(P.rmos_pos, B4R__COUNT);
+    UP(mos_pos, mos_pos, int, ip);
     UP(P.diag_slot, diag_slot, int, ip);
-    UP(P.rmos_pos, rmos_pos, int, ip);
+    UP(rmos_pos, rmos_pos, int, ip);
     UP(G->probe, probe, int, ip);
     UP(G->nbr_host, nbr, int, ip);
     UP(P.row_start, row_start, int, ip);
     UP(P.slot_col, slot_col, int, ip);
-#undef UP
-    const int64_t cnm = (int64_t)C * NM, cnc = (int64_t)C * NCAP;
+    const int64_t cnc = (int64_t)C * NCAP, ntile = ((int64_t)C * NS + MOS_TILE - 1) / MOS_TILE;
+    if (b->mos.mode == B4T_COLUMNS) {
+        if (set_upload_columns(G->set) != NGMI_OK) return fail(nullptr);
+    } else {
+        const SetRecords &R = *set_records(G->set);
+        std::vector<int> inst((size_t)C * NS, -1), rec;
+        for (int c = 0; c < C; c++)
+            for (int j = 0; j < NS; j++)
+                if (at[j] >= 0) inst[(size_t)c * NS + j] = c * NM + at[j];
+        if (padded)
+            for (size_t t = 0; t < inst.size(); t += MOS_TILE) rec.push_back(R.rec_of[inst[t]]);
+        else
+            rec = R.rec_of;
+        std::vector<double> tiles;
+        set_tiles(G->set, inst, tiles);
+        UP(R.rec, rec, double, dp);
+        UP(tiles, itile, double, dp);
+        UP(rec, rec_of, int, ip);
+    }
     if (alloc(b, (size_t)C * NVS, &dp) != NGMI_OK) return fail(nullptr);
     D.vs_brk = dp;
     CktCtl *ctl;
@@ -987,17 +1056,19 @@ int build_group(ngmi_batch *b, TopoGroup *G, const std::vector<const ngmi_circui
     D.ctl = ctl;
     if (alloc(b, (size_t)2 * C * (N + 1), &dp) != NGMI_OK) return fail(nullptr);
     D.x = dp;
-    if (alloc(b, (size_t)NLEV * B4X__COUNT * cnm, &dp) != NGMI_OK) return fail(nullptr);
+#undef UP
+    D.ntile = ntile;
+    if (alloc(b, (size_t)NLEV * MOS_ROWS * MOS_TILE * ntile, &dp) != NGMI_OK) return fail(nullptr);
     D.mstate = dp;
     if (alloc(b, (size_t)NLEV * 2 * cnc, &dp) != NGMI_OK) return fail(nullptr);
     D.cstate = dp;
-    if (alloc(b, (size_t)B4C__COUNT * cnm, &dp) != NGMI_OK) return fail(nullptr);
+    if (alloc(b, (size_t)B4C__COUNT * MOS_TILE * ntile, &dp) != NGMI_OK) return fail(nullptr);
     D.cache = dp;
     D.NA = P.NA;
     D.NR = P.NR;
     if (alloc(b, (size_t)C * (N + 1), &dp) != NGMI_OK) return fail(nullptr);
     D.bak_x = dp;
-    if (alloc(b, (size_t)C * (B4X__COUNT * (size_t)NM + 2 * (size_t)NCAP), &dp) != NGMI_OK)
+    if (alloc(b, (size_t)C * (B4X__COUNT * (size_t)NS + 2 * (size_t)NCAP), &dp) != NGMI_OK)
         return fail(nullptr);
     D.bak_s = dp;
     if (alloc(b, (size_t)C * P.NA, &dp) != NGMI_OK) return fail(nullptr);
@@ -1026,7 +1097,7 @@ int build_group(ngmi_batch *b, TopoGroup *G, const std::vector<const ngmi_circui
     }
     if (alloc(b, (size_t)C * P.NR, &dp) != NGMI_OK) return fail(nullptr);
     D.rcontrib = dp;
-    if (alloc(b, (size_t)cnm, &ip) != NGMI_OK) return fail(nullptr);
+    if (alloc(b, (size_t)C * D.NV, &ip) != NGMI_OK) return fail(nullptr);
     D.noncon = ip;
     if (alloc(b, (size_t)C * b->cap_pts, &dp) != NGMI_OK) return fail(nullptr);
     D.out_t = dp;
@@ -1301,31 +1372,56 @@ ngmi_batch *ngmi_batch_new(ngmi_circuit *const *ckts, int C, const int *probe, i
     }
     if (alloc(b, 1, &b->done_count) != NGMI_OK)
         return bail(nullptr);
-    std::vector<TranDev> Ds;
-    std::vector<B4Tab> tabs;
-    std::vector<int2> mb, sb;
+    /* the BSIM4 instances of every group, then how the batch stores and
+     * reads them: padded storage (a wavefront has one circuit and one record,
+     * read with scalar loads) unless its holes cost more than a third more
+     * wavefronts than dense storage takes and the wavefronts no longer fit
+     * two to a SIMD of the 1024 (small circuits in large batches) */
+    int64_t wp = 0, wd = 0;
+    bool records = true, pad = true;
+    std::vector<std::vector<const ngmi_circuit *>> cs(members.size());
     for (size_t g = 0; g < members.size(); g++) {
         TopoGroup *G = new TopoGroup;
         b->groups.push_back(G);
         G->ids = members[g];
-        std::vector<const ngmi_circuit *> cs;
-        for (int c : members[g]) cs.push_back(ckts[c]);
-        if (build_group(b, G, cs, probe, nprobe) != NGMI_OK) return bail(nullptr);
+        for (int c : members[g]) cs[g].push_back(ckts[c]);
+        const int rc = build_set(G, cs[g]);
+        if (rc != NGMI_OK) return bail(nullptr);
+        const B4Tab &T = *set_table(G->set);
+        if (G->NM > 0) b->mos.flags = wd == 0 || T.flags == b->mos.flags ? T.flags : -1;
+        records = records && set_records(G->set)->ok;
+        pad = pad && G->can_pad;
+        b->mos.nc = std::max(b->mos.nc, set_records(G->set)->nc);
+        wp += (int64_t)G->C * (int64_t)(G->place.size() / MOS_TILE);
+        wd += ((int64_t)G->C * G->NM + MOS_TILE - 1) / MOS_TILE;
+    }
+    b->mos.mode = !records ? B4T_COLUMNS : pad && wp <= std::max<int64_t>(wd + wd / 3, 2048) ? B4T_UNIFORM : B4T_LANES;
+    std::vector<TranDev> Ds;
+    std::vector<B4Tab> tabs;
+    std::vector<int2> sb;
+    std::vector<int4> mb;
+    for (size_t g = 0; g < members.size(); g++) {
+        TopoGroup *G = b->groups[g];
+        if (build_group(b, G, cs[g], probe, nprobe) != NGMI_OK) return bail(nullptr);
         Ds.push_back(G->D);
         tabs.push_back(*set_table(G->set));
-        /* MOSFET kernel: whole blocks per group; (group, first block) */
-        const int64_t cnm = (int64_t)G->C * G->NM;
-        const int first = (int)mb.size();
-        for (int64_t k = 0; k < (cnm + 255) / 256; k++) mb.push_back(make_int2((int)g, first));
+        if (b->mos.mode == B4T_UNIFORM) {
+            for (int c = 0; c < G->C; c++)
+                for (int w = 0; w < G->D.W; w++) mb.push_back(make_int4((int)g, c, w, 0));
+        } else {
+            for (int64_t t = 0; t < G->D.ntile; t++) mb.push_back(make_int4((int)g, (int)t, 0, 0));
+        }
         /* step kernel: one block per circuit; (group, circuit) */
         for (int c = 0; c < G->C; c++) sb.push_back(make_int2((int)g, c));
         b->lds = std::max(b->lds, G->lds);
     }
-    b->n_mos_blk = (int)mb.size();
     b->n_step_blk = (int)sb.size();
     if (upload<TranDev>(b, Ds, &b->dD) != NGMI_OK || upload<B4Tab>(b, tabs, &b->dTab) != NGMI_OK ||
-        upload<int2>(b, mb, &b->mos_blk) != NGMI_OK || upload<int2>(b, sb, &b->step_blk) != NGMI_OK)
+        upload<int4>(b, mb, &b->mos_blk) != NGMI_OK || upload<int2>(b, sb, &b->step_blk) != NGMI_OK)
         return bail(nullptr);
+    b->mos.nblk = (int)mb.size();
+    b->mos.blk = b->mos_blk;
+    b->mos.tabs = b->dTab;
     if (b->lds > 64 * 1024 && set_tran_lds_limit(b->lds) != NGMI_OK) return bail(nullptr);
     return b;
 }
@@ -1472,7 +1568,7 @@ int ngmi_batch_tran(ngmi_batch *b, double tstep, double tstop, double tmax, int6
             }
         }
         NGMI_HIP(hipMemcpyAsync(D.ctl, ctl.data(), sizeof(CktCtl) * G->C, hipMemcpyHostToDevice, s));
-        const int64_t cnm = (int64_t)G->C * G->NM, cnc = (int64_t)G->C * G->NCAP;
+        const int64_t cnc = (int64_t)G->C * G->NCAP;
         NGMI_HIP(hipMemsetAsync(D.x, 0, sizeof(double) * 2 * G->C * (size_t)(G->N + 1), s));
         if (G->uic) {
             /* CKTic (cktic.c:19-80): CKTrhs and CKTrhsOld hold the .ic
@@ -1482,9 +1578,9 @@ int ngmi_batch_tran(ngmi_batch *b, double tstep, double tstop, double tmax, int6
                                       sizeof(double) * (size_t)(G->NN + 1), sizeof(double) * (size_t)(G->NN + 1),
                                       (size_t)G->C, hipMemcpyDeviceToDevice, s));
         }
-        NGMI_HIP(hipMemsetAsync(D.mstate, 0, sizeof(double) * NLEV * B4X__COUNT * (size_t)cnm, s));
+        NGMI_HIP(hipMemsetAsync(D.mstate, 0, sizeof(double) * NLEV * MOS_ROWS * MOS_TILE * (size_t)D.ntile, s));
         NGMI_HIP(hipMemsetAsync(D.cstate, 0, sizeof(double) * NLEV * 2 * (size_t)cnc, s));
-        NGMI_HIP(hipMemsetAsync(D.cache, 0, sizeof(double) * B4C__COUNT * (size_t)cnm, s));
+        NGMI_HIP(hipMemsetAsync(D.cache, 0, sizeof(double) * B4C__COUNT * MOS_TILE * (size_t)D.ntile, s));
         NGMI_HIP(hipMemsetAsync(D.pv_owner, 0, sizeof(int) * (size_t)std::max(D.pv_slots, 1), s));
         std::vector<double> brk((size_t)G->C * G->NVS, -1.0);
         NGMI_HIP(hipMemcpyAsync(D.vs_brk, brk.data(), brk.size() * sizeof(double),
@@ -1500,7 +1596,6 @@ int ngmi_batch_tran(ngmi_batch *b, double tstep, double tstop, double tmax, int6
     }
     const TopoGroup &G0 = *b->groups[0];
     const bool one = b->groups.size() == 1;
-    const B4Tab *tab0 = set_table(G0.set);
     const bool fused = tune_get(TUNE_GUESS_FUSED) != 0;
     /* two streams: the circuits' halves alternate, so one half's latency-
      * bound step kernel runs beside the other half's BSIM4 kernel (single
@@ -1595,18 +1690,16 @@ int ngmi_batch_tran(ngmi_batch *b, double tstep, double tstop, double tmax, int6
             if (b->net) r = guess_pass(sa, 0);
             if (r != NGMI_OK) break;
             if (split) {
-                r = launch_tran_pass(tab0, &G0.D, 0, cut[1], nullptr, nullptr, nullptr, 1, nullptr, cut[1], b->lds, sa,
-                                     nullptr);
+                r = launch_tran_pass(b->mos, &G0.D, 0, cut[1], b->dD, nullptr, cut[1], b->lds, sa, nullptr);
                 if (r == NGMI_OK && b->net) r = guess_pass(s2, 1);
                 if (r == NGMI_OK)
-                    r = launch_tran_pass(tab0, &G0.D, cut[1], cut2, nullptr, nullptr, nullptr, 1, nullptr,
-                                         cut2 - cut[1], b->lds, s2, nullptr);
+                    r = launch_tran_pass(b->mos, &G0.D, cut[1], cut2, b->dD, nullptr, cut2 - cut[1], b->lds, s2, nullptr);
                 for (size_t t = 0; t < sx.size() && r == NGMI_OK; t++)
-                    r = launch_tran_pass(tab0, &G0.D, cut[t + 2], cut[t + 3], nullptr, nullptr, nullptr, 1, nullptr,
-                                         cut[t + 3] - cut[t + 2], b->lds, sx[t], nullptr);
+                    r = launch_tran_pass(b->mos, &G0.D, cut[t + 2], cut[t + 3], b->dD, nullptr, cut[t + 3] - cut[t + 2], b->lds,
+                                         sx[t], nullptr);
             } else {
-                r = launch_tran_pass(one ? tab0 : nullptr, one ? &G0.D : nullptr, 0, C, b->dTab, b->dD, b->mos_blk,
-                                     b->n_mos_blk, b->step_blk, b->n_step_blk, b->lds, sa, nullptr);
+                r = launch_tran_pass(b->mos, one ? &G0.D : nullptr, 0, C, b->dD, b->step_blk, b->n_step_blk, b->lds, sa,
+                                     nullptr);
             }
         }
         if (split && capturing && r == NGMI_OK) {
@@ -1671,15 +1764,14 @@ int ngmi_batch_tran(ngmi_batch *b, double tstep, double tstop, double tmax, int6
                 if (b->profile) NGMI_HIP(hipEventRecord(gev[2 * k + 1], s));
             }
             if (split) {
-                rc = launch_tran_pass(tab0, &G0.D, 0, half, nullptr, nullptr, nullptr, 1, nullptr,
-                                      half, b->lds, s, b->profile ? &ev[3 * k] : nullptr);
+                rc = launch_tran_pass(b->mos, &G0.D, 0, half, b->dD, nullptr, half, b->lds, s,
+                                      b->profile ? &ev[3 * k] : nullptr);
                 if (rc == NGMI_OK)
-                    rc = launch_tran_pass(tab0, &G0.D, half, C, nullptr, nullptr, nullptr, 1, nullptr,
-                                          C - half, b->lds, s2, b->profile ? &ev2[3 * k] : nullptr);
+                    rc = launch_tran_pass(b->mos, &G0.D, half, C, b->dD, nullptr, C - half, b->lds, s2,
+                                          b->profile ? &ev2[3 * k] : nullptr);
             } else {
-                rc = launch_tran_pass(one ? tab0 : nullptr, one ? &G0.D : nullptr, 0, C, b->dTab,
-                                      b->dD, b->mos_blk, b->n_mos_blk, b->step_blk, b->n_step_blk,
-                                      b->lds, s, b->profile ? &ev[3 * k] : nullptr);
+                rc = launch_tran_pass(b->mos, one ? &G0.D : nullptr, 0, C, b->dD, b->step_blk, b->n_step_blk, b->lds, s,
+                                      b->profile ? &ev[3 * k] : nullptr);
             }
             if (rc != NGMI_OK) break;
         }

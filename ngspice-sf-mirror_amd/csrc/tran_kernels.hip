@@ -22,6 +22,7 @@
 #include <climits>
 #include "ngmi_internal.h"
 #include "bsim4_eval.h"
+#include "bsim4_dev.h"
 #include "tran_types.h"
 #include "guess_types.h"
 
@@ -45,40 +46,56 @@ struct TranPrm {
     }
 };
 
+static_assert(MOS_ROWS == B4X__COUNT, "state rows of the MOSFET storage");
+
+/* the states and caches of one tile; lane = place within it */
 struct TranState {
-    double *base;
-    int64_t cnm, i;
+    NGMI_GLOBAL double *base;   /* the tile's first level */
+    unsigned lane;
     int rb;
-    __device__ __forceinline__ double *p(int l, int k) const
+    __device__ __forceinline__ NGMI_GLOBAL double *p(int l, int k) const
     {
-        return base + ((int64_t)lvl(rb, l) * B4X__COUNT + k) * cnm + i;
+        return base + (lvl(rb, l) * MOS_ROWS + k) * MOS_TILE + lane;
     }
     __device__ __forceinline__ double s(int l, int k) const { return *p(l, k); }
     __device__ __forceinline__ void set(int l, int k, double v) { *p(l, k) = v; }
 };
 
 struct TranCache {
-    double *c_;
-    int64_t cnm, i;
-    __device__ __forceinline__ double c(int k) const { return c_[k * cnm + i]; }
-    __device__ __forceinline__ void setc(int k, double v) { c_[k * cnm + i] = v; }
+    NGMI_GLOBAL double *c_;
+    unsigned lane;
+    __device__ __forceinline__ double c(int k) const { return c_[k * MOS_TILE + lane]; }
+    __device__ __forceinline__ void setc(int k, double v) { c_[k * MOS_TILE + lane] = v; }
 };
 
-/* one thread per (circuit, MOSFET) of a topology group, circuit-major
- * instances i = c * NM + j */
-template <int FL>
-__device__ __forceinline__ void tran_mos_body(const B4Tab &tab, const TranDev &D, int64_t i)
+/* what the BSIM4 kernels need of a topology group */
+struct MosArgs {
+    const CktCtl *ctl;
+    const double *x, *rec, *itile;
+    const int *nodes, *pos, *rpos, *rec_of;
+    double *mstate, *cache, *contrib, *rcontrib;
+    int *noncon;
+    int C, N, NM, NS, NA, NR;
+    double reltol, abstol;
+    __device__ __forceinline__ explicit MosArgs(const TranDev &D)
+        : ctl(D.ctl), x(D.x), rec(D.rec), itile(D.itile), nodes(D.mos_nodes), pos(D.mos_pos), rpos(D.rmos_pos),
+          rec_of(D.rec_of), mstate(D.mstate), cache(D.cache), contrib(D.contrib), rcontrib(D.rcontrib),
+          noncon(D.noncon), C(D.C), N(D.N), NM(D.NM), NS(D.NS), NA(D.NA), NR(D.NR), reltol(D.reltol),
+          abstol(D.abstol)
+    {
+    }
+};
+
+/* one MOSFET of circuit c at place j of its storage, in lane `lane` of
+ * tile `tile`; K the circuit's control block (in the constant address space
+ * where the whole wave shares it) */
+template <int FL, class P, class KP>
+__device__ __forceinline__ int tran_mos_one(const P &prm, const MosArgs &A, KP K, int c, int j, int64_t tile,
+                                            unsigned lane)
 {
-    const int64_t cnm = (int64_t)D.C * D.NM;
-    if (i >= cnm) return;
-    const int c = (int)(i / D.NM);
-    const int j = (int)(i - (int64_t)c * D.NM);
-    const CktCtl *K = D.ctl + c;
-    /* pvhold: the circuit's iteration continues with the loads it has */
-    if (K->phase >= PH_DONE || K->pvhold) return;
     B4Ckt ck;
-    /* a circuit whose step starts from the learned guess (set by
-     * k_guess_features this pass) limits against its last accepted point */
+    /* a circuit whose step starts from the learned guess (set when it asked
+     * for it) limits against its last accepted point */
     ck.mode = K->mode | (K->guess == 1 ? M_GUESSED : 0);
     ck.order = K->order;
     ck.method = K->method;
@@ -86,52 +103,109 @@ __device__ __forceinline__ void tran_mos_body(const B4Tab &tab, const TranDev &D
     for (int k = 0; k < 7; k++) ck.ag[k] = K->ag[k];
     ck.xfact = K->delta / K->deltaOld[1];
     ck.gmin = K->gminCur;
-    ck.reltol = D.reltol;
-    ck.abstol = D.abstol;
-    const double *xo = D.x + ((int64_t)K->xsel * D.C + c) * (D.N + 1);
+    ck.reltol = A.reltol;
+    ck.abstol = A.abstol;
+    const NGMI_GLOBAL int *nd = (const NGMI_GLOBAL int *)A.nodes;
+    const NGMI_GLOBAL double *xo = (const NGMI_GLOBAL double *)A.x + ((int64_t)K->xsel * A.C + c) * (A.N + 1);
     double v[4];
 #pragma unroll
-    for (int r = 0; r < 4; r++) v[r] = xo[D.mos_nodes[r * D.NM + j]];
-    TranPrm p{tab, i, tab.model_of[i]};
-    TranState st{D.mstate, cnm, i, K->rb};
-    TranCache ca{D.cache, cnm, i};
+    for (int r = 0; r < 4; r++) v[r] = xo[nd[r * A.NS + j]];
+    TranState st{(NGMI_GLOBAL double *)A.mstate + tile * (NLEV * MOS_ROWS * MOS_TILE), lane, K->rb};
+    TranCache ca{(NGMI_GLOBAL double *)A.cache + tile * (B4C__COUNT * MOS_TILE), lane};
     double J[B4S__COUNT], R[B4R__COUNT];
-    const int nc = b4_load<FL>(p, st, ca, ck, v, J, R);
+    const int nc = b4_load<FL>(prm, st, ca, ck, v, J, R);
     /* straight into the circuit's assembly-ordered contribution arrays */
-    double *ca_ = D.contrib + (int64_t)c * D.NA;
-    double *cr_ = D.rcontrib + (int64_t)c * D.NR;
+    NGMI_GLOBAL double *ca_ = (NGMI_GLOBAL double *)A.contrib + (int64_t)c * A.NA;
+    NGMI_GLOBAL double *cr_ = (NGMI_GLOBAL double *)A.rcontrib + (int64_t)c * A.NR;
+    const NGMI_GLOBAL int *pos = (const NGMI_GLOBAL int *)A.pos, *rpos = (const NGMI_GLOBAL int *)A.rpos;
 #pragma unroll
     for (int k = 0; k < B4S__COUNT; k++) {
-        const int p = D.mos_pos[k * D.NM + j];
+        const int p = pos[k * A.NS + j];
         if (p >= 0) ca_[p] = J[k];
     }
 #pragma unroll
     for (int k = 0; k < B4R__COUNT; k++) {
-        const int p = D.rmos_pos[k * D.NM + j];
+        const int p = rpos[k * A.NS + j];
         if (p >= 0) cr_[p] = R[k];
     }
-    D.noncon[i] = nc;
+    return nc;
 }
 
-/* one topology: the descriptor is a kernel argument, so every table pointer
- * is known to address global memory */
-template <int WAVES, int FL>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))
-k_tran_mos(B4Tab tab, TranDev D, int64_t i0, int64_t i1)
+/* padded storage: the wave is tile w of circuit c, one circuit and one
+ * record, so the control block and the record are scalar.
+ * pvhold: the circuit's iteration continues with the loads it has. */
+template <int FL, int NC>
+__device__ __forceinline__ void tran_mos_tile(const MosArgs &A, int c, int w)
 {
-    const int64_t i = i0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < i1) tran_mos_body<FL>(tab, D, i);
+    const NGMI_CONST CktCtl *K = (const NGMI_CONST CktCtl *)A.ctl + c;
+    if (K->phase >= PH_DONE || K->pvhold) return;
+    const int W = A.NS / MOS_TILE;
+    const unsigned lane = threadIdx.x;
+    const int j = w * MOS_TILE + (int)lane;
+    const int64_t tile = (int64_t)c * W + w;
+    int nc = 0;
+    if (((const NGMI_GLOBAL int *)A.nodes)[j] >= 0) {
+        const int r = ((const NGMI_CONST int *)A.rec_of)[tile];
+        RecPrm<NC, true> p{(const NGMI_CONST double *)A.rec + (int64_t)r * B4F__COUNT,
+                           (const NGMI_GLOBAL double *)A.itile + tile * (B4_NC_GEOM * MOS_TILE), lane};
+        nc = tran_mos_one<FL>(p, A, K, c, j, tile, lane);
+    }
+    const bool any = __ballot(nc != 0) != 0;
+    if (lane == 0) ((NGMI_GLOBAL int *)A.noncon)[tile] = any;
 }
 
-/* several topologies in one launch: blk[b] = (group, first block of the
- * group) */
-template <int WAVES>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))
-k_tran_mos_groups(const B4Tab *__restrict__ tabs, const TranDev *__restrict__ Ds,
-                  const int2 *__restrict__ blk)
+/* dense storage: places i = tile * 64 + lane, each lane its own circuit and
+ * record (or, in the column form of the table, its own columns) */
+template <int FL, bool COLS>
+__device__ __forceinline__ void tran_mos_dense(const MosArgs &A, const B4Tab &tab, int64_t tile, int64_t i_begin,
+                                               int64_t i_end)
 {
-    const int2 bg = blk[blockIdx.x];
-    tran_mos_body<-1>(tabs[bg.x], Ds[bg.x], (int64_t)(blockIdx.x - bg.y) * blockDim.x + threadIdx.x);
+    const unsigned lane = threadIdx.x;
+    const int64_t i = tile * MOS_TILE + lane;
+    if (i < i_begin || i >= i_end) return;
+    const int c = (int)(i / A.NM);
+    const int j = (int)(i - (int64_t)c * A.NM);
+    const NGMI_GLOBAL CktCtl *K = (const NGMI_GLOBAL CktCtl *)A.ctl + c;
+    if (K->phase >= PH_DONE || K->pvhold) return;
+    int nc;
+    if constexpr (COLS) {
+        TranPrm p{tab, i, tab.model_of[i]};
+        nc = tran_mos_one<FL>(p, A, K, c, j, tile, lane);
+    } else {
+        RecPrm<B4_NC_GEOM, false> p{(const NGMI_GLOBAL double *)A.rec +
+                                        (int64_t)((const NGMI_GLOBAL int *)A.rec_of)[i] * B4F__COUNT,
+                                    (const NGMI_GLOBAL double *)A.itile + tile * (B4_NC_GEOM * MOS_TILE), lane};
+        nc = tran_mos_one<FL>(p, A, K, c, j, tile, lane);
+    }
+    ((NGMI_GLOBAL int *)A.noncon)[i] = nc;
+}
+
+/* padded storage, a workgroup per tile: blk[b] = (group, circuit, tile of
+ * the circuit) */
+template <int WAVES, int FL, int NC>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))
+k_tran_mos(const TranDev *__restrict__ Ds, const int4 *__restrict__ blk)
+{
+    const NGMI_CONST int *b = (const NGMI_CONST int *)(blk + blockIdx.x);
+    tran_mos_tile<FL, NC>(MosArgs(Ds[b[0]]), b[1], b[2]);
+}
+
+/* dense storage, a workgroup per tile: blk[b] = (group, tile), places
+ * [i0, i1) of the group; without blk group 0's tiles from i0's on */
+template <int WAVES, int FL, bool COLS>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))
+k_tran_mos_dense(const TranDev *__restrict__ Ds, const B4Tab *__restrict__ tabs, const int4 *__restrict__ blk,
+                 int64_t i0, int64_t i1)
+{
+    int g = 0;
+    int64_t tile = i0 / MOS_TILE + blockIdx.x;
+    if (blk) {
+        const NGMI_CONST int *b = (const NGMI_CONST int *)(blk + blockIdx.x);
+        g = b[0];
+        tile = b[1];
+    }
+    const MosArgs A(Ds[g]);
+    tran_mos_dense<FL, COLS>(A, tabs[g], tile, i0, min(i1, (int64_t)A.C * A.NM));
 }
 
 /* ---------------- scalar helpers (thread 0 of a circuit) ---------------- */
@@ -582,27 +656,29 @@ __device__ __forceinline__ void op_memory(const TranDev &D, int c, const CktCtl 
 {
     if (what == OPA_NONE) return;
     const int tid = threadIdx.x, nt = blockDim.x, N = D.N;
-    const int64_t cnm = (int64_t)D.C * D.NM, cnc = (int64_t)D.C * D.NCAP;
+    const int64_t cnc = (int64_t)D.C * D.NCAP;
     double *x = D.x + ((int64_t)K->xsel * D.C + c) * (N + 1);
     double *bx = D.bak_x + (int64_t)c * (N + 1);
-    double *bs = D.bak_s + (int64_t)c * (B4X__COUNT * D.NM + 2 * D.NCAP);
+    double *bs = D.bak_s + (int64_t)c * (B4X__COUNT * D.NS + 2 * D.NCAP);
     const int l0 = lvl(K->rb, 0);
     for (int u = tid; u <= N; u += nt) {
         if (what == OPA_ZERO) x[u] = 0.0;
         else if (what == OPA_SAVE) bx[u] = x[u];
         else x[u] = bx[u];
     }
-    for (int q = tid; q < B4X__COUNT * D.NM; q += nt) {
-        const int k = q / D.NM, j = q - k * D.NM;
-        double *p = D.mstate + ((int64_t)l0 * B4X__COUNT + k) * cnm + (int64_t)c * D.NM + j;
-        if (what == OPA_ZERO) *p = 0.0;
-        else if (what == OPA_SAVE) bs[q] = *p;
-        else *p = bs[q];
+    for (int j = tid; j < D.NS; j += nt) {
+        double *p = D.mstate + mos_at((int64_t)c * D.NS + j, l0, 0);
+        double *b = bs + j;
+        for (int k = 0; k < B4X__COUNT; k++) {
+            if (what == OPA_ZERO) p[k * MOS_TILE] = 0.0;
+            else if (what == OPA_SAVE) b[k * D.NS] = p[k * MOS_TILE];
+            else p[k * MOS_TILE] = b[k * D.NS];
+        }
     }
     for (int q = tid; q < 2 * D.NCAP; q += nt) {
         const int k = q / D.NCAP, j = q - k * D.NCAP;
         double *p = D.cstate + ((int64_t)l0 * 2 + k) * cnc + (int64_t)c * D.NCAP + j;
-        double *b = bs + B4X__COUNT * D.NM + q;
+        double *b = bs + B4X__COUNT * D.NS + q;
         if (what == OPA_ZERO) *p = 0.0;
         else if (what == OPA_SAVE) *b = *p;
         else *p = *b;
@@ -622,7 +698,7 @@ __device__ double wave_min(double v)
 __device__ __forceinline__ double circuit_terr(const TranDev &D, const CktCtl *K, int c)
 {
     const int rb = K->rb, order = K->order;
-    const int64_t cnm = (int64_t)D.C * D.NM, cnc = (int64_t)D.C * D.NCAP;
+    const int64_t cnc = (int64_t)D.C * D.NCAP;
     double m = 1e308;
     for (int k = threadIdx.x; k < D.NCAP; k += blockDim.x) {
         const int64_t ci = (int64_t)c * D.NCAP + k;
@@ -634,16 +710,26 @@ __device__ __forceinline__ double circuit_terr(const TranDev &D, const CktCtl *K
         const double c1 = Q[((int64_t)lvl(rb, 1) * 2 + 1) * cnc];
         m = fmin(m, terr_one(q0, q1, q2, q3, c0, c1, K, D));
     }
-    for (int t = threadIdx.x; t < 3 * D.NM; t += blockDim.x) {
-        const int j = t / 3, r = t - 3 * j;
-        const int which = r == 0 ? B4X_qb : (r == 1 ? B4X_qg : B4X_qd);
-        const int64_t mi = (int64_t)c * D.NM + j;
-        const double *Q = D.mstate + (int64_t)which * cnm + mi;
-        const int64_t lv = (int64_t)B4X__COUNT * cnm;
-        const double q0 = Q[lvl(rb, 0) * lv], q1 = Q[lvl(rb, 1) * lv], q2 = Q[lvl(rb, 2) * lv];
-        const double q3 = order > 1 ? Q[lvl(rb, 3) * lv] : 0.0;
-        const double c0 = Q[lvl(rb, 0) * lv + cnm], c1 = Q[lvl(rb, 1) * lv + cnm];
-        m = fmin(m, terr_one(q0, q1, q2, q3, c0, c1, K, D));
+    /* qb, qg and qd of each MOSFET (holes hold zeros, whose bound is that of a
+     * constant charge) */
+    for (int j = threadIdx.x; j < D.NS; j += blockDim.x) {
+        const NGMI_GLOBAL double *Q =
+            (const NGMI_GLOBAL double *)D.mstate + mos_at((int64_t)c * D.NS + j, 0, B4X_qb);
+        constexpr int lv = MOS_ROWS * MOS_TILE;
+        const int l0 = lvl(rb, 0) * lv, l1 = lvl(rb, 1) * lv, l2 = lvl(rb, 2) * lv, l3 = lvl(rb, 3) * lv;
+        double q0[3], q1[3], q2[3], q3[3], c0[3], c1[3];
+#pragma unroll
+        for (int r = 0; r < 3; r++) {   /* rows qb cqb qg cqg qd cqd */
+            const int k = 2 * r * MOS_TILE;
+            q0[r] = Q[l0 + k];
+            q1[r] = Q[l1 + k];
+            q2[r] = Q[l2 + k];
+            q3[r] = order > 1 ? Q[l3 + k] : 0.0;
+            c0[r] = Q[l0 + k + MOS_TILE];
+            c1[r] = Q[l1 + k + MOS_TILE];
+        }
+#pragma unroll
+        for (int r = 0; r < 3; r++) m = fmin(m, terr_one(q0[r], q1[r], q2[r], q3[r], c0[r], c1[r], K, D));
     }
     return wave_min(m);
 }
@@ -651,13 +737,12 @@ __device__ __forceinline__ double circuit_terr(const TranDev &D, const CktCtl *K
 /* copy state level `from` to level `to` for every state of the circuit */
 __device__ __forceinline__ void copy_level(const TranDev &D, int c, int rb, int from, int to)
 {
-    const int64_t cnm = (int64_t)D.C * D.NM, cnc = (int64_t)D.C * D.NCAP;
+    const int64_t cnc = (int64_t)D.C * D.NCAP;
     const int pf = lvl(rb, from), pt = lvl(rb, to);
-    for (int t = threadIdx.x; t < B4X__COUNT * D.NM; t += blockDim.x) {
-        const int k = t / D.NM, j = t - k * D.NM;
-        const int64_t mi = (int64_t)c * D.NM + j;
-        D.mstate[((int64_t)pt * B4X__COUNT + k) * cnm + mi] =
-            D.mstate[((int64_t)pf * B4X__COUNT + k) * cnm + mi];
+    for (int j = threadIdx.x; j < D.NS; j += blockDim.x) {
+        const double *a = D.mstate + mos_at((int64_t)c * D.NS + j, pf, 0);
+        double *b = D.mstate + mos_at((int64_t)c * D.NS + j, pt, 0);
+        for (int k = 0; k < B4X__COUNT; k++) b[k * MOS_TILE] = a[k * MOS_TILE];
     }
     for (int t = threadIdx.x; t < 2 * D.NCAP; t += blockDim.x) {
         const int k = t / D.NCAP, j = t - k * D.NCAP;
@@ -1471,7 +1556,7 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
     const int mode = K->mode, rb = K->rb, xs = K->xsel;
     /* OPtran steps its own time; the sources stay at CKTtime, 0 */
     const double tnow = K->optran ? 0.0 : K->time;
-    const int64_t cnm = (int64_t)D.C * D.NM, cnc = (int64_t)D.C * D.NCAP;
+    const int64_t cnc = (int64_t)D.C * D.NCAP;
     double *xo = D.x + ((int64_t)xs * D.C + c) * (N + 1);
     double *xn = D.x + ((int64_t)(xs ^ 1) * D.C + c) * (N + 1);
     if (tid < 4) s_flag[tid] = 0;
@@ -1834,11 +1919,11 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
             }
         }
         int vote = 0;
-        const int *nc = D.noncon + (int64_t)c * D.NM;
-        for (int j0 = tid; j0 < D.NM; j0 += CONV_CHUNK * nt) {
+        const int *nc = D.noncon + (int64_t)c * D.NV;
+        for (int j0 = tid; j0 < D.NV; j0 += CONV_CHUNK * nt) {
             int v[CONV_CHUNK];
     #pragma unroll
-            for (int k = 0; k < CONV_CHUNK; k++) v[k] = (j0 + k * nt < D.NM) ? gload(nc + j0 + k * nt) : 0;
+            for (int k = 0; k < CONV_CHUNK; k++) v[k] = (j0 + k * nt < D.NV) ? gload(nc + j0 + k * nt) : 0;
     #pragma unroll
             for (int k = 0; k < CONV_CHUNK; k++) vote |= v[k];
         }
@@ -2165,40 +2250,49 @@ int set_tran_lds_limit(size_t bytes)
 }
 
 /* one Newton pass over every circuit of every topology group; with one
- * group (tab0, D0 set) the descriptor goes by value and the pass covers
- * circuits [c_begin, c_end).  ev (optional) = 3
- * events recorded before the MOSFET kernel, between the two kernels and
- * after the step kernel. */
-int launch_tran_pass(const B4Tab *tab0, const TranDev *D0, int c_begin, int c_end, const B4Tab *tabs,
-                     const TranDev *Ds, const int2 *mos_blk, int n_mos_blk, const int2 *step_blk,
-                     int n_step_blk, size_t lds_bytes, hipStream_t s, hipEvent_t *ev)
+ * group (D0 set) the step kernel's descriptor goes by value and the pass
+ * covers circuits [c_begin, c_end).  ev (optional) = 3 events recorded before
+ * the MOSFET kernel, between the two kernels and after the step kernel. */
+int launch_tran_pass(const MosLaunch &M, const TranDev *D0, int c_begin, int c_end, const TranDev *Ds,
+                     const int2 *step_blk, int n_step_blk, size_t lds_bytes, hipStream_t s, hipEvent_t *ev)
 {
-    /* mos_waves 0 (the default): one wave on a single 101-stage ring, 49.7
-     * against 53.2 us per launch with two */
-    const int waves = waves_for(TUNE_MOS_WAVES, D0 ? (int64_t)(c_end - c_begin) * D0->NM : (int64_t)n_mos_blk * 256);
     if (ev) NGMI_HIP(hipEventRecord(ev[0], s));
-    if (n_mos_blk > 0) {
-        const dim3 g((unsigned)n_mos_blk);
-        if (D0) {
-            const int64_t i0 = (int64_t)c_begin * D0->NM, i1 = (int64_t)c_end * D0->NM;
-            const dim3 gh((unsigned)((i1 - i0 + 255) / 256));
-            /* the default card's selectors compiled as constants when the
-             * whole set shares them */
-            const bool dflt = tab0->flags == B4FL_DEFAULT && tune_get(TUNE_SPECIALISE);
-            if (i1 > i0) {
-#define NGMI_MOS(W, F) hipLaunchKernelGGL((k_tran_mos<W, F>), gh, dim3(256), 0, s, *tab0, *D0, i0, i1)
-                switch (waves) {
-                case 1: if (dflt) NGMI_MOS(1, B4FL_DEFAULT); else NGMI_MOS(1, -1); break;
-                case 3: if (dflt) NGMI_MOS(3, B4FL_DEFAULT); else NGMI_MOS(3, -1); break;
-                case 4: if (dflt) NGMI_MOS(4, B4FL_DEFAULT); else NGMI_MOS(4, -1); break;
-                default: if (dflt) NGMI_MOS(2, B4FL_DEFAULT); else NGMI_MOS(2, -1); break;
-                }
+    const bool padded = M.mode == B4T_UNIFORM;
+    int64_t i0 = 0, i1 = INT64_MAX, blocks = M.nblk;
+    const int4 *blk = M.blk;
+    if (D0 && padded) {
+        blocks = (int64_t)(c_end - c_begin) * D0->W;
+        blk += (int64_t)c_begin * D0->W;
+    } else if (D0) {
+        i0 = (int64_t)c_begin * D0->NM;
+        i1 = (int64_t)c_end * D0->NM;
+        blocks = i1 > i0 ? (i1 + MOS_TILE - 1) / MOS_TILE - i0 / MOS_TILE : 0;
+        blk = nullptr;
+    }
+    if (blocks > 0) {
+        const dim3 g((unsigned)blocks), wg(64);
+        const int waves = waves_for(TUNE_MOS_WAVES, blocks * 64);
+        /* the default card's selectors compiled as constants when the whole
+         * batch shares them */
+        const bool dflt = M.flags == B4FL_DEFAULT && tune_get(TUNE_SPECIALISE);
+#define NGMI_MOS(W, ...) hipLaunchKernelGGL((k_tran_mos<W, __VA_ARGS__>), g, wg, 0, s, Ds, blk)
+#define NGMI_MOS_DENSE(W, ...) \
+    hipLaunchKernelGGL((k_tran_mos_dense<W, __VA_ARGS__>), g, wg, 0, s, Ds, M.tabs, blk, i0, i1)
+#define NGMI_W(MACRO, ...) \
+    do { \
+        if (waves == 1) MACRO(1, __VA_ARGS__); \
+        else MACRO(2, __VA_ARGS__); \
+    } while (0)
+        if (M.mode == B4T_COLUMNS) NGMI_W(NGMI_MOS_DENSE, -1, true);
+        else if (M.mode == B4T_LANES && dflt) NGMI_W(NGMI_MOS_DENSE, B4FL_DEFAULT, false);
+        else if (M.mode == B4T_LANES) NGMI_W(NGMI_MOS_DENSE, -1, false);
+        else if (!dflt) NGMI_W(NGMI_MOS, -1, B4_NC_GEOM);
+        else if (M.nc == 0) NGMI_W(NGMI_MOS, B4FL_DEFAULT, 0);
+        else if (M.nc == B4_NC_LD) NGMI_W(NGMI_MOS, B4FL_DEFAULT, B4_NC_LD);
+        else NGMI_W(NGMI_MOS, B4FL_DEFAULT, B4_NC_GEOM);
+#undef NGMI_W
+#undef NGMI_MOS_DENSE
 #undef NGMI_MOS
-            }
-        } else {
-            if (waves == 1) hipLaunchKernelGGL(k_tran_mos_groups<1>, g, dim3(256), 0, s, tabs, Ds, mos_blk);
-            else hipLaunchKernelGGL(k_tran_mos_groups<2>, g, dim3(256), 0, s, tabs, Ds, mos_blk);
-        }
         NGMI_HIP(hipGetLastError());
     }
     if (ev) NGMI_HIP(hipEventRecord(ev[1], s));

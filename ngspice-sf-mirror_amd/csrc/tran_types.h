@@ -9,6 +9,7 @@
 
 #include <cstdint>
 #include <hip/hip_runtime.h>
+#include "ngmi_internal.h"
 
 namespace ngmi {
 
@@ -81,6 +82,16 @@ enum : int {
     OP_S3_GMIN = 8, OP_S3_GMIN_FINAL = 9, OP_S3_SRC = 10
 };
 
+/* place i of the MOSFET storage, level l (physical), state row k: state rows
+ * of one tile and level are contiguous, so a wavefront reaches them from one
+ * base at constant offsets */
+constexpr int MOS_TILE = 64;
+constexpr int MOS_ROWS = 29;   /* B4X__COUNT */
+__host__ __device__ inline int64_t mos_at(int64_t i, int l, int k)
+{
+    return (((i / MOS_TILE) * NLEV + l) * MOS_ROWS + k) * MOS_TILE + i % MOS_TILE;
+}
+
 /* contribution codes of the assembly plans */
 enum : uint32_t {
     CT_MOS = 0u, CT_CAP = 1u, CT_RES = 2u, CT_ONE = 3u, CT_VSRC = 4u, CT_ZERO = 5u,
@@ -94,6 +105,18 @@ struct TranDev {
     int N;            /* unknowns (1..N, 0 = ground) */
     int NN;           /* node unknowns (1..NN); N - NN branch unknowns */
     int NM, NCAP, NRES, NVS;
+    /* MOSFET storage: circuit c's MOSFETs occupy places c NS .. c NS + NS - 1
+     * of arrays of 64-place tiles (MOS_TILE).  Padded storage: the circuit's
+     * MOSFETs are sorted by BSIM4 record and each record's part filled up
+     * with holes to whole tiles (NS = 64 W), so a wavefront of the BSIM4
+     * kernel belongs to one circuit and one record, and casts one vote
+     * (NV = W).  Dense storage: netlist order, NS = NM, a vote each (NV =
+     * NM). */
+    int NS, W, NV;
+    int64_t ntile;            /* tiles of the group */
+    const double *rec;        /* BSIM4 records, [records][B4F__COUNT] */
+    const double *itile;      /* per-instance columns, [tile][22][64] */
+    const int *rec_of;        /* record of each tile (padded) or place (dense) */
     int nslots;       /* nonzeros of L + U */
     int nlev_f, nlev_fw, nlev_bw;
     int nprobe;
@@ -105,9 +128,9 @@ struct TranDev {
     double opstep, opfinal;   /* optran's step and final time; opstep 0: deselected */
     const int *diag_slot;     /* [N+1] L+U slot of A(u, u), -1 where A has no such element */
     double *bak_x;            /* [C][N+1] CKTop's saved CKTrhsOld */
-    double *bak_s;            /* [C][29 NM + 2 NCAP] CKTop's saved CKTstate0 */
+    double *bak_s;            /* [C][29 NS + 2 NCAP] CKTop's saved CKTstate0 */
     /* topology (shared) */
-    const int *mos_nodes;     /* [4][NM] d g s b */
+    const int *mos_nodes;     /* [4][NS] d g s b, -1 at a hole */
     const int *cap_nodes;     /* [2][NCAP] */
     const int *res_nodes;     /* [2][NRES] */
     const int *vs_nodes;      /* [3][NVS] p n branch */
@@ -166,15 +189,15 @@ struct TranDev {
     /* state */
     CktCtl *ctl;              /* [C] */
     double *x;                /* [2][C][N+1] iterate buffers */
-    double *mstate;           /* [NLEV][29][C*NM] */
+    double *mstate;           /* MOSFET states, see mos_at */
     double *cstate;           /* [NLEV][2][C*NCAP] */
-    double *cache;            /* [38][C*NM] */
+    double *cache;            /* MOSFET caches, [tile][38][64] */
     int NA, NR;               /* a_code / r_code entries (contribution array lengths) */
-    const int *mos_pos;       /* [16 * NM] */
-    const int *rmos_pos;      /* [4 * NM] */
+    const int *mos_pos;       /* [16][NS] */
+    const int *rmos_pos;      /* [4][NS] */
     double *contrib;          /* [C][NA] */
     double *rcontrib;         /* [C][NR] */
-    int *noncon;              /* [C*NM] */
+    int *noncon;              /* [C][NV] votes */
     double *out_t;            /* [C][cap_pts] */
     double *out_x;            /* [C][cap_pts][nprobe] */
     int *done_count;          /* circuits finished or failed */
@@ -209,6 +232,18 @@ struct TranDev {
     int *pv_owner;
     int pv_slots, pv_ld;
     int64_t pv_stride;
+};
+
+/* how a batch's BSIM4 kernel is launched: the storage of its MOSFETs and
+ * the form of their tables (ngmi_internal.h's B4T_*: UNIFORM is padded
+ * storage, LANES and COLUMNS dense), the instance columns, the shared
+ * selector word or -1, and the workgroups' map: (group, circuit, tile of the
+ * circuit) in padded storage, (group, tile) in dense; tabs the column form's
+ * tables (device) */
+struct MosLaunch {
+    int mode = 0, nc = 0, flags = -1, nblk = 0;
+    const int4 *blk = nullptr;
+    const B4Tab *tabs = nullptr;
 };
 
 }  // namespace ngmi
