@@ -364,8 +364,7 @@ int splu_analyze(int n, const int64_t *Ap, const int *Ai, SpluSym &S)
     /* index lists, offsets, relative indices into the parent */
     S.off.resize(nfr);
     S.idx_off.resize(nfr + 1);
-    S.upd_off.resize(nfr + 1);
-    int64_t store = 0, ioff = 0, uoff = 0;
+    int64_t store = 0, ioff = 0;
     for (int f = 0; f < nfr; f++) {
         const int64_t nf = (int64_t)S.ns[f] + S.nb[f];
         if (nf > SPLU_MAX_FRONT) {
@@ -375,10 +374,8 @@ int splu_analyze(int n, const int64_t *Ap, const int *Ai, SpluSym &S)
         S.max_front = std::max(S.max_front, (int)nf);
         S.off[f] = store;
         S.idx_off[f] = ioff;
-        S.upd_off[f] = uoff;
         store += nf * nf;
         ioff += nf;
-        uoff += S.nb[f];
         S.lu_nnz += nf * nf - (int64_t)S.nb[f] * S.nb[f];
         for (int k = 0; k < S.ns[f]; k++) {
             const double rem = (double)(nf - k - 1);
@@ -386,7 +383,6 @@ int splu_analyze(int n, const int64_t *Ap, const int *Ai, SpluSym &S)
         }
     }
     S.idx_off[nfr] = ioff;
-    S.upd_off[nfr] = uoff;
     S.store = store;
     S.idx.resize(ioff);
     S.rel.assign(ioff, -1);
@@ -418,30 +414,107 @@ int splu_analyze(int n, const int64_t *Ap, const int *Ai, SpluSym &S)
         }
     }
 
-    /* every stored entry of B goes to the front that eliminates its earlier unknown */
-    S.ent_pos.resize(nnz);
+    /* every stored entry of B goes to the front that eliminates its earlier
+     * unknown: counted, then listed by front */
+    S.ent_ptr.assign(nfr + 1, 0);
+    S.ent_src.resize(nnz);
+    S.ent_rc.resize(nnz);
     for (int c = 0; c < n; c++)
         for (int64_t e = Ap[c]; e < Ap[c + 1]; e++) {
             const int r = S.rowsrc[Ai[e]];
-            const int v = pos[r] < pos[c] ? r : c;
-            const int f = fof[v];
-            const int ns = S.ns[f], nf = ns + S.nb[f];
-            const int *id = S.idx.data() + S.idx_off[f];
-            auto local = [&](int u) -> int {
-                if (pos[u] >= first[f] && pos[u] < first[f + 1]) return pos[u] - first[f];
-                const int *b = id + ns, *en = id + nf;
-                const int *it = std::lower_bound(b, en, u, [&](int a, int x) { return pos[a] < pos[x]; });
-                return (it != en && *it == u) ? (int)(it - id) : -1;
-            };
-            const int lr = local(r), lc = local(c);
-            if (lr < 0 || lc < 0) {
-                set_error("splu_analyze: entry (%d, %d) outside its front", r, c);
-                return NGMI_E_PANIC;
-            }
-            S.ent_pos[e] = S.off[f] + (int64_t)lc * nf + lr;
+            S.ent_ptr[fof[pos[r] < pos[c] ? r : c] + 1]++;
         }
+    for (int f = 0; f < nfr; f++) S.ent_ptr[f + 1] += S.ent_ptr[f];
+    {
+        std::vector<int64_t> w(S.ent_ptr.begin(), S.ent_ptr.end() - 1);
+        for (int c = 0; c < n; c++)
+            for (int64_t e = Ap[c]; e < Ap[c + 1]; e++) {
+                const int r = S.rowsrc[Ai[e]];
+                const int f = fof[pos[r] < pos[c] ? r : c];
+                const int ns = S.ns[f], nf = ns + S.nb[f];
+                const int *id = S.idx.data() + S.idx_off[f];
+                auto local = [&](int u) -> int {
+                    if (pos[u] >= first[f] && pos[u] < first[f + 1]) return pos[u] - first[f];
+                    const int *b = id + ns, *en = id + nf;
+                    const int *it = std::lower_bound(b, en, u, [&](int a, int x) { return pos[a] < pos[x]; });
+                    return (it != en && *it == u) ? (int)(it - id) : -1;
+                };
+                const int lr = local(r), lc = local(c);
+                if (lr < 0 || lc < 0) {
+                    set_error("splu_analyze: entry (%d, %d) outside its front", r, c);
+                    return NGMI_E_PANIC;
+                }
+                const int64_t q = w[f]++;
+                S.ent_src[q] = (int)e;
+                S.ent_rc[q] = (uint32_t)lr | (uint32_t)lc << 16;
+            }
+    }
+    /* the larger fronts' entries by column, and by column group the children
+     * with a boundary unknown in it */
+    S.cg_off.assign(nfr, 0);
+    S.gk_off.assign(nfr, 0);
+    {
+        std::vector<std::pair<uint32_t, int>> tmp;
+        std::vector<std::pair<int, int>> in;   /* (group, child) */
+        for (int f = 0; f < nfr; f++) {
+            const int nf = S.ns[f] + S.nb[f];
+            if (nf <= SPLU_SMALL) continue;
+            const int64_t b = S.ent_ptr[f], e = S.ent_ptr[f + 1];
+            tmp.clear();
+            for (int64_t q = b; q < e; q++) tmp.push_back({S.ent_rc[q], S.ent_src[q]});
+            std::sort(tmp.begin(), tmp.end());
+            for (int64_t q = b; q < e; q++) {
+                S.ent_rc[q] = tmp[q - b].first;
+                S.ent_src[q] = tmp[q - b].second;
+            }
+            in.clear();
+            for (int k = S.kid_ptr[f]; k < S.kid_ptr[f + 1]; k++) {
+                const int c = S.kids[k];
+                const int *rl = S.rel.data() + S.idx_off[c] + S.ns[c];   /* ascending */
+                for (int i = 0; i < S.nb[c]; i++)
+                    if (i == 0 || rl[i] / SPLU_CG != rl[i - 1] / SPLU_CG)
+                        in.push_back({rl[i] / SPLU_CG, k - S.kid_ptr[f]});
+            }
+            std::sort(in.begin(), in.end());
+            S.cg_off[f] = (int64_t)S.cg.size();
+            S.gk_off[f] = (int64_t)S.gk.size();
+            for (const auto &x : in) S.gk.push_back(x.second);
+            int64_t q = b;
+            size_t i = 0;
+            for (int g = 0; g <= (nf + SPLU_CG - 1) / SPLU_CG; g++) {
+                while (q < e && (int)(S.ent_rc[q] >> 16) < g * SPLU_CG) q++;
+                while (i < in.size() && in[i].first < g) i++;
+                S.cg.push_back((int)(q - b));
+                S.cg.push_back((int)i);
+            }
+        }
+    }
+    /* inverse of the children's relative indices; the fronts' records */
+    S.inv_off.assign(nfr, 0);
+    {
+        size_t all = 0;
+        for (int f = 0; f < nfr; f++) all += (size_t)(S.kid_ptr[f + 1] - S.kid_ptr[f]) * (S.ns[f] + S.nb[f]);
+        S.inv.reserve(all);
+        S.front.reserve(nfr);
+        S.kid.reserve(S.kids.size());
+    }
+    for (int f = 0; f < nfr; f++) {
+        const int nf = S.ns[f] + S.nb[f], nk = S.kid_ptr[f + 1] - S.kid_ptr[f];
+        S.inv_off[f] = (int64_t)S.inv.size();
+        S.front.push_back({S.ns[f], nf, nk, (int)(S.ent_ptr[f + 1] - S.ent_ptr[f]), S.off[f], S.idx_off[f],
+                           S.ent_ptr[f], S.inv_off[f], S.kid_ptr[f], S.cg_off[f], S.gk_off[f]});
+        for (int k = S.kid_ptr[f]; k < S.kid_ptr[f + 1]; k++) {
+            const int c = S.kids[k];
+            const size_t at = S.inv.size();
+            S.inv.resize(at + nf, -1);
+            const int *rl = S.rel.data() + S.idx_off[c] + S.ns[c];
+            for (int i = 0; i < S.nb[c]; i++) S.inv[at + rl[i]] = i;
+            const int nfc = S.ns[c] + S.nb[c];
+            S.kid.push_back({S.off[c] + (int64_t)S.ns[c] * nfc + S.ns[c], S.idx_off[c] + S.ns[c], nfc, 0});
+        }
+    }
 
-    /* levels by height; extend-add lists by (height of the parent, child slot) */
+    /* levels by height, fronts of one by size */
     S.H = 0;
     for (int f = 0; f < nfr; f++) S.H = std::max(S.H, S.height[f]);
     S.lev_ptr.assign(S.H + 2, 0);
@@ -452,20 +525,9 @@ int splu_analyze(int n, const int64_t *Ap, const int *Ai, SpluSym &S)
         std::vector<int> w(S.lev_ptr.begin(), S.lev_ptr.end() - 1);
         for (int f = 0; f < nfr; f++) S.lev[w[S.height[f]]++] = f;
     }
-    S.max_slots = 0;
-    for (int f = 0; f < nfr; f++) S.max_slots = std::max(S.max_slots, S.kid_ptr[f + 1] - S.kid_ptr[f]);
-    S.ea_ptr.assign((size_t)(S.H + 1) * S.max_slots + 1, 0);
-    S.ea.clear();
     for (int h = 0; h <= S.H; h++)
-        for (int s = 0; s < S.max_slots; s++) {
-            for (int q = S.lev_ptr[h]; q < S.lev_ptr[h + 1]; q++) {
-                const int f = S.lev[q];
-                if (S.kid_ptr[f] + s < S.kid_ptr[f + 1]) S.ea.push_back(S.kids[S.kid_ptr[f] + s]);
-            }
-            S.ea_ptr[(size_t)h * S.max_slots + s + 1] = (int)S.ea.size();
-        }
-    S.max_lev = 0;
-    for (int h = 0; h <= S.H; h++) S.max_lev = std::max(S.max_lev, S.lev_ptr[h + 1] - S.lev_ptr[h]);
+        std::stable_sort(S.lev.begin() + S.lev_ptr[h], S.lev.begin() + S.lev_ptr[h + 1],
+                         [&](int a, int b) { return S.ns[a] + S.nb[a] < S.ns[b] + S.nb[b]; });
     return NGMI_OK;
 }
 

@@ -11,10 +11,26 @@
 namespace ngmi {
 
 constexpr int SPLU_LEAF = 64;          /* nested dissection stops at this many vertices */
-constexpr int SPLU_NB = 32;            /* panel width of the front factorization */
-constexpr int SPLU_TILE = 32;          /* trailing-update tile edge (16 x 16 threads, 2 x 2 each) */
+/* fronts up to this many unknowns are assembled and factored in LDS by one
+ * workgroup (141 x 140 doubles = 154 KiB of the CU's 160) */
+constexpr int SPLU_SMALL = 140;
+constexpr int SPLU_NB = 64;            /* panel width of the larger fronts */
+constexpr int SPLU_CG = 16;            /* columns a workgroup assembles of a larger front */
 constexpr int SPLU_MAX_FRONT = 8000;   /* a front's right-hand side and the solve kernels'
                                           static LDS fit 64 KB */
+
+/* what the numeric kernels need of a front, in one record, and of each of
+ * its children (kid0 on): where the Schur complement starts in the store, its
+ * leading dimension, where its boundary's part of the solves' work vector
+ * starts */
+struct SpluFront {
+    int ns, nf, nkid, nent;
+    int64_t off, idx, ent, inv, kid0, cg, gk;
+};
+struct SpluKid {
+    int64_t schur, wk;
+    int ld, pad;
+};
 
 struct SpluSym {
     int n = 0;
@@ -24,16 +40,26 @@ struct SpluSym {
     std::vector<int> ns, nb, parent, height;
     std::vector<int64_t> off;            /* front storage offset (doubles), nf x nf column-major */
     std::vector<int64_t> idx_off;        /* index list offset, ns + nb entries */
-    std::vector<int64_t> upd_off;        /* forward-solve update vector offset, nb entries */
     std::vector<int> idx;                /* unknowns: pivots, then boundary by elimination order */
     std::vector<int> rel;                /* at a boundary slot: its index in the parent's list */
     std::vector<int> kid_ptr, kids;
-    std::vector<int64_t> ent_pos;        /* CSC entry -> front storage position */
+    /* CSC entries by front (that of the earlier eliminated unknown): source
+     * entry and local position, row | column << 16; in a larger front by
+     * column, cg[cg_off[f] + 2 g] = first entry (from ent_ptr[f]) of columns
+     * SPLU_CG g on, cg[.. + 2 g + 1] = first (from gk_off[f]) of the children
+     * with a boundary unknown among them, listed in gk */
+    std::vector<int64_t> ent_ptr, cg_off, gk_off;
+    std::vector<int> ent_src, cg, gk;
+    std::vector<SpluFront> front;
+    std::vector<SpluKid> kid;
+    std::vector<uint32_t> ent_rc;
+    /* at inv_off[f] + q nf + r the boundary index in child q of the front's
+     * local unknown r, or -1 */
+    std::vector<int64_t> inv_off;
+    std::vector<int> inv;
     int H = 0;                           /* largest height */
-    std::vector<int> lev_ptr, lev;       /* fronts by height */
-    int max_slots = 0;                   /* most children of one front */
-    std::vector<int> ea_ptr, ea;         /* children by (parent height, child slot) */
-    int max_lev = 0, max_front = 0;
+    std::vector<int> lev_ptr, lev;       /* fronts by height, by size within one */
+    int max_front = 0;
     int64_t store = 0, lu_nnz = 0;
     double flops = 0;
 };

@@ -169,3 +169,50 @@ def test_concurrent_with_a_transient_batch():
         t, x = b2.waveform(c)
         assert np.array_equal(t, alone[c][0]) and np.array_equal(x, alone[c][1])
     print('6 concurrent refactor+solves and 4 ring waveforms identical to the runs alone', flush=True)
+
+
+def _bordered(leaves, chain, border, touch, seed):
+    """leaves chains of unknowns, each tied to touch of the border's, which
+    is dense; diagonally dominant by rows and columns"""
+    g = workloads.rng(seed, leaves)
+    n, base = leaves * chain + border, np.arange(leaves) * chain
+    r, c = [], []
+    for i in range(1, chain):
+        r += [base + i, base + i - 1]
+        c += [base + i - 1, base + i]
+    for t in range(touch):
+        x = leaves * chain + g.integers(0, border, leaves)
+        r += [base + t % chain, x]
+        c += [x, base + t % chain]
+    e = leaves * chain + np.arange(border)
+    r, c = np.concatenate(r + [np.repeat(e, border)]), np.concatenate(c + [np.tile(e, border)])
+    A = sp.csc_matrix((g.uniform(-1, 1, len(r)), (r, c)), shape=(n, n))
+    d = 1.0 + np.asarray(abs(A).sum(axis=0)).ravel() + np.asarray(abs(A).sum(axis=1)).ravel()
+    A = sp.csc_matrix(A + sp.diags(d))
+    A.sort_indices()
+    return A
+
+
+# one front (leaves 0) around the 16-pivot steps, the 64-pivot panels, the
+# edges of 64-row chunks and the 140 unknowns one workgroup takes; trees whose
+# root gathers from many children, in LDS and 16 columns a workgroup
+@pytest.mark.parametrize('leaves,chain,border,touch', [
+    (0, 1, n, 0) for n in (1, 2, 15, 16, 17, 33, 63, 64, 65, 129, 139, 140, 141, 142, 192, 193, 257, 391)
+] + [(200, 4, 8, 2), (900, 3, 60, 3), (1000, 4, 130, 6), (1000, 4, 300, 6), (5000, 3, 100, 3), (64, 1, 65, 1)])
+def test_front_sizes(leaves, chain, border, touch):
+    print('case: %d leaves of %d, %d of a border of %d each' % (leaves, chain, touch, border), flush=True)
+    A = _bordered(leaves, chain, border, touch, 11) if leaves else _bordered(1, 1, max(border - 1, 1), 1, 11)
+    if border == 1 and not leaves:
+        A = A[:1, :1].tocsc()
+    n = A.shape[0]
+    b = workloads.rng(12, n).uniform(-1, 1, n)
+    s = ngmi.SparseLU(n, A.indptr.astype(np.int64), A.indices.astype(np.int32))
+    x = _gpu(s, A.data, b)
+    print('n %d, %s' % (n, s.info()), flush=True)
+    # |b - A x| <= 3 n u |L||U||x|; with diagonals above their row's and
+    # column's sums |L||U| stays below 2 |A|
+    na = abs(A).sum(axis=1).max()
+    assert np.abs(A @ x - b).max() <= 6 * n * 2.0 ** -53 * na * np.abs(x).max()
+    ref = spla.spsolve(A, b)
+    assert np.abs(x - ref).max() <= 12 * n * 2.0 ** -53 * na * np.abs(ref).max()   # |A^-1| <= 1
+    assert np.array_equal(x, _gpu(s, A.data, b))
