@@ -15,20 +15,13 @@
 #include "mlp_types.h"
 
 namespace ngmi {
-int launch_gemm_bf16(const unsigned short *A, int64_t as0, int64_t as1, const unsigned short *B,
-                     int64_t bs0, int64_t bs1, const float *bias, float *Z, float *C,
-                     unsigned short *Cb, int ldc, int M, int N, int K, int epi, hipStream_t s,
-                     const int *Mdev = nullptr);
+int launch_gemm_bf16(const unsigned short *A, const unsigned short *B, const float *bias, unsigned short *Cb, int M,
+                     int N, int K, hipStream_t s, const int *Mdev);
 __global__ void k_f32_to_bf16(const float *x, unsigned short *y, int64_t n);
-__global__ void k_silu_back(const float *dY, const float *Z, float *dZ, unsigned short *dZb,
-                            int64_t n);
-int launch_colsum(const float *Xf, const unsigned short *Xb, const float *wt, float *part, float *out,
-                  int M, int N, hipStream_t s);
-__global__ void k_adam(float *w, unsigned short *wb, const float *g, float *m, float *v, int64_t n,
-                       float lr, float b1, float b2, float eps, float c1, float c2);
-__global__ void k_head(const unsigned short *H, const unsigned short *w, const float *b,
-                       const float *target, float *y, float *dy, int M, int K, const int *Mdev);
-__global__ void k_head_back(const unsigned short *w, const float *dy, float *dH, int M, int K);
+__global__ void k_train_transpose(const unsigned short *wb, unsigned short *wbt);
+int launch_train_step(const TrainBufs &B, const float *X, const float *target, int M, const AdamStep &A, hipStream_t s);
+__global__ void k_head(const unsigned short *H, const unsigned short *w, const float *b, float *y, int M, int K,
+                       const int *Mdev);
 int launch_guess_net(const unsigned short *wb, const float *wf, const float *X, int *count, int maxRows,
                      const int64_t *dest, const double2 *base, double *x, float *yout,
                      unsigned long long *rows_total, hipStream_t s);
@@ -46,19 +39,17 @@ constexpr int64_t OFF_W1 = MLP_OFF_W1, OFF_B1 = MLP_OFF_B1, OFF_W2 = MLP_OFF_W2,
 
 struct ngmi_mlp {
     float *w = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;   /* NPARAM each */
-    unsigned short *wb = nullptr;                                   /* BF16 copy */
-    int cap = 0;                                                    /* rows allocated */
-    unsigned short *xb = nullptr, *h1 = nullptr, *h2 = nullptr, *h3 = nullptr, *dzb = nullptr;
-    float *z1 = nullptr, *z2 = nullptr, *z3 = nullptr, *dh = nullptr, *dz = nullptr;
-    float *y = nullptr, *dy = nullptr;
-    float *part = nullptr;                                          /* column-sum partials */
+    unsigned short *wb = nullptr, *wbt = nullptr;                   /* BF16 copy; W2, W3 transposed */
+    int cap = 0;                                                    /* training rows allocated */
+    unsigned short *xo = nullptr, *h1 = nullptr, *h2 = nullptr, *dz1 = nullptr, *dz2 = nullptr, *dz3 = nullptr;
+    float *y = nullptr, *cols = nullptr, *dw = nullptr;
     int64_t step = 0;
     /* inference-only buffers (BF16 activations, ping-pong) */
     int icap = 0;
     unsigned short *ixb = nullptr, *ia = nullptr, *ib = nullptr;
     ~ngmi_mlp()
     {
-        void *ps[] = {w, g, m, v, wb, xb, h1, h2, h3, dzb, z1, z2, z3, dh, dz, y, dy, part, ixb, ia, ib};
+        void *ps[] = {w, g, m, v, wb, wbt, xo, h1, h2, dz1, dz2, dz3, y, cols, dw, ixb, ia, ib};
         for (void *p : ps) (void)hipFree(p);
     }
     int ensure_infer(int rows)
@@ -72,25 +63,20 @@ struct ngmi_mlp {
         icap = rows;
         return NGMI_OK;
     }
-    int ensure(int rows)
+    int ensure(int rows)   /* a multiple of 32 */
     {
         if (rows <= cap) return NGMI_OK;
-        void *ps[] = {xb, h1, h2, h3, dzb, z1, z2, z3, dh, dz, y, dy};
-        for (void *p : ps) (void)hipFree(p);
+        cap = 0;
+        void **ps[] = {(void **)&xo, (void **)&h1, (void **)&h2, (void **)&dz1, (void **)&dz2, (void **)&dz3,
+                       (void **)&y, (void **)&cols, (void **)&dw};
         const size_t r = (size_t)rows;
-        NGMI_HIP(hipMalloc(&xb, r * IN_PAD * 2));
-        NGMI_HIP(hipMalloc(&h1, r * H * 2));
-        NGMI_HIP(hipMalloc(&h2, r * H * 2));
-        NGMI_HIP(hipMalloc(&h3, r * H * 2));
-        NGMI_HIP(hipMalloc(&dzb, r * H * 2));
-        NGMI_HIP(hipMalloc(&z1, r * H * 4));
-        NGMI_HIP(hipMalloc(&z2, r * H * 4));
-        NGMI_HIP(hipMalloc(&z3, r * H * 4));
-        NGMI_HIP(hipMalloc(&dh, r * H * 4));
-        NGMI_HIP(hipMalloc(&dz, r * H * 4));
-        NGMI_HIP(hipMalloc(&y, r * 4));
-        NGMI_HIP(hipMalloc(&dy, r * 4));
-        if (!part) NGMI_HIP(hipMalloc(&part, (size_t)64 * H * 4));
+        const size_t bytes[] = {r * IN_PAD * 2, r * H * 2, r * H * 2, r * H * 2, r * H * 2, r * H * 2, r * 4,
+                                r / 32 * TR_PART * 4, (size_t)train_splits(rows) * NPARAM * 4};
+        for (void **p : ps) {
+            (void)hipFree(*p);
+            *p = nullptr;
+        }
+        for (size_t i = 0; i < sizeof(ps) / sizeof(*ps); i++) NGMI_HIP(hipMalloc(ps[i], bytes[i]));
         cap = rows;
         return NGMI_OK;
     }
@@ -116,23 +102,14 @@ __global__ void k_pack_input(const float *__restrict__ X, unsigned short *__rest
     }
 }
 
-int forward(ngmi_mlp *n, const float *X, int M, int Mpad, hipStream_t s)
+/* the BF16 copies of the master weights */
+int refresh_bf16(ngmi_mlp *n)
 {
-    int rc;
-    hipLaunchKernelGGL(k_pack_input, dim3(blocks((int64_t)Mpad * IN_PAD)), dim3(256), 0, s, X, n->xb,
-                       M, Mpad);
+    hipLaunchKernelGGL(k_f32_to_bf16, dim3(blocks(NPARAM)), dim3(256), 0, 0, n->w, n->wb, (int64_t)NPARAM);
     NGMI_HIP(hipGetLastError());
-    const unsigned short *wb = n->wb;
-    /* Z = X W^T + b: A(i,k) = X[i*K + k], B(j,k) = W[j*K + k] */
-    if ((rc = launch_gemm_bf16(n->xb, IN_PAD, 1, wb + OFF_W1, IN_PAD, 1, n->w + OFF_B1, n->z1,
-                               nullptr, n->h1, H, Mpad, H, IN_PAD, 2, s)))
-        return rc;
-    if ((rc = launch_gemm_bf16(n->h1, H, 1, wb + OFF_W2, H, 1, n->w + OFF_B2, n->z2, nullptr, n->h2,
-                               H, Mpad, H, H, 2, s)))
-        return rc;
-    if ((rc = launch_gemm_bf16(n->h2, H, 1, wb + OFF_W3, H, 1, n->w + OFF_B3, n->z3, nullptr, n->h3,
-                               H, Mpad, H, H, 2, s)))
-        return rc;
+    hipLaunchKernelGGL(k_train_transpose, dim3(H), dim3(H), 0, 0, n->wb, n->wbt);
+    NGMI_HIP(hipGetLastError());
+    NGMI_HIP(hipDeviceSynchronize());
     return NGMI_OK;
 }
 
@@ -150,17 +127,11 @@ int forward_infer(const ngmi_mlp *n, const float *X, float *y, int maxRows, int 
                        X, xb, maxRows, Mpad, dcount);
     NGMI_HIP(hipGetLastError());
     const unsigned short *wb = n->wb;
-    if ((rc = launch_gemm_bf16(xb, IN_PAD, 1, wb + OFF_W1, IN_PAD, 1, n->w + OFF_B1, nullptr,
-                               nullptr, ia, H, Mpad, H, IN_PAD, 2, s, dcount)))
-        return rc;
-    if ((rc = launch_gemm_bf16(ia, H, 1, wb + OFF_W2, H, 1, n->w + OFF_B2, nullptr, nullptr, ib,
-                               H, Mpad, H, H, 2, s, dcount)))
-        return rc;
-    if ((rc = launch_gemm_bf16(ib, H, 1, wb + OFF_W3, H, 1, n->w + OFF_B3, nullptr, nullptr, ia,
-                               H, Mpad, H, H, 2, s, dcount)))
-        return rc;
+    if ((rc = launch_gemm_bf16(xb, wb + OFF_W1, n->w + OFF_B1, ia, Mpad, H, IN_PAD, s, dcount))) return rc;
+    if ((rc = launch_gemm_bf16(ia, wb + OFF_W2, n->w + OFF_B2, ib, Mpad, H, H, s, dcount))) return rc;
+    if ((rc = launch_gemm_bf16(ib, wb + OFF_W3, n->w + OFF_B3, ia, Mpad, H, H, s, dcount))) return rc;
     hipLaunchKernelGGL(k_head, dim3(std::min(blocks(maxRows), 1024)), dim3(256), 0, s, ia, wb + OFF_W4,
-                       n->w + OFF_B4, nullptr, y, nullptr, maxRows, H, dcount);
+                       n->w + OFF_B4, y, maxRows, H, dcount);
     NGMI_HIP(hipGetLastError());
     return NGMI_OK;
 }
@@ -248,7 +219,7 @@ ngmi_mlp *ngmi_mlp_new(unsigned long long seed)
     }
     if (hipMalloc(&n->w, NPARAM * 4) != hipSuccess || hipMalloc(&n->g, NPARAM * 4) != hipSuccess ||
         hipMalloc(&n->m, NPARAM * 4) != hipSuccess || hipMalloc(&n->v, NPARAM * 4) != hipSuccess ||
-        hipMalloc(&n->wb, NPARAM * 2) != hipSuccess ||
+        hipMalloc(&n->wb, NPARAM * 2) != hipSuccess || hipMalloc(&n->wbt, 2 * MLP_SZ_W2 * 2) != hipSuccess ||
         hipMemcpy(n->w, w.data(), NPARAM * 4, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(n->m, 0, NPARAM * 4) != hipSuccess || hipMemset(n->v, 0, NPARAM * 4) != hipSuccess ||
         hipMemset(n->g, 0, NPARAM * 4) != hipSuccess) {
@@ -256,9 +227,7 @@ ngmi_mlp *ngmi_mlp_new(unsigned long long seed)
         delete n;
         return nullptr;
     }
-    hipLaunchKernelGGL(k_f32_to_bf16, dim3(blocks(NPARAM)), dim3(256), 0, 0, n->w, n->wb,
-                       (int64_t)NPARAM);
-    if (hipDeviceSynchronize() != hipSuccess) {
+    if (refresh_bf16(n)) {
         delete n;
         return nullptr;
     }
@@ -280,11 +249,7 @@ int ngmi_mlp_set_params(ngmi_mlp *n, const float *host)
 {
     if (!n || !host) return NGMI_E_PANIC;
     NGMI_HIP(hipMemcpy(n->w, host, NPARAM * 4, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_f32_to_bf16, dim3(blocks(NPARAM)), dim3(256), 0, 0, n->w, n->wb,
-                       (int64_t)NPARAM);
-    NGMI_HIP(hipGetLastError());
-    NGMI_HIP(hipDeviceSynchronize());
-    return NGMI_OK;
+    return refresh_bf16(n);
 }
 
 /* y[M] = network(X[M x 16]); device pointers */
@@ -296,13 +261,9 @@ int ngmi_mlp_forward(ngmi_mlp *n, const float *X, float *y, int M, void *stream)
     if (tune_get(TUNE_GUESS_FUSED))
         return launch_guess_net(n->wb, n->w, X, nullptr, M, nullptr, nullptr, nullptr, y, nullptr, s);
     const int Mpad = (M + 31) / 32 * 32;
-    int rc = n->ensure(Mpad);
+    const int rc = n->ensure_infer(Mpad);
     if (rc) return rc;
-    if ((rc = forward(n, X, M, Mpad, s))) return rc;
-    hipLaunchKernelGGL(k_head, dim3(blocks(M)), dim3(256), 0, s, n->h3, n->wb + OFF_W4,
-                       n->w + OFF_B4, nullptr, y, nullptr, M, H, nullptr);
-    NGMI_HIP(hipGetLastError());
-    return NGMI_OK;
+    return forward_infer(n, X, y, M, Mpad, n->ixb, n->ia, n->ib, nullptr, s);
 }
 
 /* ngmi_mlp_forward without allocating: the work buffers are the library's
@@ -336,41 +297,15 @@ int ngmi_mlp_train_step(ngmi_mlp *n, const float *X, const float *target, int M,
     const int Mpad = (M + 31) / 32 * 32;
     int rc = n->ensure(Mpad);
     if (rc) return rc;
-    if ((rc = forward(n, X, M, Mpad, s))) return rc;
-    float *g = n->g;
-    const unsigned short *wb = n->wb;
-    hipLaunchKernelGGL(k_head, dim3(blocks(M)), dim3(256), 0, s, n->h3, wb + OFF_W4, n->w + OFF_B4,
-                       target, n->y, n->dy, M, H, nullptr);
-    NGMI_HIP(hipGetLastError());
-    /* padded rows carry no gradient */
-    if (Mpad > M) NGMI_HIP(hipMemsetAsync(n->dy + M, 0, (size_t)(Mpad - M) * 4, s));
-    if ((rc = launch_colsum(nullptr, n->h3, n->dy, n->part, g + OFF_W4, Mpad, H, s))) return rc;
-    if ((rc = launch_colsum(n->dy, nullptr, nullptr, n->part, g + OFF_B4, Mpad, 1, s))) return rc;
-    hipLaunchKernelGGL(k_head_back, dim3(blocks((int64_t)Mpad * H)), dim3(256), 0, s, wb + OFF_W4, n->dy,
-                       n->dh, Mpad, H);
-    NGMI_HIP(hipGetLastError());
-    struct L { const unsigned short *hin; int kin; float *z; int64_t ow, ob; };
-    const L layers[3] = {{n->xb, IN_PAD, n->z1, OFF_W1, OFF_B1},
-                         {n->h1, H, n->z2, OFF_W2, OFF_B2},
-                         {n->h2, H, n->z3, OFF_W3, OFF_B3}};
-    for (int li = 2; li >= 0; li--) {
-        const L &Ly = layers[li];
-        const int64_t nz = (int64_t)Mpad * H;
-        hipLaunchKernelGGL(k_silu_back, dim3(blocks(nz)), dim3(256), 0, s, n->dh, Ly.z, n->dz, n->dzb,
-                           nz);
-        NGMI_HIP(hipGetLastError());
-        /* dW[o][i] = sum_m dZ[m][o] Hin[m][i] */
-        if ((rc = launch_gemm_bf16(n->dzb, 1, H, Ly.hin, 1, Ly.kin, nullptr, nullptr, g + Ly.ow,
-                                   nullptr, Ly.kin, H, Ly.kin, Mpad, 0, s)))
-            return rc;
-        if ((rc = launch_colsum(n->dz, nullptr, nullptr, n->part, g + Ly.ob, Mpad, H, s))) return rc;
-        if (li > 0) {
-            /* dHin[m][i] = sum_o dZ[m][o] W[o][i] */
-            if ((rc = launch_gemm_bf16(n->dzb, H, 1, wb + Ly.ow, 1, Ly.kin, nullptr, nullptr, n->dh,
-                                       nullptr, Ly.kin, Mpad, Ly.kin, H, 0, s)))
-                return rc;
-        }
+    AdamStep A{lr, 0.9f, 0.999f, 1e-8f, 1.0f, 1.0f};
+    if (lr > 0) {
+        n->step++;
+        A.c1 = 1.0f - std::pow(A.b1, (float)n->step);
+        A.c2 = 1.0f - std::pow(A.b2, (float)n->step);
     }
+    const TrainBufs B{n->w, n->g, n->m, n->v, n->wb, n->wbt, n->y, n->xo, n->h1, n->h2, n->dz1, n->dz2, n->dz3,
+                      n->cols, n->dw};
+    if ((rc = launch_train_step(B, X, target, M, A, s))) return rc;
     if (loss_host) {
         std::vector<float> yh(M), th(M);
         NGMI_HIP(hipMemcpyAsync(yh.data(), n->y, (size_t)M * 4, hipMemcpyDeviceToHost, s));
@@ -379,14 +314,6 @@ int ngmi_mlp_train_step(ngmi_mlp *n, const float *X, const float *target, int M,
         double acc = 0;
         for (int i = 0; i < M; i++) acc += (double)(yh[i] - th[i]) * (yh[i] - th[i]);
         *loss_host = (float)(acc / M);
-    }
-    if (lr > 0) {
-        n->step++;
-        const float b1 = 0.9f, b2 = 0.999f;
-        const float c1 = 1.0f - std::pow(b1, (float)n->step), c2 = 1.0f - std::pow(b2, (float)n->step);
-        hipLaunchKernelGGL(k_adam, dim3(blocks(NPARAM)), dim3(256), 0, s, n->w, n->wb, g, n->m, n->v,
-                           (int64_t)NPARAM, lr, b1, b2, 1e-8f, c1, c2);
-        NGMI_HIP(hipGetLastError());
     }
     return NGMI_OK;
 }

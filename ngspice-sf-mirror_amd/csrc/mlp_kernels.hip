@@ -3,12 +3,17 @@
  * BF16 weights and activations on the matrix cores (v_mfma_f32_32x32x16
  * bf16, FP32 accumulate), FP32 master weights and Adam for training.
  *
- * One kernel computes C[i][j] = sum_k A(i,k) B(j,k) (+ bias[j]) for strided
- * BF16 operands, so the forward pass (X W^T), the input gradient (dY W) and
- * the weight gradient (dY^T X) are the same kernel with different strides.
- * Each wavefront owns a 32 x 32 tile of C; lane l feeds rows/cols l % 32 and
- * the k octet (l / 32) * 8 .. +7 of every 16-deep step, and receives
- * C rows (v / 4) * 8 + (l / 32) * 4 + v % 4, column l % 32, v = 0..15.
+ * On matrix-core tiles lane l feeds rows/cols l % 32 and the k octet
+ * (l / 32) * 8 .. +7 of every 16-deep step, and receives C rows
+ * (v / 4) * 8 + (l / 32) * 4 + v % 4, column l % 32, v = 0..15.
+ *
+ * Layer-by-layer inference is k_gemm_bf16 per layer.  A training step is
+ * three launches: k_train_rows (forward and backward of a tile of rows),
+ * k_train_dw (weight gradients, split over the rows) and k_train_apply
+ * (their sums, and Adam).  At 4000 rows they take 22.7, 12.0 and 7.0 us, a
+ * step 60 us from call to call; as 24 launches, a layer's product, SiLU
+ * derivative and column sums each their own and the weight gradients 64
+ * waves with all 4000 rows in series, it was 471 us.
  *
  * Inference inside the transient uses k_guess_net instead: one kernel from
  * the feature rows to the nodes' starting values, with the weights held in
@@ -31,24 +36,16 @@ __device__ __forceinline__ f32x16 mfma16(bf16x8 a, bf16x8 b, f32x16 acc)
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
 }
 
-/* epilogue modes */
-enum { EPI_NONE = 0, EPI_BIAS = 1, EPI_BIAS_SILU = 2 };
-
 /*
- * grid: (N/32, tiles) wavefronts of 64 lanes; M, N multiples of 32, K a
- * multiple of 16.  Row tiles are visited grid-stride, so with Mdev (a device
- * row count below M) the launch can be sized to the machine and the work
- * follows the rows actually present.  Outputs: C (fp32, ldc) and, when Cb
- * is set, a BF16 copy of the activated values; Z (fp32) receives the
- * pre-activation.  CONTIG: as1 == bs1 == 1, so each lane's k octet is one
- * 16-byte load per operand.
+ * One hidden layer: Cb[i][j] = hidden_out(bias[j] + sum_k A[i][k] B[j][k]),
+ * grid: (N/32, tiles) wavefronts of 64 lanes, each a 32 x 32 tile; M, N
+ * multiples of 32, K a multiple of 16.  Row tiles are visited grid-stride,
+ * so with Mdev (a device row count below M) the launch can be sized to the
+ * machine and the work follows the rows actually present.
  */
-template <bool CONTIG>
 __global__ void __launch_bounds__(64)
-k_gemm_bf16(const unsigned short *__restrict__ A, int64_t as0, int64_t as1,
-            const unsigned short *__restrict__ B, int64_t bs0, int64_t bs1,
-            const float *__restrict__ bias, float *__restrict__ Z, float *__restrict__ C,
-            unsigned short *__restrict__ Cb, int ldc, int M, int N, int K, int epi,
+k_gemm_bf16(const unsigned short *__restrict__ A, const unsigned short *__restrict__ B,
+            const float *__restrict__ bias, unsigned short *__restrict__ Cb, int M, int N, int K,
             const int *__restrict__ Mdev)
 {
     const int l = threadIdx.x;
@@ -56,39 +53,21 @@ k_gemm_bf16(const unsigned short *__restrict__ A, int64_t as0, int64_t as1,
     if (Mdev) M = min(M, *Mdev);
     const int r = l & 31, kq = (l >> 5) * 8;
     for (int i0 = blockIdx.y * 32; i0 < M; i0 += gridDim.y * 32) {
-        /* with a bias the accumulator starts from it (the column is the
-         * lane's, the same for all 16 values) */
-        const float acc0 = (epi != EPI_NONE && j0 + r < N) ? bias[j0 + r] : 0.0f;
+        /* the accumulator starts from the bias (the column is the lane's,
+         * the same for all 16 values) */
+        const float acc0 = bias[j0 + r];
         f32x16 acc;
 #pragma unroll
         for (int v = 0; v < 16; v++) acc[v] = acc0;
-        const unsigned short *pa = A + (int64_t)(i0 + r) * as0;
-        const unsigned short *pb = B + (int64_t)(j0 + r) * bs0;
-        for (int k0 = 0; k0 < K; k0 += 16) {
-            bf16x8 a, b;
-            if (CONTIG) {
-                a = *reinterpret_cast<const bf16x8 *>(pa + k0 + kq);
-                b = *reinterpret_cast<const bf16x8 *>(pb + k0 + kq);
-            } else {
-#pragma unroll
-                for (int q = 0; q < 8; q++) {
-                    a[q] = __builtin_bit_cast(__bf16, pa[(int64_t)(k0 + kq + q) * as1]);
-                    b[q] = __builtin_bit_cast(__bf16, pb[(int64_t)(k0 + kq + q) * bs1]);
-                }
-            }
-            acc = mfma16(a, b, acc);
-        }
+        const unsigned short *pa = A + (int64_t)(i0 + r) * K;
+        const unsigned short *pb = B + (int64_t)(j0 + r) * K;
+        for (int k0 = 0; k0 < K; k0 += 16)
+            acc = mfma16(*reinterpret_cast<const bf16x8 *>(pa + k0 + kq),
+                         *reinterpret_cast<const bf16x8 *>(pb + k0 + kq), acc);
 #pragma unroll
         for (int v = 0; v < 16; v++) {
             const int i = i0 + (v >> 2) * 8 + (l >> 5) * 4 + (v & 3);
-            const int j = j0 + r;
-            if (i >= M || j >= N) continue;
-            const float z = acc[v];
-            if (Z) Z[(int64_t)i * ldc + j] = z;
-            /* with EPI_BIAS_SILU, Cb gets hidden_out(z) */
-            const float y = (epi == EPI_BIAS_SILU) ? silu(z) : z;
-            if (C) C[(int64_t)i * ldc + j] = y;
-            if (Cb) Cb[(int64_t)i * ldc + j] = f2bf(y);
+            if (i < M) Cb[(int64_t)i * N + j0 + r] = hidden_out(acc[v]);
         }
     }
 }
@@ -99,94 +78,12 @@ __global__ void k_f32_to_bf16(const float *__restrict__ x, unsigned short *__res
     if (i < n) y[i] = f2bf(x[i]);
 }
 
-/* dZ = dY * silu'(Z), written as BF16 (next GEMM operand) and FP32 */
-__global__ void k_silu_back(const float *__restrict__ dY, const float *__restrict__ Z,
-                            float *__restrict__ dZ, unsigned short *__restrict__ dZb, int64_t n)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float z = Z[i];
-    const float s = 1.0f / (1.0f + __expf(-z));
-    const float g = dY[i] * (s * (1.0f + z * (1.0f - s)));
-    dZ[i] = g;
-    dZb[i] = f2bf(g);
-}
-
-/* two-stage column sums, deterministic: part[p][j] = sum over the rows of
- * chunk p of wt[i] * X[i][j] (X fp32 or BF16, wt optional), block = 64
- * columns x 4 row lanes; then out[j] = sum_p part[p][j] in order */
-__global__ void __launch_bounds__(256)
-k_colsum_part(const float *__restrict__ Xf, const unsigned short *__restrict__ Xb,
-              const float *__restrict__ wt, float *__restrict__ part, int M, int N, int chunk)
-{
-    __shared__ float red[4][64];
-    const int cx = threadIdx.x & 63, ry = threadIdx.x >> 6;
-    const int j = blockIdx.x * 64 + cx;
-    const int i0 = blockIdx.y * chunk, i1 = min(M, i0 + chunk);
-    float s = 0.0f;
-    if (j < N) {
-        for (int i = i0 + ry; i < i1; i += 4) {
-            const float x = Xf ? Xf[(int64_t)i * N + j] : bf2f(Xb[(int64_t)i * N + j]);
-            s += wt ? wt[i] * x : x;
-        }
-    }
-    red[ry][cx] = s;
-    __syncthreads();
-    if (ry == 0 && j < N)
-        part[(int64_t)blockIdx.y * N + j] = ((red[0][cx] + red[1][cx]) + red[2][cx]) + red[3][cx];
-}
-
-__global__ void k_colsum_final(const float *__restrict__ part, float *__restrict__ out, int P, int N)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= N) return;
-    float s = 0.0f;
-    for (int p = 0; p < P; p++) s += part[(int64_t)p * N + j];
-    out[j] = s;
-}
-
-constexpr int COLSUM_PARTS = 64;
-
-/* out[j] = sum_i wt[i] X[i][j] for an M x N matrix; part holds
- * COLSUM_PARTS x N floats */
-int launch_colsum(const float *Xf, const unsigned short *Xb, const float *wt, float *part, float *out,
-                  int M, int N, hipStream_t s)
-{
-    const int P = std::max(1, std::min(COLSUM_PARTS, (M + 127) / 128));
-    const int chunk = (M + P - 1) / P;
-    hipLaunchKernelGGL(k_colsum_part, dim3((unsigned)((N + 63) / 64), (unsigned)P), dim3(256), 0, s,
-                       Xf, Xb, wt, part, M, N, chunk);
-    NGMI_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_colsum_final, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, part, out, P,
-                       N);
-    NGMI_HIP(hipGetLastError());
-    return NGMI_OK;
-}
-
-/* Adam on FP32 master weights, refreshing the BF16 copy */
-__global__ void k_adam(float *__restrict__ w, unsigned short *__restrict__ wb,
-                       const float *__restrict__ g, float *__restrict__ m, float *__restrict__ v,
-                       int64_t n, float lr, float b1, float b2, float eps, float c1, float c2)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-    w[i] = wi;
-    if (wb) wb[i] = f2bf(wi);
-}
-
 /* output layer (256 -> 1) forward: y[i] = b + the in-order sum of the
  * blocks' dot products over MLP_HEAD_BLOCK hidden units, each accumulated
- * in order with FMA (k_guess_net sums the same way); and the MSE gradient
- * dy = 2 (y - t) / M.  K is a multiple of MLP_HEAD_BLOCK. */
+ * in order with FMA (k_guess_net sums the same way).  K is a multiple of
+ * MLP_HEAD_BLOCK. */
 __global__ void k_head(const unsigned short *__restrict__ H, const unsigned short *__restrict__ w,
-                       const float *__restrict__ b, const float *__restrict__ target,
-                       float *__restrict__ y, float *__restrict__ dy, int M, int K,
+                       const float *__restrict__ b, float *__restrict__ y, int M, int K,
                        const int *__restrict__ Mdev)
 {
     if (Mdev) M = min(M, *Mdev);
@@ -198,18 +95,7 @@ __global__ void k_head(const unsigned short *__restrict__ H, const unsigned shor
             s += p;
         }
         y[i] = s;
-        if (target) dy[i] = 2.0f * (s - target[i]) / (float)M;
     }
-}
-
-/* output layer backward, input gradient: dH[i][k] = dy[i] w[k] (fp32) */
-__global__ void k_head_back(const unsigned short *__restrict__ w, const float *__restrict__ dy,
-                            float *__restrict__ dH, int M, int K)
-{
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (int64_t)M * K) return;
-    const int i = (int)(e / K), k = (int)(e - (int64_t)i * K);
-    dH[e] = dy[i] * bf2f(w[k]);
 }
 
 /* ---------------- fused inference for the transient ---------------- */
@@ -343,6 +229,363 @@ k_guess_net(const float *__restrict__ X, const unsigned short *__restrict__ wb, 
             count[1] = 0;
         }
     }
+}
+
+/* ---------------- training ---------------- */
+
+/* The operands of the weight gradients, whose matrix-core steps run along
+ * the rows: element (row, column) of a matrix of C columns at
+ * ((row / 8) * C + column) * 8 + row % 8, so that a lane's octet of rows is
+ * one 16-byte load and 32 lanes' are 512 consecutive bytes. */
+__device__ __forceinline__ int64_t oct_at(int64_t row, int C, int col) { return ((row >> 3) * C + col) * 8 + (row & 7); }
+
+/* 32 x 32 tile of A (32 rows, BF16, LDS) times this wave's weights, k in
+ * order, from acc on */
+template <int STEPS>
+__device__ __forceinline__ f32x16 tr_product(const unsigned short *A, int lda, const bf16x8 (&w)[STEPS], f32x16 acc,
+                                             int l)
+{
+    const unsigned short *pa = A + (l & 31) * lda + (l >> 5) * 8;
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) acc = mfma16(*reinterpret_cast<const bf16x8 *>(pa + 16 * s), w[s], acc);
+    return acc;
+}
+
+template <int STEPS>
+__device__ __forceinline__ void tr_weights(bf16x8 (&w)[STEPS], const unsigned short *__restrict__ W, int ldw, int j, int l)
+{
+    const unsigned short *p = W + (int64_t)j * ldw + (l >> 5) * 8;
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) w[s] = *reinterpret_cast<const bf16x8 *>(p + 16 * s);
+}
+
+/* this wave's tile, rounded to BF16: rows to LDS (the next product's
+ * operand) and, in octets of rows, to memory */
+__device__ __forceinline__ void tr_put(const unsigned short (&h)[16], unsigned short *lds, unsigned short *__restrict__ oct,
+                                       int64_t i0, int j, int l)
+{
+#pragma unroll
+    for (int v = 0; v < 16; v++) lds[((v >> 2) * 8 + (l >> 5) * 4 + (v & 3)) * GN_HLD + j] = h[v];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const uint2 u = make_uint2(h[4 * q] | (unsigned)h[4 * q + 1] << 16, h[4 * q + 2] | (unsigned)h[4 * q + 3] << 16);
+        *reinterpret_cast<uint2 *>(oct + oct_at(i0 + 8 * q + 4 * (l >> 5), MLP_HID, j)) = u;
+    }
+}
+
+/* the sum over the tile's 32 rows of a column, both halves of the wave */
+__device__ __forceinline__ float tr_colsum(const float (&g)[16])
+{
+    float s = 0.0f;
+#pragma unroll
+    for (int v = 0; v < 16; v++) s += g[v];
+    return s + __shfl_xor(s, 32);
+}
+
+/* dH times the derivative of SiLU at z */
+__device__ __forceinline__ float silu_back(float dh, float z)
+{
+    const float s = 1.0f / (1.0f + __expf(-z));
+    return dh * (s * (1.0f + z * (1.0f - s)));
+}
+
+/*
+ * Forward and backward of 32 rows a workgroup: the rows' gradients need
+ * nothing of the other rows, so pre-activations stay in registers (the wave
+ * that forms a layer's columns also forms their gradients) and activations
+ * and gradients go from layer to layer through LDS.  Out come y, the weight
+ * gradients' operands in octets of rows, and the tile's column sums (part:
+ * b1, b2, b3, w4, b4).  The matrix-core steps and the element-wise code are
+ * those of the inference kernels; rows from M on have zero gradients.  wbt:
+ * W2 and W3 transposed, so that both directions load octets.  Each layer's
+ * weights load during the layer before.  Bound by that chain of seven
+ * barriers and by 530 KB of weights from L2 for every workgroup: 22.7 us at
+ * 4000 rows, where 125 workgroups leave half of the CUs idle.
+ */
+__global__ void __launch_bounds__(GN_THREADS)
+k_train_rows(const float *__restrict__ X, const float *__restrict__ target, int M, const unsigned short *__restrict__ wb,
+             const unsigned short *__restrict__ wbt, const float *__restrict__ wf, float *__restrict__ yout,
+             unsigned short *__restrict__ xo, unsigned short *__restrict__ h1o, unsigned short *__restrict__ h2o,
+             unsigned short *__restrict__ dz1o, unsigned short *__restrict__ dz2o, unsigned short *__restrict__ dz3o,
+             float *__restrict__ part)
+{
+    __shared__ __align__(16) unsigned short xs[32 * GN_XLD];
+    __shared__ __align__(16) unsigned short ha[32 * GN_HLD];
+    __shared__ __align__(16) unsigned short hb[32 * GN_HLD];
+    __shared__ float w4s[MLP_HID];
+    __shared__ float ps[32][GN_HEAD_BLOCKS + 1];
+    __shared__ float dys[32];
+    const int tid = threadIdx.x, l = tid & 63, j = (tid >> 6) * 32 + (l & 31), r4 = (l >> 5) * 4;
+    const int64_t i0 = (int64_t)blockIdx.x * 32;
+    float *pt = part + (int64_t)blockIdx.x * TR_PART;
+    bf16x8 wa[MLP_HID / 16], wc[MLP_HID / 16], w1[MLP_IN_PAD / 16];
+    {
+        const int rr = tid >> 4, cc = tid & 15;
+        const unsigned short v = f2bf(i0 + rr < M ? X[(i0 + rr) * MLP_IN + cc] : 0.0f);
+        xs[rr * GN_XLD + cc] = v;
+        xs[rr * GN_XLD + MLP_IN + cc] = 0;
+        xo[oct_at(i0 + rr, MLP_IN_PAD, cc)] = v;
+        xo[oct_at(i0 + rr, MLP_IN_PAD, MLP_IN + cc)] = 0;
+    }
+    if (tid < MLP_HID) w4s[tid] = bf2f(wb[MLP_OFF_W4 + tid]);
+    tr_weights(w1, wb + MLP_OFF_W1, MLP_IN_PAD, j, l);
+    tr_weights(wa, wb + MLP_OFF_W2, MLP_HID, j, l);
+    const float b1 = wf[MLP_OFF_B1 + j], b2 = wf[MLP_OFF_B2 + j], b3 = wf[MLP_OFF_B3 + j], b4 = wf[MLP_OFF_B4];
+    const float tg = tid < 32 && i0 + tid < M ? target[i0 + tid] : 0.0f;
+    f32x16 z1, z2, z3;
+    unsigned short h[16];
+#pragma unroll
+    for (int v = 0; v < 16; v++) z1[v] = b1;
+    __syncthreads();
+    z1 = tr_product(xs, GN_XLD, w1, z1, l);
+#pragma unroll
+    for (int v = 0; v < 16; v++) h[v] = hidden_out(z1[v]);
+    tr_put(h, ha, h1o, i0, j, l);
+    tr_weights(wc, wb + MLP_OFF_W3, MLP_HID, j, l);
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 16; v++) z2[v] = b2;
+    z2 = tr_product(ha, GN_HLD, wa, z2, l);
+#pragma unroll
+    for (int v = 0; v < 16; v++) h[v] = hidden_out(z2[v]);
+    tr_put(h, hb, h2o, i0, j, l);
+    tr_weights(wa, wbt + MLP_SZ_W2, MLP_HID, j, l);   /* W3 transposed */
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 16; v++) z3[v] = b3;
+    z3 = tr_product(hb, GN_HLD, wc, z3, l);
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        h[v] = hidden_out(z3[v]);
+        ha[((v >> 2) * 8 + r4 + (v & 3)) * GN_HLD + j] = h[v];
+    }
+    __syncthreads();
+    if (tid < 32 * GN_HEAD_BLOCKS) {
+        const int rr = tid / GN_HEAD_BLOCKS, cb = tid % GN_HEAD_BLOCKS;
+        const unsigned short *hr = ha + rr * GN_HLD + cb * MLP_HEAD_BLOCK;
+        float p = 0.0f;
+#pragma unroll
+        for (int e = 0; e < MLP_HEAD_BLOCK; e++) p = fmaf(bf2f(hr[e]), w4s[cb * MLP_HEAD_BLOCK + e], p);
+        ps[rr][cb] = p;
+    }
+    __syncthreads();
+    if (tid < 64) {
+        float dy = 0.0f;
+        if (tid < 32) {
+            float y = b4;
+#pragma unroll
+            for (int cb = 0; cb < GN_HEAD_BLOCKS; cb++) y += ps[tid][cb];
+            if (i0 + tid < M) {
+                yout[i0 + tid] = y;
+                dy = 2.0f * (y - tg) / (float)M;
+            }
+            dys[tid] = dy;
+        }
+#pragma unroll
+        for (int o = 16; o > 0; o >>= 1) dy += __shfl_xor(dy, o);
+        if (tid == 0) pt[4 * MLP_HID] = dy;
+    }
+    __syncthreads();
+    float g[16];
+    {
+        float u[16];
+        const float w4 = w4s[j];
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const float dy = dys[(v >> 2) * 8 + r4 + (v & 3)];
+            u[v] = dy * bf2f(h[v]);
+            g[v] = silu_back(dy * w4, z3[v]);
+            h[v] = f2bf(g[v]);
+        }
+        const float su = tr_colsum(u), sg = tr_colsum(g);
+        if (l < 32) pt[3 * MLP_HID + j] = su, pt[2 * MLP_HID + j] = sg;
+    }
+    tr_put(h, hb, dz3o, i0, j, l);
+    tr_weights(wc, wbt, MLP_HID, j, l);               /* W2 transposed */
+    __syncthreads();
+    z3 = tr_product(hb, GN_HLD, wa, f32x16{}, l);
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        g[v] = silu_back(z3[v], z2[v]);
+        h[v] = f2bf(g[v]);
+    }
+    tr_put(h, ha, dz2o, i0, j, l);
+    {
+        const float sg = tr_colsum(g);
+        if (l < 32) pt[MLP_HID + j] = sg;
+    }
+    __syncthreads();
+    z3 = tr_product(ha, GN_HLD, wc, f32x16{}, l);
+#pragma unroll
+    for (int v = 0; v < 16; v++) {
+        g[v] = silu_back(z3[v], z1[v]);
+        h[v] = f2bf(g[v]);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const uint2 u = make_uint2(h[4 * q] | (unsigned)h[4 * q + 1] << 16, h[4 * q + 2] | (unsigned)h[4 * q + 3] << 16);
+        *reinterpret_cast<uint2 *>(dz1o + oct_at(i0 + 8 * q + r4, MLP_HID, j)) = u;
+    }
+    const float sg = tr_colsum(g);
+    if (l < 32) pt[j] = sg;
+}
+
+/* dW[o][i] = sum_m dZ[m][o] Hin[m][i] of the rows [y chunk, (y + 1) chunk)
+ * into part y: a 64 x 64 tile (64 x 32 of W1) a wave, 2 x 2 matrix-core
+ * tiles.  chunk is a multiple of 16.  A tile of 64 x 64 reads each operand 4
+ * times instead of 8; 12.0 us at 4000 rows (15 parts, 540 waves), bound by the
+ * loads' latency and the parts' 8.4 MB. */
+constexpr int DW_STEPS = 8;   /* matrix-core steps loaded at a time */
+
+template <int NI>
+__device__ __forceinline__ void dw_tile(const unsigned short *__restrict__ dz, const unsigned short *__restrict__ hin,
+                                        int kin, int o0, int c0, int m0, int m1, float *__restrict__ out, int l)
+{
+    const int r = l & 31, half = l >> 5;
+    const unsigned short *pa = dz + ((int64_t)(m0 / 8 + half) * MLP_HID + o0 + r) * 8;
+    const unsigned short *pb = hin + ((int64_t)(m0 / 8 + half) * kin + c0 + r) * 8;
+    f32x16 acc[2][NI] = {};
+    for (int m = m0; m < m1; m += 16 * DW_STEPS) {   /* a batch's loads in flight together */
+        bf16x8 a[DW_STEPS][2], b[DW_STEPS][NI];
+#pragma unroll
+        for (int q = 0; q < DW_STEPS; q++) {
+            const int mm = min(m + 16 * q, m1 - 16) - m0;
+#pragma unroll
+            for (int t = 0; t < 2; t++) a[q][t] = *reinterpret_cast<const bf16x8 *>(pa + (int64_t)mm * MLP_HID + 256 * t);
+#pragma unroll
+            for (int t = 0; t < NI; t++) b[q][t] = *reinterpret_cast<const bf16x8 *>(pb + (int64_t)mm * kin + 256 * t);
+        }
+#pragma unroll
+        for (int q = 0; q < DW_STEPS; q++)
+            if (m + 16 * q < m1) {
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+#pragma unroll
+                    for (int u = 0; u < NI; u++) acc[t][u] = mfma16(a[q][t], b[q][u], acc[t][u]);
+            }
+    }
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int u = 0; u < NI; u++)
+#pragma unroll
+            for (int v = 0; v < 16; v++)
+                out[(int64_t)(o0 + 32 * t + (v >> 2) * 8 + half * 4 + (v & 3)) * kin + c0 + 32 * u + r] = acc[t][u][v];
+}
+
+__global__ void __launch_bounds__(64)
+k_train_dw(const unsigned short *__restrict__ xo, const unsigned short *__restrict__ h1o,
+           const unsigned short *__restrict__ h2o, const unsigned short *__restrict__ dz1o,
+           const unsigned short *__restrict__ dz2o, const unsigned short *__restrict__ dz3o, int rows, int chunk,
+           float *__restrict__ part)
+{
+    const int l = threadIdx.x, t = blockIdx.x, o0 = (t & 3) * 64, c0 = (t >> 2 & 3) * 64;
+    const int m0 = blockIdx.y * chunk, m1 = min(rows, m0 + chunk);
+    float *out = part + (int64_t)blockIdx.y * MLP_NPARAM;
+    if (t < 16) dw_tile<2>(dz2o, h1o, MLP_HID, o0, c0, m0, m1, out + MLP_OFF_W2, l);
+    else if (t < 32) dw_tile<2>(dz3o, h2o, MLP_HID, o0, c0, m0, m1, out + MLP_OFF_W3, l);
+    else dw_tile<1>(dz1o, xo, MLP_IN_PAD, o0, 0, m0, m1, out + MLP_OFF_W1, l);
+}
+
+/* Adam on an FP32 master weight */
+__device__ __forceinline__ float adam(float *__restrict__ w, float *__restrict__ m, float *__restrict__ v, float gi,
+                                      const AdamStep &A)
+{
+    const float mi = A.b1 * *m + (1.0f - A.b1) * gi;
+    const float vi = A.b2 * *v + (1.0f - A.b2) * gi * gi;
+    *m = mi;
+    *v = vi;
+    return *w = *w - A.lr * (mi / A.c1) / (sqrtf(vi / A.c2) + A.eps);
+}
+
+/* The gradients from their parts, in order, and with lr > 0 an Adam step on
+ * them, refreshing the BF16 copies.  A workgroup takes 16 x 16 weights (the
+ * transposed copy written through LDS), or, after the weights, 16 of the
+ * column-summed parameters with 16 threads each. */
+constexpr int TR_TILES_W1 = (int)(MLP_SZ_W1 / 256), TR_TILES_W2 = (int)(MLP_SZ_W2 / 256);
+__global__ void __launch_bounds__(256)
+k_train_apply(const float *__restrict__ dw, int S, const float *__restrict__ cols, int tiles, float *__restrict__ g,
+              float *__restrict__ w, unsigned short *__restrict__ wb, unsigned short *__restrict__ wbt,
+              float *__restrict__ m, float *__restrict__ v, AdamStep A)
+{
+    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+    int b = blockIdx.x;
+    if (b < TR_TILES_W1 + 2 * TR_TILES_W2) {
+        __shared__ unsigned short T[16][17];
+        int kin = MLP_IN_PAD;
+        int64_t off = MLP_OFF_W1, toff = -1;
+        if (b >= TR_TILES_W1) {
+            b -= TR_TILES_W1;
+            const bool w3 = b >= TR_TILES_W2;
+            kin = MLP_HID;
+            off = w3 ? MLP_OFF_W3 : MLP_OFF_W2;
+            toff = w3 ? MLP_SZ_W2 : 0;
+            if (w3) b -= TR_TILES_W2;
+        }
+        const int o0 = b / (kin / 16) * 16, c0 = b % (kin / 16) * 16;
+        const int64_t i = off + (int64_t)(o0 + ty) * kin + c0 + tx;
+        float s = 0.0f;
+        int p = 0;
+        for (; p + 8 <= S; p += 8) {
+            float t[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++) t[q] = dw[(p + q) * MLP_NPARAM + i];
+#pragma unroll
+            for (int q = 0; q < 8; q++) s += t[q];
+        }
+        for (; p < S; p++) s += dw[p * MLP_NPARAM + i];
+        g[i] = s;
+        if (!(A.lr > 0)) return;
+        const unsigned short nb = f2bf(adam(w + i, m + i, v + i, s, A));
+        wb[i] = nb;
+        if (toff < 0) return;
+        T[ty][tx] = nb;
+        __syncthreads();
+        wbt[toff + (int64_t)(c0 + ty) * MLP_HID + o0 + tx] = T[tx][ty];
+        return;
+    }
+    b -= TR_TILES_W1 + 2 * TR_TILES_W2;
+    __shared__ float R[16][17];
+    const int c = b * 16 + tx;
+    float s = 0.0f;
+#pragma unroll 8
+    for (int p = ty; p < tiles; p += 16) s += cols[(int64_t)p * TR_PART + min(c, TR_COLS - 1)];
+    R[ty][tx] = s;
+    __syncthreads();
+    if (ty != 0 || c >= TR_COLS) return;
+    s = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 16; q++) s += R[q][tx];
+    const int k = c / MLP_HID;
+    const int64_t i = (k == 0 ? MLP_OFF_B1 : k == 1 ? MLP_OFF_B2 : k == 2 ? MLP_OFF_B3 : k == 3 ? MLP_OFF_W4 : MLP_OFF_B4) +
+                      c % MLP_HID;
+    g[i] = s;
+    if (A.lr > 0) wb[i] = f2bf(adam(w + i, m + i, v + i, s, A));
+}
+
+/* W2 and W3 of wb transposed into wbt */
+__global__ void k_train_transpose(const unsigned short *__restrict__ wb, unsigned short *__restrict__ wbt)
+{
+    const int o = blockIdx.x, i = threadIdx.x;
+    wbt[(int64_t)i * MLP_HID + o] = wb[MLP_OFF_W2 + (int64_t)o * MLP_HID + i];
+    wbt[MLP_SZ_W2 + (int64_t)i * MLP_HID + o] = wb[MLP_OFF_W3 + (int64_t)o * MLP_HID + i];
+}
+
+int launch_train_step(const TrainBufs &B, const float *X, const float *target, int M, const AdamStep &A, hipStream_t s)
+{
+    const int rows = (M + 31) / 32 * 32, tiles = rows / 32;
+    hipLaunchKernelGGL(k_train_rows, dim3((unsigned)tiles), dim3(GN_THREADS), 0, s, X, target, M, B.wb, B.wbt, B.w, B.y,
+                       B.x, B.h1, B.h2, B.dz1, B.dz2, B.dz3, B.cols);
+    NGMI_HIP(hipGetLastError());
+    const int S = train_splits(rows), chunk = ((rows / 16 + S - 1) / S) * 16;
+    hipLaunchKernelGGL(k_train_dw, dim3(36, (unsigned)S), dim3(64), 0, s, B.x, B.h1, B.h2, B.dz1, B.dz2, B.dz3, rows,
+                       chunk, B.dw);
+    NGMI_HIP(hipGetLastError());
+    const unsigned apply = TR_TILES_W1 + 2 * TR_TILES_W2 + (TR_COLS + 15) / 16;
+    hipLaunchKernelGGL(k_train_apply, dim3(apply), dim3(256), 0, s, B.dw, S, B.cols, tiles, B.g, B.w, B.wb, B.wbt, B.m,
+                       B.v, A);
+    NGMI_HIP(hipGetLastError());
+    return NGMI_OK;
 }
 
 /* The same network with the weights streamed from L2 per tile instead of
@@ -489,10 +732,8 @@ int launch_guess_net(const unsigned short *wb, const float *wf, const float *X, 
     return NGMI_OK;
 }
 
-int launch_gemm_bf16(const unsigned short *A, int64_t as0, int64_t as1, const unsigned short *B,
-                     int64_t bs0, int64_t bs1, const float *bias, float *Z, float *C,
-                     unsigned short *Cb, int ldc, int M, int N, int K, int epi, hipStream_t s,
-                     const int *Mdev)
+int launch_gemm_bf16(const unsigned short *A, const unsigned short *B, const float *bias, unsigned short *Cb, int M,
+                     int N, int K, hipStream_t s, const int *Mdev)
 {
     if (M % 32 || N % 32 || K % 16) {
         set_error("gemm shape %d x %d x %d not a multiple of 32 x 32 x 16", M, N, K);
@@ -501,12 +742,7 @@ int launch_gemm_bf16(const unsigned short *A, int64_t as0, int64_t as1, const un
     /* with a device row count the grid is sized to the machine (8 XCDs x
      * 32 CUs x a few waves per tile column) and strides over the tiles */
     const int tiles = Mdev ? std::min(M / 32, 2048) : M / 32;
-    if (as1 == 1 && bs1 == 1)
-        hipLaunchKernelGGL(k_gemm_bf16<true>, dim3(N / 32, tiles), dim3(64), 0, s, A, as0, as1, B, bs0,
-                           bs1, bias, Z, C, Cb, ldc, M, N, K, epi, Mdev);
-    else
-        hipLaunchKernelGGL(k_gemm_bf16<false>, dim3(N / 32, tiles), dim3(64), 0, s, A, as0, as1, B,
-                           bs0, bs1, bias, Z, C, Cb, ldc, M, N, K, epi, Mdev);
+    hipLaunchKernelGGL(k_gemm_bf16, dim3(N / 32, tiles), dim3(64), 0, s, A, B, bias, Cb, M, N, K, Mdev);
     NGMI_HIP(hipGetLastError());
     return NGMI_OK;
 }

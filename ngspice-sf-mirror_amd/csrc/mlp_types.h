@@ -39,6 +39,33 @@ __device__ __forceinline__ float silu(float z) { return z * __builtin_amdgcn_rcp
  * at the pre-activation z; output BF16 */
 __device__ __forceinline__ unsigned short hidden_out(float z) { return f2bf(silu(z)); }
 
+/* ---- training ---- */
+
+/* a row tile's column sums: b1, b2, b3, w4 (256 each), b4; padded to whole
+ * 64-byte lines */
+constexpr int TR_COLS = 4 * MLP_HID + 1, TR_PART = (TR_COLS + 15) / 16 * 16;
+
+/* parts the weight gradients' rows are split in: 256 rows each, a chain of 16
+ * matrix-core steps, until there are 32 parts (1152 waves; more would cost
+ * more in writing and summing parts, 0.56 MB each, than a shorter chain
+ * gains) */
+inline int train_splits(int rows) { return rows < 512 ? 1 : rows / 256 > 32 ? 32 : rows / 256; }
+
+struct AdamStep {
+    float lr, b1, b2, eps, c1, c2;   /* lr <= 0: gradients only */
+};
+
+/* device buffers of a training step: parameters, their BF16 copy and W2, W3
+ * transposed; outputs y; BF16 inputs, activations and gradients in octets of
+ * rows; column sums by row tile; weight gradients by part */
+struct TrainBufs {
+    float *w, *g, *m, *v;
+    unsigned short *wb, *wbt;
+    float *y;
+    unsigned short *x, *h1, *h2, *dz1, *dz2, *dz3;
+    float *cols, *dw;
+};
+
 }  // namespace ngmi
 
 #endif

@@ -89,3 +89,33 @@ def test_training_reduces_loss():
     last = net.train_step(dX.data_ptr(), dT.data_ptr(), M, 0.0)
     print('loss %.3e -> %.3e' % (first, last), flush=True)
     assert last < 0.1 * first
+
+
+@pytest.mark.parametrize('M', [1, 31, 32, 33, 511, 512, 545, 8240])
+def test_gradients_after_a_step(M):
+    """Row tiles' ends, one to 32 parts of the rows (8240: a last part with
+    none), and the weights' copies after Adam: the gradients of a second step
+    on the updated parameters.  Bar: the backward operands' BF16 rounding, as
+    above; a sum over rows split in parts only shortens its chains."""
+    print('case: guess network two steps M=%d' % M, flush=True)
+    rng = np.random.default_rng(100 + M)
+    net = ngmi.GuessNet(seed=9)
+    X = rng.normal(size=(M, 16)).astype(np.float32)
+    T = rng.normal(scale=0.1, size=M).astype(np.float32)
+    dX, dT = torch.from_numpy(X).cuda(), torch.from_numpy(T).cuda()
+    before = net.params()
+    net.train_step(dX.data_ptr(), dT.data_ptr(), M, 1e-2)
+    p, g1 = net.params(), net.params(grads=True)
+    # Adam's first step is lr g / (|g| + eps)
+    want = before - 1e-2 * g1 / (np.abs(g1) + 1e-8)
+    assert np.abs(p - want).max() <= 1e-5 * 1e-2 + 2.0 ** -22
+    loss = net.train_step(dX.data_ptr(), dT.data_ptr(), M, 0.0)
+    assert np.array_equal(net.params(), p)
+    _, loss_ref, g_ref = reference(net, p, X, T)
+    assert abs(loss - loss_ref) <= 1e-3 * loss_ref + 1e-7
+    for name, gg, gr in zip(['W1', 'b1', 'W2', 'b2', 'W3', 'b3', 'w4', 'b4'],
+                            net.unpack(net.params(grads=True)), g_ref):
+        gg = np.asarray(gg, dtype=np.float64).reshape(-1)
+        err = np.abs(gg - gr).max() / max(np.abs(gr).max(), 1e-30)
+        print('grad %-3s scaled err %.2e' % (name, err), flush=True)
+        assert err < 2e-2, name
