@@ -43,6 +43,7 @@
 
 #include "ngmi_internal.h"
 #include "splu_types.h"
+#include "fp64.h"
 
 using namespace ngmi;
 
@@ -89,19 +90,6 @@ __device__ __forceinline__ void static_for(F f)
         f(std::integral_constant<int, B>());
         static_for<B + 1, E>(f);
     }
-}
-
-/* 1 / p: v_rcp_f64 of the mantissa (2^-24) with two Newton steps, the second
- * on the exact remainder: equal to 1.0 / p for every one of 2.6e8 random
- * mantissas, without the scaled division sequence's branch for the range's
- * ends */
-__device__ __forceinline__ double recip(double p)
-{
-    const double m = __builtin_amdgcn_frexp_mant(p);
-    double r = __builtin_amdgcn_rcp(m);
-    r = fma(fma(-m, r, 1.0), r, r);
-    r = fma(fma(-m, r, 1.0), r, r);
-    return __builtin_amdgcn_ldexp(r, -__builtin_amdgcn_frexp_exp(p));
 }
 
 struct SpDev {
@@ -764,14 +752,6 @@ __global__ void __launch_bounds__(WG) k_sp_fwd_small(SpDev d, const int *__restr
         if (k < ns) y[id[k]] = v[q];
         else if (k < nf) w[k] = v[q];
     }
-}
-
-/* q = a / b from r ~ 1 / b: one correction of a r by its exact remainder,
- * off the dependent chain of a full division */
-__device__ __forceinline__ double div_by(double a, double b, double r)
-{
-    const double q = a * r;
-    return fma(fma(-q, b, a), r, q);
 }
 
 /* backward substitution of one small front a workgroup: the pivots' rows of

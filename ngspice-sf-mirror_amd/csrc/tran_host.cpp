@@ -50,16 +50,6 @@ using namespace ngmi;
  * would need more than ASM_MAXPART partial sums */
 constexpr int ASM_LEAF = 16;
 constexpr int ASM_MAXPART = 48;
-/* LU and substitution program records: PROG_INTS ints, of which the last
- * 4 * PROG_INLINE are the inline term groups */
-constexpr int PROG_INLINE = 3;
-constexpr int PROG_INTS = 4 + 4 * PROG_INLINE;
-/* record kinds (bits 20-21 of the first int): a plain entry, a partial sum
- * of one chunk of a long entry's terms (into a partial slot), and the
- * combine that adds a long entry's partial sums */
-constexpr int PROG_PLAIN = 0, PROG_PARTIAL = 1, PROG_COMBINE = 2;
-/* entries with more terms run as partial sums over several lanes */
-constexpr int SPLIT_TERMS = 24;
 /* dense workspaces for KLU's pivoting: at most PV_POOL_SLOTS per topology
  * within PV_POOL_BYTES (one at least), none when one would exceed
  * PV_SLOT_MAX_BYTES */
@@ -618,6 +608,15 @@ int analyze(const ngmi_circuit &c0, Plan &P)
                 by[e.lev].push_back({k, -1});
             }
         }
+        /* a wavefront takes as long as its longest entry: entries of a level
+         * with the same number of term groups side by side, then the partial
+         * sums (an entry's stay in a row) and the combines */
+        auto groups = [&](const Item &it) {
+            return it.chunk == -1 ? ((int)ps[it.idx].terms.size() + 3) / 4 : it.chunk >= 0 ? SPLIT_TERMS : SPLIT_TERMS + 1;
+        };
+        for (auto &its : by)
+            std::stable_sort(its.begin(), its.end(),
+                             [&](const Item &a, const Item &b) { return groups(a) < groups(b); });
         return by;
     };
     const auto fby = items(fe), wby = items(we), bby = items(be);
@@ -653,6 +652,9 @@ int analyze(const ngmi_circuit &c0, Plan &P)
         }
         const int n = (int)lev_out.size();
         lev_out.push_back((int)(ent.size() / PROG_INTS));
+        /* the kernel's first loads need a record and a term group */
+        if (ent.empty()) ent.assign(PROG_INTS, 0);
+        if (term.empty()) term.assign(4, pad);
         return n;
     };
     std::vector<int> f_lev, f_ent, fw_lev, fw_ent, bw_lev, bw_ent;

@@ -24,6 +24,7 @@
 #include "bsim4_eval.h"
 #include "bsim4_dev.h"
 #include "tran_types.h"
+#include "fp64.h"
 #include "guess_types.h"
 
 namespace ngmi {
@@ -210,6 +211,16 @@ k_tran_mos_dense(const TranDev *__restrict__ Ds, const B4Tab *__restrict__ tabs,
 
 /* ---------------- scalar helpers (thread 0 of a circuit) ---------------- */
 
+/* A circuit's workgroup is one wavefront or four; what bounds both is a chain
+ * of memory and LDS latencies.  A 101-stage ring alone takes 71000 cycles a
+ * pass with four: LU 18800 (17 levels), substitutions 18500, assembly 13000,
+ * capacitors and sources 7200; with one, every level waiting for memory and
+ * the sources' breakpoints found one after the other, 121000.  The dense
+ * factorization, the guess's rows and the sources' breakpoints are the first
+ * wavefront's alone, ordered by wave_sync. */
+constexpr int ONE_WAVE = 64;
+constexpr int STEP_WIDE = 4 * ONE_WAVE;
+
 __device__ int almost_equal_ulps(double A, double B, int maxUlps)
 {   /* equality.c:22-60 */
     if (A == B) return 1;
@@ -291,31 +302,46 @@ __device__ double vsrc_value(const double *vp, int mode, double tnow, double ste
     return P.V2 + (P.V1 - P.V2) * (time - (P.TR + P.PW)) / P.TF;
 }
 
+/* VSRCaccept, vsrcacct.c:20-160 (PULSE corners), by one wavefront: a source
+ * a lane finds its next corner; the first lane enters those reached into the
+ * breakpoints, in source order */
 __device__ __forceinline__ int vsrc_accept(const TranDev &D, int c, CktCtl *K)
-{   /* vsrcacct.c:20-160 (PULSE corners) */
+{
     if (!(K->mode & (M_TRAN | M_TRANOP))) return 0;
-    for (int k = 0; k < D.NVS; k++) {
-        const double *vp = D.vs_par + ((int64_t)c * D.NVS + k) * VSP;
-        if (vp[1] == 0.0) continue;
+    const int lane = threadIdx.x;
+    const double now = K->time, minb = K->minBreak, step = K->step;
+    for (int k0 = 0; k0 < D.NVS; k0 += ONE_WAVE) {
+        const int k = k0 + lane;
         double *brk = D.vs_brk + (int64_t)c * D.NVS + k;
-        const Pulse P = pulse_params(vp, K->step);
-        double time = K->time - P.TD;
-        if (K->time >= *brk) {
-            double wait;
-            if (time >= P.PER) {
-                const double basetime = P.PER * floor(time / P.PER);
-                time -= basetime;
+        bool hit = false;
+        double next = 0.0;
+        if (k < D.NVS) {
+            const double *vp = D.vs_par + ((int64_t)c * D.NVS + k) * VSP;
+            if (vp[1] != 0.0 && now >= *brk) {
+                const Pulse P = pulse_params(vp, step);
+                double time = now - P.TD, wait;
+                if (time >= P.PER) {
+                    const double basetime = P.PER * floor(time / P.PER);
+                    time -= basetime;
+                }
+                const double atime = time + minb;
+                if (atime < 0.0) wait = -time;
+                else if (atime < P.TR) wait = P.TR - time;
+                else if (atime < P.TR + P.PW) wait = P.TR + P.PW - time;
+                else if (atime < P.TR + P.PW + P.TF) wait = P.TR + P.PW + P.TF - time;
+                else wait = P.PER - time;
+                next = now + wait;
+                *brk = next - minb;
+                hit = true;
             }
-            const double atime = time + K->minBreak;
-            if (atime < 0.0) wait = -time;
-            else if (atime < P.TR) wait = P.TR - time;
-            else if (atime < P.TR + P.PW) wait = P.TR + P.PW - time;
-            else if (atime < P.TR + P.PW + P.TF) wait = P.TR + P.PW + P.TF - time;
-            else wait = P.PER - time;
-            *brk = K->time + wait;
-            if (set_break(K, *brk)) return -1;
-            *brk -= K->minBreak;
         }
+        int bad = 0;
+        for (unsigned long long m = __ballot(hit); m && !bad; m &= m - 1) {
+            const double t = __shfl(next, __ffsll(m) - 1);
+            if (lane == 0) bad = set_break(K, t) != 0;
+            bad = __shfl(bad, 0);
+        }
+        if (bad) return -1;
     }
     return 0;
 }
@@ -685,12 +711,17 @@ __device__ __forceinline__ void op_memory(const TranDev &D, int c, const CktCtl 
     }
 }
 
-/* minimum of one value per lane over the step kernel's workgroup, which
- * is one wavefront: register exchanges, no LDS (min is exact in any order) */
-__device__ double wave_min(double v)
+/* minimum of one value per lane over the step kernel's workgroup (min is
+ * exact in any order); a barrier of its own after every lane's value */
+__device__ __forceinline__ double group_min(double v)
 {
+    __shared__ double m[4];
 #pragma unroll
     for (int s = 32; s > 0; s >>= 1) v = fmin(v, __shfl_xor(v, s));
+    if ((threadIdx.x & 63) == 0) m[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = m[0];
+    for (int w = 1; w < (int)(blockDim.x >> 6); w++) v = fmin(v, m[w]);
     return v;
 }
 
@@ -731,7 +762,7 @@ __device__ __forceinline__ double circuit_terr(const TranDev &D, const CktCtl *K
 #pragma unroll
         for (int r = 0; r < 3; r++) m = fmin(m, terr_one(q0[r], q1[r], q2[r], q3[r], c0[r], c1[r], K, D));
     }
-    return wave_min(m);
+    return group_min(m);
 }
 
 /* copy state level `from` to level `to` for every state of the circuit */
@@ -973,69 +1004,185 @@ __device__ __forceinline__ Prog load_prog(const int4 *base, int e)
     return r;
 }
 
-/* further term groups loaded per batch by the one lane that owns a long
- * row (a supply node's row has ~45 groups on the adder) */
-constexpr int TERM_BATCH = 8;
+/* a record's term groups beyond the inline ones (a circuit's supply row has
+ * hundreds of terms, in partial sums; many rows have 13 to 24) */
+struct Extra {
+    uint4 w[PROG_EXTRA];
+    __device__ __forceinline__ const Extra &get(const Prog &) const { return *this; }
+};
 
-/* acc minus the record's term groups, in order: the inline ones, then the
- * further groups [h.z, h.w), TERM_BATCH at a time, loaded unconditionally
- * (clamped to the last group) so that the wait counts stay exact */
-__device__ __forceinline__ double lu_row_terms(double acc, const Prog &r, const uint4 *T,
+__device__ __forceinline__ Extra load_extra(const uint4 *T, const Prog &r)
+{
+    const int n = ((r.h.x >> 20) & 3) == PROG_COMBINE ? 0 : r.h.w - r.h.z;
+    Extra x;
+#pragma unroll
+    for (int k = 0; k < PROG_EXTRA; k++) x.w[k] = gload(T + (n > 0 ? r.h.z + min(k, n - 1) : 0));
+    return x;
+}
+
+/* ... loaded when they are needed */
+struct ExtraLate {
+    const uint4 *T;
+    __device__ __forceinline__ Extra get(const Prog &r) const { return load_extra(T, r); }
+};
+
+/* acc minus the record's term groups, in order.  The lanes' groups are read
+ * from LDS together, absent ones as the pad (a product of two zeros), with
+ * the branches taken by the wavefront's longest entry: entries of a level
+ * are ordered by their groups. */
+template <class E>
+__device__ __forceinline__ double lu_row_terms(double acc, const Prog &r, const E &ex, uint32_t pad,
                                                const double *x, const double *y)
 {
-    const int g = (r.h.x >> 16) & 3;
-    if (g > 0) acc = sub_terms(acc, r.g0, x, y);
-    if (g > 1) acc = sub_terms(acc, r.g1, x, y);
-    if (g > 2) acc = sub_terms(acc, r.g2, x, y);
-    for (int q = r.h.z; q < r.h.w; q += TERM_BATCH) {
-        uint4 w[TERM_BATCH];
+    const int g = (r.h.x >> 16) & 3, n = r.h.w - r.h.z;
+    if (!__any(g > 1)) return __any(g > 0) ? sub_terms(acc, r.g0, x, y) : acc;
+    auto three = [&](const uint4 (&w)[3]) {
+        double a[12], b[12];
 #pragma unroll
-        for (int k = 0; k < TERM_BATCH; k++) w[k] = gload(T + min(q + k, r.h.w - 1));
+        for (int k = 0; k < 3; k++) {
+            const uint32_t q[4] = {w[k].x, w[k].y, w[k].z, w[k].w};
 #pragma unroll
-        for (int k = 0; k < TERM_BATCH; k++)
-            if (q + k < r.h.w) acc = sub_terms(acc, w[k], x, y);
+            for (int i = 0; i < 4; i++) {
+                a[4 * k + i] = x[q[i] & 0xffffu];
+                b[4 * k + i] = y[q[i] >> 16];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 12; k++) acc -= a[k] * b[k];
+    };
+    three({r.g0, r.g1, r.g2});
+    if (__any(n > 0)) {
+        const Extra t = ex.get(r);
+        uint4 w[PROG_EXTRA];
+#pragma unroll
+        for (int k = 0; k < PROG_EXTRA; k++) w[k] = k < n ? t.w[k] : make_uint4(pad, pad, pad, pad);
+        three(w);
     }
     return acc;
 }
 
-/* record kinds (bits 20-21 of the header's first int) */
-constexpr int PROG_PARTIAL = 1, PROG_COMBINE = 2;
-
-/* acc plus the partial sums [h.z, h.w) of a combine record, in order */
-__device__ __forceinline__ double add_parts(double acc, const Prog &r, const double *part)
+/* acc / piv, from the pivot's reciprocal unless the quotient's steps could
+ * leave the range of normal numbers */
+__device__ __forceinline__ double quotient(double acc, double piv, double inv)
 {
-    for (int p = r.h.z; p < r.h.w; p++) acc += part[p];
+    const double p = fabs(piv), a = fabs(acc);
+    if (p > 0x1p-400 && p < 0x1p400 && a > 0x1p-500 && a < 0x1p500) return div_by(acc, piv, inv);
+    return acc / piv;
+}
+
+/* doubles of a sum read together */
+constexpr int TERM_BATCH = 8;
+
+/* acc plus part[p0, p1) in order, read TERM_BATCH at a time */
+__device__ __forceinline__ double sum_parts(double acc, const double *part, int p0, int p1)
+{
+    for (int p = p0; p < p1; p += TERM_BATCH) {
+        double t[TERM_BATCH];
+#pragma unroll
+        for (int k = 0; k < TERM_BATCH; k++) t[k] = part[min(p + k, p1 - 1)];
+#pragma unroll
+        for (int k = 0; k < TERM_BATCH; k++)
+            if (p + k < p1) acc += t[k];
+    }
     return acc;
 }
 
-/* Level-scheduled program: entries of level L (lev[L] .. lev[L+1]) are
- * independent; a barrier separates levels.  Lane t runs the entries
- * lev[0] + t + k nt, whatever their level, and keeps the records of its
- * next two entries in flight.  Where levels are narrow (a chain of a few
- * entries each) those records belong to levels far ahead, so their loads
- * overlap many levels' work. */
+/* acc plus the partial sums of a combine record */
+__device__ __forceinline__ double add_parts(double acc, const Prog &r, const double *part)
+{
+    return sum_parts(acc, part, r.h.z, r.h.w);
+}
+
+/* one wavefront's memory accesses before it are seen by all its lanes after
+ * it */
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+/* Level-scheduled programs: entries of level L (lev[L] .. lev[L+1], the table
+ * staged in LDS) are independent; a barrier separates levels.  All record
+ * loads are unconditional (clamped to the last entry), so that the compiler's
+ * wait counts stay exact.
+ *
+ * One wavefront: lane t runs the entries t + k 64, whatever their level, and
+ * keeps the records of its next two in flight.  Every level has some lane
+ * loading its next record, so each waits for memory (~1700 cycles where the
+ * circuit is alone), which the compute unit's other circuits cover. */
 template <class F>
-__device__ __forceinline__ void run_levels(const int *lev, const int4 *ent, int nlev, int tid, int nt,
-                                           F body)
-{   /* lev: the level table staged in LDS */
+__device__ __forceinline__ void run_levels(const int *lev, const int4 *ent, const uint4 *T, int nlev, int tid, F body)
+{
     if (nlev <= 0) return;
     const int total = lev[nlev];
-    if (total <= lev[0]) return;
-    int e = lev[0] + tid;
-    /* unconditional prefetches (clamped to the last entry), so that the
-     * compiler's wait counts stay exact */
+    int e = tid;
     Prog p0 = load_prog(ent, min(e, total - 1));
-    Prog p1 = load_prog(ent, min(e + nt, total - 1));
+    Prog p1 = load_prog(ent, min(e + ONE_WAVE, total - 1));
     for (int L = 0; L < nlev; L++) {
         const int end = lev[L + 1];
         while (e < end) {
             const Prog cur = p0;
             p0 = p1;
-            p1 = load_prog(ent, min(e + 2 * nt, total - 1));
-            body(cur);
-            e += nt;
+            p1 = load_prog(ent, min(e + 2 * ONE_WAVE, total - 1));
+            body(cur, ExtraLate{T});
+            e += ONE_WAVE;
         }
         __syncthreads();
+    }
+}
+
+/* a wide workgroup's first records of a program, a lane's of three windows */
+struct Ahead {
+    Prog a, b, c;
+};
+
+__device__ __forceinline__ Ahead load_ahead(const int4 *ent, int total, int tid)
+{
+    constexpr int nt = STEP_WIDE;
+    const int last = max(total - 1, 0);   /* an empty program has one record of padding */
+    return {load_prog(ent, min(tid, last)), load_prog(ent, min(tid + nt, last)), load_prog(ent, min(tid + 2 * nt, last))};
+}
+
+/* Four wavefronts: the entries, in order, are taken in windows of 256: lane t
+ * has entry t of each, and runs it when its level comes.  A window's records
+ * (h: the first three's) are loaded three windows ahead, all lanes at once,
+ * and its term groups beyond the record, from T, a window ahead; a level
+ * waits for memory only where its window begins. */
+template <class F>
+__device__ __forceinline__ void run_levels_wide(const int *lev, const int4 *ent, const uint4 *T, int nlev, int tid,
+                                                Ahead &h, F body)
+{
+    constexpr int nt = STEP_WIDE;
+    if (nlev <= 0) return;
+    const int total = __builtin_amdgcn_readfirstlane(lev[nlev]);
+    int L = 0, start = 0, end = __builtin_amdgcn_readfirstlane(lev[1]);
+    auto window = [&](const Prog &r, const Extra &x, int base) {
+        const int e = base + tid, stop = base + nt;
+        while (start < stop) {
+            const int next = lev[min(L + 2, nlev)];
+            if (e >= start && e < end) body(r, x);
+            if (end > stop) break;   /* the level goes on in the next window */
+            __syncthreads();
+            if (++L >= nlev) break;
+            start = end;
+            end = __builtin_amdgcn_readfirstlane(next);
+        }
+    };
+    Extra xa = load_extra(T, h.a), xb, xc;
+    for (int base = 0; L < nlev && base < total; base += 3 * nt) {
+        xb = load_extra(T, h.b);
+        window(h.a, xa, base);
+        if (L >= nlev) break;
+        h.a = load_prog(ent, min(base + 3 * nt + tid, total - 1));
+        xc = load_extra(T, h.c);
+        window(h.b, xb, base + nt);
+        if (L >= nlev) break;
+        h.b = load_prog(ent, min(base + 4 * nt + tid, total - 1));
+        xa = load_extra(T, h.a);
+        window(h.c, xc, base + 2 * nt);
+        if (L >= nlev) break;
+        h.c = load_prog(ent, min(base + 5 * nt + tid, total - 1));
     }
 }
 
@@ -1044,23 +1191,38 @@ __device__ __forceinline__ void run_levels(const int *lev, const int4 *ent, int 
  * four values, U leaves per batch with the next batch's loads in flight;
  * past-the-end loads are clamped to the last leaf so that the wait counts
  * stay exact. */
+template <int U>
+struct PlainAhead {
+    int da[U / 2], db[U / 2];
+    double4 va[U / 2], vb[U / 2];
+};
+
+template <int U>
+__device__ __forceinline__ PlainAhead<U> plain_ahead(const int *dest, const double4 *val, int n, int tid, int nt)
+{
+    PlainAhead<U> p;
+    constexpr int H = U / 2;
+    const int last = max(n - 1, 0);
+#pragma unroll
+    for (int k = 0; k < H; k++) {
+        const int e = min(tid + k * nt, last), f = min(tid + (H + k) * nt, last);
+        p.da[k] = gload(dest + e);
+        p.va[k] = gload4(val + e);
+        p.db[k] = gload(dest + f);
+        p.vb[k] = gload4(val + f);
+    }
+    return p;
+}
+
 template <int U, class F>
 __device__ __forceinline__ void run_plain(const int *dest, const double4 *val, int n, int tid, int nt,
-                                          F body)
+                                          PlainAhead<U> &p, F body)
 {
     if (n <= 0) return;
     /* two half-batches of U/2 leaves each, held in scalar registers */
     constexpr int H = U / 2;
-    int da[H], db[H];
-    double4 va[H], vb[H];
-#pragma unroll
-    for (int k = 0; k < H; k++) {
-        const int e = min(tid + k * nt, n - 1), f = min(tid + (H + k) * nt, n - 1);
-        da[k] = gload(dest + e);
-        va[k] = gload4(val + e);
-        db[k] = gload(dest + f);
-        vb[k] = gload4(val + f);
-    }
+    int (&da)[H] = p.da, (&db)[H] = p.db;
+    double4 (&va)[H] = p.va, (&vb)[H] = p.vb;
     for (int e0 = tid; e0 < n; e0 += U * nt) {
         int dc[H], dd[H];
         double4 vc[H], vd[H];
@@ -1096,22 +1258,36 @@ __device__ __forceinline__ void run_plain(const int *dest, const double4 *val, i
  * one batch earlier.  With MULTI, the second group of each current leaf
  * that has one is requested before the next leaves' loads, so waiting for
  * it does not wait for them (loads complete in order). */
-template <int U, bool MULTI, class F>
-__device__ __forceinline__ void run_leaves(const int4 *leaf, const double4 *val, const uint4 *code,
-                                           int e_begin, int n, int tid, int nt, F body)
+template <int U>
+struct LeavesAhead {
+    Rec r[U];
+    double4 v[U];
+};
+
+template <int U>
+__device__ __forceinline__ LeavesAhead<U> leaves_ahead(const int4 *leaf, const double4 *val, int e_begin, int n, int tid,
+                                                       int nt)
 {
-    if (n <= e_begin) return;
     /* prefetch loads are unconditional (past-the-end indices clamped to the
      * last leaf): the compiler can then count exactly how many loads are
      * outstanding and wait only for the ones a leaf needs */
-    Rec rb[U];
-    double4 vb[U];
+    LeavesAhead<U> p;
 #pragma unroll
     for (int k = 0; k < U; k++) {
-        const int e = min(e_begin + tid + k * nt, n - 1);
-        rb[k] = load_rec(leaf, e);
-        vb[k] = gload4(val + e);
+        const int e = max(min(e_begin + tid + k * nt, n - 1), 0);
+        p.r[k] = load_rec(leaf, e);
+        p.v[k] = gload4(val + e);
     }
+    return p;
+}
+
+template <int U, bool MULTI, class F>
+__device__ __forceinline__ void run_leaves(const int4 *leaf, const double4 *val, const uint4 *code,
+                                           int e_begin, int n, int tid, int nt, LeavesAhead<U> &p, F body)
+{
+    if (n <= e_begin) return;
+    Rec (&rb)[U] = p.r;
+    double4 (&vb)[U] = p.v;
     for (int e0 = e_begin + tid; e0 < n; e0 += U * nt) {
         Rec rc[U];
         double4 vc[U];
@@ -1169,14 +1345,11 @@ __device__ __forceinline__ double rhs_value(uint32_t code, double mv, const doub
     return (code & CT_NEG) ? -v : v;
 }
 
-/* one wavefront per circuit: the level-scheduled LU program has a few
- * dozen entries per level, and a one-wave workgroup makes each level's
- * barrier nearly free while many circuits share a compute unit */
-constexpr int STEP_THREADS = 64;
-static_assert(STEP_THREADS == 64, "the step kernel's reductions assume one wavefront");
 /* assembly leaves whose loads are issued together, per lane */
 constexpr int ASM_UNROLL = 4;
 constexpr int PLAIN_UNROLL = 8;
+/* ... and by four wavefronts, all of them ahead of the capacitors */
+constexpr int WIDE_PLAIN = 4, WIDE_LEAVES = 2;
 /* unknowns (and device votes) a lane loads together in the convergence test */
 constexpr int CONV_CHUNK = 8;
 
@@ -1253,7 +1426,8 @@ __device__ __forceinline__ bool guess_feature_row(double v0, double v1, double v
  */
 __device__ __forceinline__ void guess_rows(const TranDev &D, const CktCtl *K, int c, int *list)
 {
-    const int tid = threadIdx.x, nt = blockDim.x;
+    constexpr int nt = ONE_WAVE;
+    const int tid = threadIdx.x;
     const int lane = (int)__lane_id();
     const int s0 = (K->hpos + 3) & 3, s1 = (K->hpos + 2) & 3, s2 = (K->hpos + 1) & 3, s3 = K->hpos;
     const double t0 = K->ht[s0], t1 = K->ht[s1], t2 = K->ht[s2], t3 = K->ht[s3], h = K->delta;
@@ -1287,7 +1461,7 @@ __device__ __forceinline__ void guess_rows(const TranDev &D, const CktCtl *K, in
     int first = 0;
     if (tid == 0) first = atomicAdd(D.gcount + 2 * hs, n_on);
     first = __shfl(first, 0);
-    __syncthreads();   /* the list is complete */
+    wave_sync();   /* the list is complete */
     for (int k = tid; k < n_on; k += nt) {
         const int u = list[k];
         double nbv[8];
@@ -1322,7 +1496,7 @@ constexpr int PV_POLLS = 1 << 22;
 constexpr int PV_NO_WORKSPACE = 108;
 
 /* the largest of one value per lane (ties to the lowest key) with its
- * index, and a sum, over the one-wavefront workgroup; fixed exchange order */
+ * index, and a sum, over one wavefront; fixed exchange order */
 __device__ __forceinline__ void wave_argmax(double &v, int &key, int &i)
 {
 #pragma unroll
@@ -1382,7 +1556,7 @@ __device__ __forceinline__ int pivot_solve(const TranDev &D, CktCtl *K, int c, c
         }
         s_ws = got;
     }
-    __syncthreads();
+    wave_sync();
     const int ws = s_ws;
     if (ws < 0) return PV_BUSY;
     const int64_t nld = (int64_t)N * ld;
@@ -1391,9 +1565,9 @@ __device__ __forceinline__ int pivot_solve(const TranDev &D, CktCtl *K, int c, c
     double *Rs = D.pv_rs + (int64_t)c * N;
     int *prow_g = D.pv_row + (int64_t)c * N;
 
-    for (int64_t e = tid; e < nld; e += STEP_THREADS) A0[e] = 0.0;
-    __syncthreads();
-    for (int a = tid; a < N; a += STEP_THREADS) {
+    for (int64_t e = tid; e < nld; e += ONE_WAVE) A0[e] = 0.0;
+    wave_sync();
+    for (int a = tid; a < N; a += ONE_WAVE) {
         const int s0 = gload(D.row_start + a), s1 = gload(D.row_start + a + 1);
         double *row = A0 + (int64_t)a * ld;
         double m = 0.0;
@@ -1405,7 +1579,7 @@ __device__ __forceinline__ int pivot_solve(const TranDev &D, CktCtl *K, int c, c
         row[N] = z[a];
         Rs[a] = m == 0.0 ? 1.0 : m;
     }
-    __syncthreads();
+    wave_sync();
     /* scratch over lu, z and what follows: multipliers (later the solution),
      * the pivot row's values, then the bookkeeping */
     double *lval = sm, *uval = sm + N, *x = sm;
@@ -1416,8 +1590,8 @@ __device__ __forceinline__ int pivot_solve(const TranDev &D, CktCtl *K, int c, c
 
     int status;
     for (;;) {
-        for (int64_t e = tid; e < nld; e += STEP_THREADS) W[e] = A0[e];
-        for (int a = tid; a < N; a += STEP_THREADS) {
+        for (int64_t e = tid; e < nld; e += ONE_WAVE) W[e] = A0[e];
+        for (int a = tid; a < N; a += ONE_WAVE) {
             Pinv[a] = full ? -1 - a : -1;
             Pd[a] = a;
             prw[a] = full ? a : prow_g[a];
@@ -1426,7 +1600,7 @@ __device__ __forceinline__ int pivot_solve(const TranDev &D, CktCtl *K, int c, c
             if (full) K->pvfull++;
             else K->pvrefac++;
         }
-        __syncthreads();
+        wave_sync();
         status = PV_OK;
         for (int k = 0; k < N; k++) {
             int p;
@@ -1434,7 +1608,7 @@ __device__ __forceinline__ int pivot_solve(const TranDev &D, CktCtl *K, int c, c
                 /* the candidates' original rows break ties */
                 double best = -1.0;
                 int bkey = INT_MAX, bi = N;
-                for (int a = tid; a < N; a += STEP_THREADS)
+                for (int a = tid; a < N; a += ONE_WAVE)
                     if (Pinv[a] < 0) {
                         const double v = fabs(W[(int64_t)a * ld + k]) / Rs[a];
                         const int key = gload(D.perm_unknown + N + a);
@@ -1456,7 +1630,7 @@ __device__ __forceinline__ int pivot_solve(const TranDev &D, CktCtl *K, int c, c
                 status = PV_SINGULAR;
                 break;
             }
-            __syncthreads();
+            wave_sync();
             if (tid == 0) {
                 if (full) {
                     const int d = Pd[k];
@@ -1469,11 +1643,11 @@ __device__ __forceinline__ int pivot_solve(const TranDev &D, CktCtl *K, int c, c
                 }
                 Pinv[p] = k;
             }
-            __syncthreads();
+            wave_sync();
             /* rows still to eliminate with a nonzero in column k, and their
              * multipliers; the pivot row's nonzeros right of column k */
             int nr = 0, nc = 0;
-            for (int a0 = 0; a0 < N; a0 += STEP_THREADS) {
+            for (int a0 = 0; a0 < N; a0 += ONE_WAVE) {
                 const int a = a0 + tid;
                 const double xv = (a < N && Pinv[a] < 0) ? W[(int64_t)a * ld + k] : 0.0;
                 const bool on = xv != 0.0;
@@ -1486,7 +1660,7 @@ __device__ __forceinline__ int pivot_solve(const TranDev &D, CktCtl *K, int c, c
                 nr += __popcll(m);
             }
             const double *pr = W + (int64_t)p * ld;
-            for (int j0 = k + 1; j0 <= N; j0 += STEP_THREADS) {
+            for (int j0 = k + 1; j0 <= N; j0 += ONE_WAVE) {
                 const int j = j0 + tid;
                 const double u = j <= N ? pr[j] : 0.0;
                 const bool on = u != 0.0;
@@ -1498,43 +1672,44 @@ __device__ __forceinline__ int pivot_solve(const TranDev &D, CktCtl *K, int c, c
                 }
                 nc += __popcll(m);
             }
-            __syncthreads();
+            wave_sync();
             const int tot = nr * nc;
-            for (int e = tid; e < tot; e += STEP_THREADS) {
+            for (int e = tid; e < tot; e += ONE_WAVE) {
                 const int r = e / nc, q = e - r * nc;
                 double *w = W + (int64_t)rl[r] * ld + cl[q];
                 *w = fma(-lval[r], uval[q], *w);
             }
-            __syncthreads();
+            wave_sync();
         }
         if (status == PV_OK || full) break;
         full = true;
         *refailed = true;
-        __syncthreads();
+        wave_sync();
     }
     if (status == PV_OK) {
-        __syncthreads();
+        wave_sync();
         for (int k = N - 1; k >= 0; k--) {
             const double *row = W + (int64_t)prw[k] * ld;
             double acc = 0.0;
-            for (int j = k + 1 + tid; j < N; j += STEP_THREADS) acc = fma(row[j], x[j], acc);
+            for (int j = k + 1 + tid; j < N; j += ONE_WAVE) acc = fma(row[j], x[j], acc);
             acc = wave_sum(acc);
             if (tid == 0) x[k] = (row[N] - acc) / row[k];
-            __syncthreads();
+            wave_sync();
         }
         if (full)
-            for (int k = tid; k < N; k += STEP_THREADS) prow_g[k] = prw[k];
-        __syncthreads();
+            for (int k = tid; k < N; k += ONE_WAVE) prow_g[k] = prw[k];
+        wave_sync();
         /* x lies in lu's part of the scratch (nslots >= N), clear of z */
-        for (int k = tid; k < N; k += STEP_THREADS) z[k] = x[k];
+        for (int k = tid; k < N; k += ONE_WAVE) z[k] = x[k];
     }
     __threadfence();
-    __syncthreads();
+    wave_sync();
     if (tid == 0) atomicExch(D.pv_owner + ws, 0);
     return status;
 }
 
 /* circuit c of the topology D, one workgroup */
+template <bool WIDE>
 __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
 {
     extern __shared__ double sm[];
@@ -1542,8 +1717,13 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
     __shared__ int s_act;
     __shared__ int s_guess;
     __shared__ int s_pvbad;
+    __shared__ int s_quit;     /* the iteration ends with the solve */
+    __shared__ int s_next;     /* what follows a finished Newton run */
+    __shared__ int s_opt;      /* ... an OPtran step */
+    __shared__ int s_stop;
 
-    const int tid = threadIdx.x, nt = blockDim.x;
+    const int tid = threadIdx.x;
+    constexpr int nt = WIDE ? STEP_WIDE : ONE_WAVE;
     CktCtl *K = D.ctl + c;
     if (K->phase >= PH_DONE) return;
     const int N = D.N;
@@ -1559,8 +1739,28 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
     const int64_t cnc = (int64_t)D.C * D.NCAP;
     double *xo = D.x + ((int64_t)xs * D.C + c) * (N + 1);
     double *xn = D.x + ((int64_t)(xs ^ 1) * D.C + c) * (N + 1);
+    const uint4 *AC = reinterpret_cast<const uint4 *>(D.a_code);
+    const uint4 *RC = reinterpret_cast<const uint4 *>(D.r_code);
+    /* the circuit's contribution values, four per group: consecutive leaves
+     * read consecutive groups, so a wavefront's loads are contiguous */
+    const double4 *AV = reinterpret_cast<const double4 *>(D.contrib + (int64_t)c * D.NA);
+    const double4 *RV = reinterpret_cast<const double4 *>(D.rcontrib + (int64_t)c * D.NR);
+    /* a wide workgroup's last wavefront assembles the right-hand side beside
+     * the matrix; the first leaves' loads wait beside the capacitors' */
+    const bool rhs = WIDE && tid >= STEP_WIDE - ONE_WAVE;
+    const int tw = rhs ? ONE_WAVE : STEP_WIDE - ONE_WAVE, tl = rhs ? tid - (STEP_WIDE - ONE_WAVE) : tid;
+    PlainAhead<WIDE_PLAIN> p0;
+    LeavesAhead<WIDE_LEAVES> p1, p2;
+    if constexpr (WIDE) {
+        const int4 *leaf = rhs ? D.r_leaf : D.a_leaf;
+        const double4 *V = rhs ? RV : AV;
+        const int n0 = rhs ? D.n_rplain : D.n_aplain, n1 = rhs ? D.n_rleaf1 : D.n_aleaf1, n2 = rhs ? D.n_rleaf : D.n_aleaf;
+        p0 = plain_ahead<WIDE_PLAIN>(rhs ? D.r_dest : D.a_dest, V, n0, tl, tw);
+        p1 = leaves_ahead<WIDE_LEAVES>(leaf, V, n0, n1, tl, tw);
+        p2 = leaves_ahead<WIDE_LEAVES>(leaf, V, n1, n2, tl, tw);
+    }
     if (tid < 4) s_flag[tid] = 0;
-    if (tid == 0) s_pvbad = 0;
+    if (tid == 0) s_pvbad = s_quit = 0;
     /* NIiter factors afresh (SMPreorder, klu_factor) when NISHOULDREORDER
      * is set, on INITJCT and on the first INITTRAN iteration
      * (niiter.c:107-146), else refactors on the current pivot rows */
@@ -1616,7 +1816,7 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
         capg[k] = geq;
         capq[k] = ceq;
     }
-    for (int k = tid; k < D.NVS; k += nt)
+    for (int k = nt - 1 - tid; k < D.NVS; k += nt)   /* from the last lane: the first ones have capacitors */
     {
         /* vsrcload.c:453-457: the operating point scales sources by
          * CKTsrcFact */
@@ -1653,12 +1853,6 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
     for (int k = tid; k <= D.nlev_f; k += nt) levf[k] = gload(D.f_lev + k);
     for (int k = tid; k <= D.nlev_fw; k += nt) levw[k] = gload(D.fw_lev + k);
     for (int k = tid; k <= D.nlev_bw; k += nt) levb[k] = gload(D.bw_lev + k);
-    const uint4 *AC = reinterpret_cast<const uint4 *>(D.a_code);
-    const uint4 *RC = reinterpret_cast<const uint4 *>(D.r_code);
-    /* the circuit's contribution values, four per group: consecutive leaves
-     * read consecutive groups, so a wavefront's loads are contiguous */
-    const double4 *AV = reinterpret_cast<const double4 *>(D.contrib + (int64_t)c * D.NA);
-    const double4 *RV = reinterpret_cast<const double4 *>(D.rcontrib + (int64_t)c * D.NR);
     /* the sum of one leaf: its first group (codes from the record, values
      * already loaded), then its further groups in order */
     auto a_leaf_sum = [&](const Rec &lf, const double4 &m0, const uint4 &w1, const double4 &m1) {
@@ -1684,29 +1878,6 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
         if (lf.h.x < D.nslots) lu[lf.h.x] = ((lf.h.w & 1) && icz) ? 1.0 : acc;
         else part[lf.h.x - D.nslots] = acc;
     };
-    /* single-group leaves: no further groups, and no code that could load
-     * them (a load anywhere in the body makes the compiler wait for all
-     * outstanding loads after it, the prefetched leaves' included) */
-    run_plain<PLAIN_UNROLL>(D.a_dest, AV, D.n_aplain, tid, nt, [&](int d, double4 m) {
-        double acc = 0.0;
-        acc += m.x;
-        acc += m.y;
-        acc += m.z;
-        acc += m.w;
-        if (d < D.nslots) lu[d] = acc;
-        else part[d - D.nslots] = acc;
-    });
-    run_leaves<ASM_UNROLL, false>(D.a_leaf, AV, AC, D.n_aplain, D.n_aleaf1, tid, nt,
-                                  [&](const Rec &lf, const double4 &m0, const uint4 &, const double4 &) {
-        double acc = 0.0;
-        acc += mat_value(lf.g.x, m0.x, capg, icz);
-        acc += mat_value(lf.g.y, m0.y, capg, icz);
-        acc += mat_value(lf.g.z, m0.z, capg, icz);
-        acc += mat_value(lf.g.w, m0.w, capg, icz);
-        if (lf.h.x < D.nslots) lu[lf.h.x] = ((lf.h.w & 1) && icz) ? 1.0 : acc;
-        else part[lf.h.x - D.nslots] = acc;
-    });
-    run_leaves<ASM_UNROLL, true>(D.a_leaf, AV, AC, D.n_aleaf1, D.n_aleaf, tid, nt, a_leaf_sum);
     auto r_leaf_sum = [&](const Rec &lf, const double4 &m0, const uint4 &w1, const double4 &m1) {
         double acc = 0.0;
         acc += rhs_value(lf.g.x, m0.x, capq, vsv);
@@ -1730,7 +1901,28 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
         if (lf.h.x < N) z[lf.h.x] = acc;
         else part[D.n_apart + lf.h.x - N] = acc;
     };
-    run_plain<PLAIN_UNROLL>(D.r_dest, RV, D.n_rplain, tid, nt, [&](int d, double4 m) {
+    /* single-group leaves: no further groups, and no code that could load
+     * them (a load anywhere in the body makes the compiler wait for all
+     * outstanding loads after it, the prefetched leaves' included) */
+    auto a_plain = [&](int d, double4 m) {
+        double acc = 0.0;
+        acc += m.x;
+        acc += m.y;
+        acc += m.z;
+        acc += m.w;
+        if (d < D.nslots) lu[d] = acc;
+        else part[d - D.nslots] = acc;
+    };
+    auto a_single = [&](const Rec &lf, const double4 &m0, const uint4 &, const double4 &) {
+        double acc = 0.0;
+        acc += mat_value(lf.g.x, m0.x, capg, icz);
+        acc += mat_value(lf.g.y, m0.y, capg, icz);
+        acc += mat_value(lf.g.z, m0.z, capg, icz);
+        acc += mat_value(lf.g.w, m0.w, capg, icz);
+        if (lf.h.x < D.nslots) lu[lf.h.x] = ((lf.h.w & 1) && icz) ? 1.0 : acc;
+        else part[lf.h.x - D.nslots] = acc;
+    };
+    auto r_plain = [&](int d, double4 m) {
         double acc = 0.0;
         acc += m.x;
         acc += m.y;
@@ -1738,9 +1930,8 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
         acc += m.w;
         if (d < N) z[d] = acc;
         else part[D.n_apart + d - N] = acc;
-    });
-    run_leaves<ASM_UNROLL, false>(D.r_leaf, RV, RC, D.n_rplain, D.n_rleaf1, tid, nt,
-                                  [&](const Rec &lf, const double4 &m0, const uint4 &, const double4 &) {
+    };
+    auto r_single = [&](const Rec &lf, const double4 &m0, const uint4 &, const double4 &) {
         double acc = 0.0;
         acc += rhs_value(lf.g.x, m0.x, capq, vsv);
         acc += rhs_value(lf.g.y, m0.y, capq, vsv);
@@ -1748,21 +1939,58 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
         acc += rhs_value(lf.g.w, m0.w, capq, vsv);
         if (lf.h.x < N) z[lf.h.x] = acc;
         else part[D.n_apart + lf.h.x - N] = acc;
-    });
-    run_leaves<ASM_UNROLL, true>(D.r_leaf, RV, RC, D.n_rleaf1, D.n_rleaf, tid, nt, r_leaf_sum);
+    };
+    if constexpr (WIDE) {
+        if (!rhs) {
+            run_plain(D.a_dest, AV, D.n_aplain, tl, tw, p0, a_plain);
+            run_leaves<WIDE_LEAVES, false>(D.a_leaf, AV, AC, D.n_aplain, D.n_aleaf1, tl, tw, p1, a_single);
+            run_leaves<WIDE_LEAVES, true>(D.a_leaf, AV, AC, D.n_aleaf1, D.n_aleaf, tl, tw, p2, a_leaf_sum);
+        } else {
+            run_plain(D.r_dest, RV, D.n_rplain, tl, tw, p0, r_plain);
+            run_leaves<WIDE_LEAVES, false>(D.r_leaf, RV, RC, D.n_rplain, D.n_rleaf1, tl, tw, p1, r_single);
+            run_leaves<WIDE_LEAVES, true>(D.r_leaf, RV, RC, D.n_rleaf1, D.n_rleaf, tl, tw, p2, r_leaf_sum);
+        }
+    } else {
+        {
+            auto p = plain_ahead<PLAIN_UNROLL>(D.a_dest, AV, D.n_aplain, tid, nt);
+            run_plain(D.a_dest, AV, D.n_aplain, tid, nt, p, a_plain);
+        }
+        {
+            auto p = leaves_ahead<ASM_UNROLL>(D.a_leaf, AV, D.n_aplain, D.n_aleaf1, tid, nt);
+            run_leaves<ASM_UNROLL, false>(D.a_leaf, AV, AC, D.n_aplain, D.n_aleaf1, tid, nt, p, a_single);
+        }
+        {
+            auto p = leaves_ahead<ASM_UNROLL>(D.a_leaf, AV, D.n_aleaf1, D.n_aleaf, tid, nt);
+            run_leaves<ASM_UNROLL, true>(D.a_leaf, AV, AC, D.n_aleaf1, D.n_aleaf, tid, nt, p, a_leaf_sum);
+        }
+        {
+            auto p = plain_ahead<PLAIN_UNROLL>(D.r_dest, RV, D.n_rplain, tid, nt);
+            run_plain(D.r_dest, RV, D.n_rplain, tid, nt, p, r_plain);
+        }
+        {
+            auto p = leaves_ahead<ASM_UNROLL>(D.r_leaf, RV, D.n_rplain, D.n_rleaf1, tid, nt);
+            run_leaves<ASM_UNROLL, false>(D.r_leaf, RV, RC, D.n_rplain, D.n_rleaf1, tid, nt, p, r_single);
+        }
+        {
+            auto p = leaves_ahead<ASM_UNROLL>(D.r_leaf, RV, D.n_rleaf1, D.n_rleaf, tid, nt);
+            run_leaves<ASM_UNROLL, true>(D.r_leaf, RV, RC, D.n_rleaf1, D.n_rleaf, tid, nt, p, r_leaf_sum);
+        }
+    }
+    Ahead hf;
+    if constexpr (WIDE)
+        hf = load_ahead(reinterpret_cast<const int4 *>(D.f_ent), D.nlev_f > 0 ? gload(D.f_lev + D.nlev_f) : 0, tid);
     __syncthreads();
+    /* the matrix's combines from the first lane on, the right-hand side's
+     * from the last back */
     for (int e = tid; e < D.n_acomb; e += nt) {
         const int4 cb = gload(D.a_comb + e);
-        double acc = 0.0;
-        for (int p = cb.y; p < cb.z; p++) acc += part[p];
+        double acc = sum_parts(0.0, part, cb.y, cb.z);
         if ((cb.w & 1) && icz) acc = 1.0;
         lu[cb.x] = acc;
     }
-    for (int e = tid; e < D.n_rcomb; e += nt) {
+    for (int e = nt - 1 - tid; e < D.n_rcomb; e += nt) {
         const int4 cb = gload(D.r_comb + e);
-        double acc = 0.0;
-        for (int p = cb.y; p < cb.z; p++) acc += part[D.n_apart + p];
-        z[cb.x] = acc;
+        z[cb.x] = sum_parts(0.0, part + D.n_apart, cb.y, cb.z);
     }
     if (icz && D.n_icrow) {
         __syncthreads();
@@ -1788,13 +2016,14 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
     if (!uic_op) {
         bool refailed = false;
         if (dense) {
-            const int r = pivot_solve(D, K, c, lu, z, sm, full, &refailed);
-            if (r == PV_BUSY) {
-                if (tid == 0) fail(D, K, PV_NO_WORKSPACE);
-                return;
+            if (tid < ONE_WAVE) {
+                const int r = pivot_solve(D, K, c, lu, z, sm, full, &refailed);
+                if (tid == 0 && r == PV_BUSY) {
+                    fail(D, K, PV_NO_WORKSPACE);
+                    s_quit = 1;
+                }
+                if (tid == 0 && r == PV_SINGULAR) s_flag[0] = 1;
             }
-            if (r == PV_SINGULAR && tid == 0) s_flag[0] = 1;
-            __syncthreads();
         } else {
             if (reorder && can_pivot) {
                 /* KLU's row scale factors of the matrix being factored (klu_scale.c:
@@ -1809,48 +2038,62 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
                 }
             }
 
+            const uint32_t pad_lu = (uint32_t)D.nslots * 0x10001u, pad_z = (uint32_t)D.nslots | (uint32_t)N << 16;
+            const uint4 *FT = reinterpret_cast<const uint4 *>(D.f_term), *WT = reinterpret_cast<const uint4 *>(D.fw_term);
+            const uint4 *BT = reinterpret_cast<const uint4 *>(D.bw_term);
+            const int4 *FE = reinterpret_cast<const int4 *>(D.f_ent), *WE = reinterpret_cast<const int4 *>(D.fw_ent);
+            const int4 *BE = reinterpret_cast<const int4 *>(D.bw_ent);
             /* LU factorisation, entry-wise Doolittle by dependency levels, then the
              * two substitutions; see run_levels for the load schedule */
-            const uint4 *FT = reinterpret_cast<const uint4 *>(D.f_term);
-            run_levels(levf, reinterpret_cast<const int4 *>(D.f_ent), D.nlev_f, tid, nt,
-                       [&](const Prog &r) {
-                           const int t = r.h.x & 0xffff, kind = (r.h.x >> 20) & 3;
-                           if (kind == PROG_PARTIAL) {
-                               part[t] = lu_row_terms(0.0, r, FT, lu, lu);
-                               return;
-                           }
-                           const double acc = (kind == PROG_COMBINE) ? add_parts(lu[t], r, part)
-                                                                     : lu_row_terms(lu[t], r, FT, lu, lu);
-                           lu[t] = (r.h.y >= 0) ? acc / lu[r.h.y] : acc;
-                       });
+            auto lu_entry = [&](const Prog &r, const auto &ex) {
+                const int t = r.h.x & 0xffff, kind = (r.h.x >> 20) & 3;
+                if (kind == PROG_PARTIAL) {
+                    part[t] = lu_row_terms(0.0, r, ex, pad_lu, lu, lu);
+                    return;
+                }
+                /* the pivot's reciprocal forms beside the terms */
+                double acc = lu[t];
+                const double piv = lu[max(r.h.y, 0)], inv = recip(piv);
+                acc = (kind == PROG_COMBINE) ? add_parts(acc, r, part)
+                                             : lu_row_terms(acc, r, ex, pad_lu, lu, lu);
+                lu[t] = (r.h.y >= 0) ? quotient(acc, piv, inv) : acc;
+            };
             /* forward substitution (unit L) */
-            const uint4 *WT = reinterpret_cast<const uint4 *>(D.fw_term);
-            run_levels(levw, reinterpret_cast<const int4 *>(D.fw_ent), D.nlev_fw, tid, nt,
-                       [&](const Prog &r) {
-                           const int a = r.h.x & 0xffff, kind = (r.h.x >> 20) & 3;
-                           if (kind == PROG_PARTIAL) part[a] = lu_row_terms(0.0, r, WT, lu, z);
-                           else if (kind == PROG_COMBINE) z[a] = add_parts(z[a], r, part);
-                           else z[a] = lu_row_terms(z[a], r, WT, lu, z);
-                       });
+            auto fw_row = [&](const Prog &r, const auto &ex) {
+                const int a = r.h.x & 0xffff, kind = (r.h.x >> 20) & 3;
+                if (kind == PROG_PARTIAL) part[a] = lu_row_terms(0.0, r, ex, pad_z, lu, z);
+                else if (kind == PROG_COMBINE) z[a] = add_parts(z[a], r, part);
+                else z[a] = lu_row_terms(z[a], r, ex, pad_z, lu, z);
+            };
             /* back substitution */
-            const uint4 *BT = reinterpret_cast<const uint4 *>(D.bw_term);
-            run_levels(levb, reinterpret_cast<const int4 *>(D.bw_ent), D.nlev_bw, tid, nt,
-                       [&](const Prog &r) {
-                           const int a = r.h.x & 0xffff, kind = (r.h.x >> 20) & 3;
-                           if (kind == PROG_PARTIAL) {
-                               part[a] = lu_row_terms(0.0, r, BT, lu, z);
-                               return;
-                           }
-                           const double acc = (kind == PROG_COMBINE) ? add_parts(z[a], r, part)
-                                                                     : lu_row_terms(z[a], r, BT, lu, z);
-                           if (r.h.y < 0) {   /* a forward row of the block-by-block solve */
-                               z[a] = acc;
-                               return;
-                           }
-                           const double piv = lu[r.h.y];
-                           if (piv == 0.0 || !isfinite(piv)) s_flag[0] = 1;   /* E_SINGULAR */
-                           z[a] = acc / piv;
-                       });
+            auto bw_row = [&](const Prog &r, const auto &ex) {
+                const int a = r.h.x & 0xffff, kind = (r.h.x >> 20) & 3;
+                if (kind == PROG_PARTIAL) {
+                    part[a] = lu_row_terms(0.0, r, ex, pad_z, lu, z);
+                    return;
+                }
+                double acc = z[a];
+                const double piv = lu[max(r.h.y, 0)], inv = recip(piv);
+                acc = (kind == PROG_COMBINE) ? add_parts(acc, r, part)
+                                             : lu_row_terms(acc, r, ex, pad_z, lu, z);
+                if (r.h.y < 0) {   /* a forward row of the block-by-block solve */
+                    z[a] = acc;
+                    return;
+                }
+                if (piv == 0.0 || !isfinite(piv)) s_flag[0] = 1;   /* E_SINGULAR */
+                z[a] = quotient(acc, piv, inv);
+            };
+            if constexpr (WIDE) {
+                Ahead hw = load_ahead(WE, levw[D.nlev_fw], tid);
+                run_levels_wide(levf, FE, FT, D.nlev_f, tid, hf, lu_entry);
+                Ahead hb = load_ahead(BE, levb[D.nlev_bw], tid);
+                run_levels_wide(levw, WE, WT, D.nlev_fw, tid, hw, fw_row);
+                run_levels_wide(levb, BE, BT, D.nlev_bw, tid, hb, bw_row);
+            } else {
+                run_levels(levf, FE, FT, D.nlev_f, tid, lu_entry);
+                run_levels(levw, WE, WT, D.nlev_fw, tid, fw_row);
+                run_levels(levb, BE, BT, D.nlev_bw, tid, bw_row);
+            }
             if (can_pivot && reorder) {
                 /* would klu_factor keep the static rows?  Column k's diagonal stays
                  * the pivot when its scaled magnitude is at least pivrel times every
@@ -1872,15 +2115,17 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
             }
             if (can_pivot) {
                 __syncthreads();
-                if (s_flag[0] || s_pvbad) {
+                if (tid == 0 && (s_flag[0] || s_pvbad)) {
                     /* klu_factor would pivot elsewhere, or the refactor met a zero
                      * pivot: the iteration continues next pass with a dense
                      * factorization */
-                    if (tid == 0) K->pvhold = 1;
-                    return;
+                    K->pvhold = 1;
+                    s_quit = 1;
                 }
             }
         }
+        __syncthreads();
+        if (s_quit) return;
         if (tid == 0 && can_pivot && !s_flag[0]) {
             /* a successful SMPreorder clears NISHOULDREORDER; a refactor that
              * met a zero pivot and was factored afresh in the same iteration
@@ -2016,6 +2261,8 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
         op_memory(D, c, K, act - ACT_OPMEM);
         return;
     }
+    /* every wavefront has read a shared word or a scalar of K, and met a
+     * barrier, before the first lane writes it again */
     if (act == 10) {
         copy_level(D, c, K->rb, 0, 1);
         __syncthreads();
@@ -2034,34 +2281,34 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
                 K->delta = K->delta / 8;
                 if (K->firsttime) K->mode = (K->mode & M_UIC) | M_TRAN | M_INITTRAN;
                 K->order = 1;
-                s_act = ACT_RETRY;
+                s_next = ACT_RETRY;
             } else if (K->firsttime) {
                 K->firsttime = 0;
-                s_act = ACT_ACCEPT;
+                s_next = ACT_ACCEPT;
             } else {
-                s_act = ACT_LTE1;
+                s_next = ACT_LTE1;
             }
         }
         __syncthreads();
-        act = s_act;
+        act = s_next;
         if (act == ACT_LTE1) {
             const double t1 = circuit_terr(D, K, c);
             if (tid == 0) {
                 const double nd = fmin(2 * K->delta, t1);
 
                 if (nd > .9 * K->delta) {
-                    s_act = (K->order == 1 && K->maxOrder > 1) ? 30 : ACT_ACCEPT;
-                    if (s_act == 30) K->order = 2;
+                    s_next = (K->order == 1 && K->maxOrder > 1) ? 30 : ACT_ACCEPT;
+                    if (s_next == 30) K->order = 2;
                     else K->delta = nd;
                 } else {
                     K->time = K->time - K->delta;
                     if (!K->optran) K->rejected++;
                     K->delta = nd;
-                    s_act = ACT_RETRY;
+                    s_next = ACT_RETRY;
                 }
             }
             __syncthreads();
-            act = s_act;
+            act = s_next;
             if (act == 30) {
                 const double t2 = circuit_terr(D, K, c);
                 if (tid == 0) {
@@ -2073,42 +2320,46 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
             }
         }
     }
-    if (act == ACT_ACCEPT && K->optran) {
+    const bool optran = act == ACT_ACCEPT && K->optran;
+    __syncthreads();
+    if (optran) {
         /* OPtran's nextTime (optran.c:430-490): no output.  Its CKTaccept
          * runs VSRCaccept at CKTtime 0 into the transient's breakpoints,
          * which leaves them as the transient's own first accept at time 0
          * does; that accept runs below, so it is not repeated here. */
         if (tid == 0) {
-            s_act = ACT_NONE;
+            s_opt = ACT_NONE;
             if (K->time > K->breaks[0]) clr_break(K);
             if (almost_equal_ulps(K->time, K->finalTime, 100)) {
                 optran_end(K);
-                s_act = 10;
+                s_opt = 10;
             } else {
                 resume_block(K);
                 if (loop_top(K)) fail(D, K, 104);
             }
         }
         __syncthreads();
-        if (s_act != 10) return;
+        if (s_opt != 10) return;
         /* the operating point is found: into the transient, as after CKTop */
         copy_level(D, c, K->rb, 0, 1);
         __syncthreads();
     }
     if (act == ACT_ACCEPT) {
         /* nextTime: (dctran.c:352-455) */
-        if (tid == 0) {
-            s_act = ACT_ACCEPT;
-            if (vsrc_accept(D, c, K)) {
-                fail(D, K, 1);
-                s_act = ACT_STOP;
-            } else {
-                if (K->time > K->breaks[0]) clr_break(K);
-                K->accepted++;
+        if (tid < ONE_WAVE) {
+            const int bad = vsrc_accept(D, c, K);
+            if (tid == 0) {
+                s_stop = bad != 0;
+                if (bad) {
+                    fail(D, K, 1);
+                } else {
+                    if (K->time > K->breaks[0]) clr_break(K);
+                    K->accepted++;
+                }
             }
         }
         __syncthreads();
-        if (s_act == ACT_STOP) return;
+        if (s_stop) return;
         /* CKTdump: rhsOld of the accepted point; under UIC not at time 0
          * (dctran.c:416-419) */
         const double *xold = D.x + ((int64_t)K->xsel * D.C + c) * (N + 1);
@@ -2158,22 +2409,24 @@ __device__ __forceinline__ void tran_step_body(const TranDev &D, int c)
     /* the next step starts from the learned guess: its feature rows (the
      * LU workspace in LDS is free by now) */
     __syncthreads();
-    if (s_guess) guess_rows(D, K, c, reinterpret_cast<int *>(sm));
+    if (s_guess && tid < ONE_WAVE) guess_rows(D, K, c, reinterpret_cast<int *>(sm));
 }
 
 /* one topology, one workgroup per circuit, circuits c0.. */
-__global__ void __launch_bounds__(STEP_THREADS)
+template <bool WIDE>
+__global__ void __launch_bounds__(WIDE ? STEP_WIDE : ONE_WAVE)
 k_tran_step(TranDev D, int c0)
 {
-    tran_step_body(D, c0 + blockIdx.x);
+    tran_step_body<WIDE>(D, c0 + blockIdx.x);
 }
 
 /* several topologies: blk[b] = (group, circuit) */
-__global__ void __launch_bounds__(STEP_THREADS)
+template <bool WIDE>
+__global__ void __launch_bounds__(WIDE ? STEP_WIDE : ONE_WAVE)
 k_tran_step_groups(const TranDev *__restrict__ Ds, const int2 *__restrict__ blk)
 {
     const int2 bg = blk[blockIdx.x];
-    tran_step_body(Ds[bg.x], bg.y);
+    tran_step_body<WIDE>(Ds[bg.x], bg.y);
 }
 
 /* the same rows for caller-supplied windows: row i from t[4i..4i+3],
@@ -2242,10 +2495,11 @@ int launch_zero_int(int *p, hipStream_t s)
 
 int set_tran_lds_limit(size_t bytes)
 {
-    NGMI_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_tran_step),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
-    NGMI_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_tran_step_groups),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    const void *f[] = {reinterpret_cast<const void *>(&k_tran_step<false>),
+                       reinterpret_cast<const void *>(&k_tran_step<true>),
+                       reinterpret_cast<const void *>(&k_tran_step_groups<false>),
+                       reinterpret_cast<const void *>(&k_tran_step_groups<true>)};
+    for (const void *k : f) NGMI_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
     return NGMI_OK;
 }
 
@@ -2296,12 +2550,18 @@ int launch_tran_pass(const MosLaunch &M, const TranDev *D0, int c_begin, int c_e
         NGMI_HIP(hipGetLastError());
     }
     if (ev) NGMI_HIP(hipEventRecord(ev[1], s));
-    if (D0)
-        hipLaunchKernelGGL(k_tran_step, dim3((unsigned)(c_end - c_begin)), dim3(STEP_THREADS),
-                           lds_bytes, s, *D0, c_begin);
-    else
-        hipLaunchKernelGGL(k_tran_step_groups, dim3((unsigned)n_step_blk), dim3(STEP_THREADS),
-                           lds_bytes, s, Ds, step_blk);
+    const int ns = D0 ? c_end - c_begin : n_step_blk;
+    /* four wavefronts a circuit while they are all resident (two such
+     * workgroups fit a compute unit's registers: 2 x 256), else one, of which
+     * eight fit.  Adders of 16 bits, ms with one / four: 64 circuits 127 / 97,
+     * 512 231 / 204; halves of 300 189 / 171, of 600 317 / 313, of 768 390 /
+     * 406, of 1024 615 / 660; a 101-stage ring alone 32.0 / 25.6 */
+    const bool wide = ns <= 512;
+    const dim3 g((unsigned)ns), wg(wide ? STEP_WIDE : ONE_WAVE);
+    if (D0 && wide) hipLaunchKernelGGL(k_tran_step<true>, g, wg, lds_bytes, s, *D0, c_begin);
+    else if (D0) hipLaunchKernelGGL(k_tran_step<false>, g, wg, lds_bytes, s, *D0, c_begin);
+    else if (wide) hipLaunchKernelGGL(k_tran_step_groups<true>, g, wg, lds_bytes, s, Ds, step_blk);
+    else hipLaunchKernelGGL(k_tran_step_groups<false>, g, wg, lds_bytes, s, Ds, step_blk);
     NGMI_HIP(hipGetLastError());
     if (ev) NGMI_HIP(hipEventRecord(ev[2], s));
     return NGMI_OK;

@@ -246,6 +246,19 @@ struct MosLaunch {
     const B4Tab *tabs = nullptr;
 };
 
+/* LU and substitution program records: PROG_INTS ints, of which the last
+ * 4 * PROG_INLINE are the inline term groups */
+constexpr int PROG_INLINE = 3;
+constexpr int PROG_INTS = 4 + 4 * PROG_INLINE;
+/* term groups a record can have beyond its inline ones */
+constexpr int PROG_EXTRA = 3;
+/* entries with more terms run as partial sums over several lanes */
+constexpr int SPLIT_TERMS = 4 * (PROG_INLINE + PROG_EXTRA);
+/* record kinds (bits 20-21 of the first int): a plain entry, a partial sum
+ * of one chunk of a long entry's terms (into a partial slot), and the
+ * combine that adds a long entry's partial sums */
+constexpr int PROG_PLAIN = 0, PROG_PARTIAL = 1, PROG_COMBINE = 2;
+
 }  // namespace ngmi
 
 #endif

@@ -174,3 +174,32 @@ def test_gather_assembly_matches_ordered_sum():
     ref = np.zeros(nnz)
     np.add.at(ref, e2z, src)
     assert np.array_equal(d_ax.cpu().numpy(), ref)
+
+
+# the three forms of the device table: tiles run once per record in them
+# (one record; a few in the same tiles; a last tile of one device), a record
+# a lane (many tiles, each with every record), a column per field (no two
+# devices alike)
+@pytest.mark.parametrize('n,geometries,spread', [(1, 1, False), (65, 1, False), (777, 7, True), (777, 7, False),
+                                                 (25601, 8, True), (129, 129, True)])
+def test_table_forms(n, geometries, spread):
+    print('case: %d devices of %d geometries, %s' % (n, geometries, 'interleaved' if spread else 'in runs'), flush=True)
+    rng = np.random.default_rng(n + geometries)
+    rec = np.arange(n) % geometries if spread else np.arange(n) * geometries // n
+    model_idx = (rec % 2).astype(np.int32)
+    params = {'l': np.exp(rng.uniform(np.log(45e-9), np.log(1e-6), geometries))[rec],
+              'w': np.exp(rng.uniform(np.log(100e-9), np.log(10e-6), geometries))[rec],
+              'ad': rng.uniform(0, 1e-12, geometries)[rec], 'as': rng.uniform(0, 1e-12, geometries)[rec],
+              'delvto': rng.normal(0, 0.03, n)}
+    models = [workloads.BASE_NMOS, workloads.BASE_PMOS]
+    g, o = GpuEval(models, model_idx, params), OracleBatch(models, model_idx, params)
+    sign = np.where(model_idx == 0, 1.0, -1.0)
+    vterm = sign * np.array([rng.uniform(0, 1.2, n), rng.uniform(0, 1.2, n), np.zeros(n), rng.uniform(-0.4, 0, n)])
+    gst = [np.zeros((29, n)) for _ in range(3)]
+    ost = [s.copy() for s in gst]
+    h = workloads.H_STEP
+    kw = dict(ag=(1 / h, -1 / h, 0, 0, 0, 0, 0), order=1)
+    for mode in (ngmi.MODETRAN | ngmi.MODEINITTRAN, ngmi.MODETRAN | ngmi.MODEINITFLOAT):
+        gout = g.load(mode, vterm, gst, **kw)
+        os_, or_, onc = o.load(mode, vterm, ost, **kw)
+        _check_all(gout, gst, o, o.cache, os_, or_, onc, ost)

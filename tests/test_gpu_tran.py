@@ -265,3 +265,31 @@ def test_operating_point_stepping():
             ora = _oracle(d, tstop)
             assert eng[2]['iterations'] == ora[2]['iterations'], (eng[2], ora[2])
             _compare('%s-%s' % (tag, how), eng, ora, d['nnodes'])
+
+
+@pytest.mark.parametrize('name,count,klu', [('ring3', 513, False), ('ring45', 1040, False), ('adder1', 1025, False),
+                                            ('adder5', 513, True)])
+def test_step_widths(name, count, klu):
+    """A circuit alone (its step by four wavefronts) and as one of more than
+    two to a compute unit (by one): the same sums in the same order, so the
+    waveforms are equal bit for bit.  adder5 on KLU's order, whose solve runs
+    block by block; its supply rows are partial sums and combines."""
+    print('case: %s alone and %d times, klu order %s' % (name, count, klu), flush=True)
+    desc = (workloads.ring_oscillator(stages=int(name[4:])) if name.startswith('ring')
+            else workloads.mc_adder(7, bits=int(name[5:])))
+    tstop = 0.15e-9 if name.startswith('ring') else 1.05e-9
+
+    def run(n):
+        circ = [ngmi.Circuit(desc) for _ in range(n)]
+        for c in circ:
+            if klu:
+                c.use_klu_order()
+        b = ngmi.Batch(circ, max_points=4096)
+        rc, _ = b.tran(desc['tstep'], tstop)
+        assert rc == 0, ngmi.last_error()
+        return [b.waveform(k, b.info()['unknowns']) for k in (0, n // 2, n - 1)]
+
+    alone = run(1)[0]
+    assert len(alone[0]) > 5
+    for t, x in run(count):
+        assert np.array_equal(t, alone[0]) and np.array_equal(x, alone[1])
