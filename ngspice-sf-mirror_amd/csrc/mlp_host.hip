@@ -41,15 +41,16 @@ struct ngmi_mlp {
     float *w = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;   /* NPARAM each */
     unsigned short *wb = nullptr, *wbt = nullptr;                   /* BF16 copy; W2, W3 transposed */
     int cap = 0;                                                    /* training rows allocated */
-    unsigned short *xo = nullptr, *h1 = nullptr, *h2 = nullptr, *dz1 = nullptr, *dz2 = nullptr, *dz3 = nullptr;
-    float *y = nullptr, *cols = nullptr, *dw = nullptr;
+    unsigned short *xo = nullptr, *h1 = nullptr, *h2 = nullptr, *h3 = nullptr;
+    unsigned short *dz1 = nullptr, *dz2 = nullptr, *dz3 = nullptr;
+    float *df1 = nullptr, *df2 = nullptr, *df3 = nullptr, *y = nullptr, *dy = nullptr, *cols = nullptr;
     int64_t step = 0;
     /* inference-only buffers (BF16 activations, ping-pong) */
     int icap = 0;
     unsigned short *ixb = nullptr, *ia = nullptr, *ib = nullptr;
     ~ngmi_mlp()
     {
-        void *ps[] = {w, g, m, v, wb, wbt, xo, h1, h2, dz1, dz2, dz3, y, cols, dw, ixb, ia, ib};
+        void *ps[] = {w, g, m, v, wb, wbt, xo, h1, h2, h3, dz1, dz2, dz3, df1, df2, df3, y, dy, cols, ixb, ia, ib};
         for (void *p : ps) (void)hipFree(p);
     }
     int ensure_infer(int rows)
@@ -67,11 +68,12 @@ struct ngmi_mlp {
     {
         if (rows <= cap) return NGMI_OK;
         cap = 0;
-        void **ps[] = {(void **)&xo, (void **)&h1, (void **)&h2, (void **)&dz1, (void **)&dz2, (void **)&dz3,
-                       (void **)&y, (void **)&cols, (void **)&dw};
-        const size_t r = (size_t)rows;
-        const size_t bytes[] = {r * IN_PAD * 2, r * H * 2, r * H * 2, r * H * 2, r * H * 2, r * H * 2, r * 4,
-                                r / 32 * TR_PART * 4, (size_t)train_splits(rows) * NPARAM * 4};
+        void **ps[] = {(void **)&xo, (void **)&h1, (void **)&h2, (void **)&h3, (void **)&dz1, (void **)&dz2,
+                       (void **)&dz3, (void **)&df1, (void **)&df2, (void **)&df3, (void **)&y, (void **)&dy,
+                       (void **)&cols};
+        const size_t r = (size_t)rows, hb = r * H * 2, hf = r * H * 4;
+        const size_t bytes[] = {r * IN_PAD * 2, hb, hb, hb, hb, hb, hb, hf, hf, hf, r * 4, r * 4,
+                                (size_t)TR_PARTS * TR_PART * 4};
         for (void **p : ps) {
             (void)hipFree(*p);
             *p = nullptr;
@@ -303,8 +305,8 @@ int ngmi_mlp_train_step(ngmi_mlp *n, const float *X, const float *target, int M,
         A.c1 = 1.0f - std::pow(A.b1, (float)n->step);
         A.c2 = 1.0f - std::pow(A.b2, (float)n->step);
     }
-    const TrainBufs B{n->w, n->g, n->m, n->v, n->wb, n->wbt, n->y, n->xo, n->h1, n->h2, n->dz1, n->dz2, n->dz3,
-                      n->cols, n->dw};
+    const TrainBufs B{n->w,  n->g,  n->m,   n->v,   n->wb,  n->wbt, n->y,   n->dy,  n->xo,  n->h1,
+                      n->h2, n->dz1, n->dz2, n->dz3, n->h3, n->df1, n->df2, n->df3, n->cols};
     if ((rc = launch_train_step(B, X, target, M, A, s))) return rc;
     if (loss_host) {
         std::vector<float> yh(M), th(M);

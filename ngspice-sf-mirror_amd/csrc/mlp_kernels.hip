@@ -9,11 +9,11 @@
  *
  * Layer-by-layer inference is k_gemm_bf16 per layer.  A training step is
  * three launches: k_train_rows (forward and backward of a tile of rows),
- * k_train_dw (weight gradients, split over the rows) and k_train_apply
- * (their sums, and Adam).  At 4000 rows they take 22.7, 12.0 and 7.0 us, a
- * step 60 us from call to call; as 24 launches, a layer's product, SiLU
- * derivative and column sums each their own and the weight gradients 64
- * waves with all 4000 rows in series, it was 471 us.
+ * k_train_dw (weight gradients and the parts of the column sums) and
+ * k_train_apply (the column sums, and Adam).  At 4000 rows they take 24.5,
+ * 14.5 and 5.1 us; as 24 launches, a layer's product, SiLU derivative and
+ * column sums each their own and the weight gradients 64 waves that waited
+ * for every load, a step was 471 us.
  *
  * Inference inside the transient uses k_guess_net instead: one kernel from
  * the feature rows to the nodes' starting values, with the weights held in
@@ -273,13 +273,13 @@ __device__ __forceinline__ void tr_put(const unsigned short (&h)[16], unsigned s
     }
 }
 
-/* the sum over the tile's 32 rows of a column, both halves of the wave */
-__device__ __forceinline__ float tr_colsum(const float (&g)[16])
+/* this wave's tile of pre-activation gradients, FP32 by rows (the column
+ * sums' operand) */
+__device__ __forceinline__ void tr_rows(const float (&g)[16], float *__restrict__ out, int64_t i0, int j, int l)
 {
-    float s = 0.0f;
+    float *p = out + (i0 + (l >> 5) * 4) * MLP_HID + j;
 #pragma unroll
-    for (int v = 0; v < 16; v++) s += g[v];
-    return s + __shfl_xor(s, 32);
+    for (int v = 0; v < 16; v++) p[((v >> 2) * 8 + (v & 3)) * MLP_HID] = g[v];
 }
 
 /* dH times the derivative of SiLU at z */
@@ -293,21 +293,18 @@ __device__ __forceinline__ float silu_back(float dh, float z)
  * Forward and backward of 32 rows a workgroup: the rows' gradients need
  * nothing of the other rows, so pre-activations stay in registers (the wave
  * that forms a layer's columns also forms their gradients) and activations
- * and gradients go from layer to layer through LDS.  Out come y, the weight
- * gradients' operands in octets of rows, and the tile's column sums (part:
- * b1, b2, b3, w4, b4).  The matrix-core steps and the element-wise code are
- * those of the inference kernels; rows from M on have zero gradients.  wbt:
- * W2 and W3 transposed, so that both directions load octets.  Each layer's
- * weights load during the layer before.  Bound by that chain of seven
- * barriers and by 530 KB of weights from L2 for every workgroup: 22.7 us at
- * 4000 rows, where 125 workgroups leave half of the CUs idle.
+ * and gradients go from layer to layer through LDS.  Out come y and dy, the
+ * weight gradients' operands in octets of rows, and by rows the operands of
+ * the column sums (h3, and the gradients in FP32).  The matrix-core steps and
+ * the element-wise code are those of the inference kernels; rows from M on
+ * have zero gradients.  wbt: W2 and W3 transposed, so that both directions
+ * load octets.  Each layer's weights load during the layer before.  Bound by
+ * that chain of seven barriers and by 530 KB of weights from L2 for every
+ * workgroup: 24.5 us at 4000 rows, where 125 workgroups leave half of the
+ * CUs idle.
  */
 __global__ void __launch_bounds__(GN_THREADS)
-k_train_rows(const float *__restrict__ X, const float *__restrict__ target, int M, const unsigned short *__restrict__ wb,
-             const unsigned short *__restrict__ wbt, const float *__restrict__ wf, float *__restrict__ yout,
-             unsigned short *__restrict__ xo, unsigned short *__restrict__ h1o, unsigned short *__restrict__ h2o,
-             unsigned short *__restrict__ dz1o, unsigned short *__restrict__ dz2o, unsigned short *__restrict__ dz3o,
-             float *__restrict__ part)
+k_train_rows(const float *__restrict__ X, const float *__restrict__ target, int M, TrainBufs B)
 {
     __shared__ __align__(16) unsigned short xs[32 * GN_XLD];
     __shared__ __align__(16) unsigned short ha[32 * GN_HLD];
@@ -317,15 +314,16 @@ k_train_rows(const float *__restrict__ X, const float *__restrict__ target, int 
     __shared__ float dys[32];
     const int tid = threadIdx.x, l = tid & 63, j = (tid >> 6) * 32 + (l & 31), r4 = (l >> 5) * 4;
     const int64_t i0 = (int64_t)blockIdx.x * 32;
-    float *pt = part + (int64_t)blockIdx.x * TR_PART;
+    const unsigned short *__restrict__ wb = B.wb, *__restrict__ wbt = B.wbt;
+    const float *__restrict__ wf = B.w;
     bf16x8 wa[MLP_HID / 16], wc[MLP_HID / 16], w1[MLP_IN_PAD / 16];
     {
         const int rr = tid >> 4, cc = tid & 15;
         const unsigned short v = f2bf(i0 + rr < M ? X[(i0 + rr) * MLP_IN + cc] : 0.0f);
         xs[rr * GN_XLD + cc] = v;
         xs[rr * GN_XLD + MLP_IN + cc] = 0;
-        xo[oct_at(i0 + rr, MLP_IN_PAD, cc)] = v;
-        xo[oct_at(i0 + rr, MLP_IN_PAD, MLP_IN + cc)] = 0;
+        B.x[oct_at(i0 + rr, MLP_IN_PAD, cc)] = v;
+        B.x[oct_at(i0 + rr, MLP_IN_PAD, MLP_IN + cc)] = 0;
     }
     if (tid < MLP_HID) w4s[tid] = bf2f(wb[MLP_OFF_W4 + tid]);
     tr_weights(w1, wb + MLP_OFF_W1, MLP_IN_PAD, j, l);
@@ -340,7 +338,7 @@ k_train_rows(const float *__restrict__ X, const float *__restrict__ target, int 
     z1 = tr_product(xs, GN_XLD, w1, z1, l);
 #pragma unroll
     for (int v = 0; v < 16; v++) h[v] = hidden_out(z1[v]);
-    tr_put(h, ha, h1o, i0, j, l);
+    tr_put(h, ha, B.h1, i0, j, l);
     tr_weights(wc, wb + MLP_OFF_W3, MLP_HID, j, l);
     __syncthreads();
 #pragma unroll
@@ -348,7 +346,7 @@ k_train_rows(const float *__restrict__ X, const float *__restrict__ target, int 
     z2 = tr_product(ha, GN_HLD, wa, z2, l);
 #pragma unroll
     for (int v = 0; v < 16; v++) h[v] = hidden_out(z2[v]);
-    tr_put(h, hb, h2o, i0, j, l);
+    tr_put(h, hb, B.h2, i0, j, l);
     tr_weights(wa, wbt + MLP_SZ_W2, MLP_HID, j, l);   /* W3 transposed */
     __syncthreads();
 #pragma unroll
@@ -357,7 +355,9 @@ k_train_rows(const float *__restrict__ X, const float *__restrict__ target, int 
 #pragma unroll
     for (int v = 0; v < 16; v++) {
         h[v] = hidden_out(z3[v]);
-        ha[((v >> 2) * 8 + r4 + (v & 3)) * GN_HLD + j] = h[v];
+        const int i = (v >> 2) * 8 + r4 + (v & 3);
+        ha[i * GN_HLD + j] = h[v];
+        B.h3[(i0 + i) * MLP_HID + j] = h[v];
     }
     __syncthreads();
     if (tid < 32 * GN_HEAD_BLOCKS) {
@@ -369,38 +369,28 @@ k_train_rows(const float *__restrict__ X, const float *__restrict__ target, int 
         ps[rr][cb] = p;
     }
     __syncthreads();
-    if (tid < 64) {
-        float dy = 0.0f;
-        if (tid < 32) {
-            float y = b4;
+    if (tid < 32) {
+        float y = b4, dy = 0.0f;
 #pragma unroll
-            for (int cb = 0; cb < GN_HEAD_BLOCKS; cb++) y += ps[tid][cb];
-            if (i0 + tid < M) {
-                yout[i0 + tid] = y;
-                dy = 2.0f * (y - tg) / (float)M;
-            }
-            dys[tid] = dy;
+        for (int cb = 0; cb < GN_HEAD_BLOCKS; cb++) y += ps[tid][cb];
+        if (i0 + tid < M) {
+            B.y[i0 + tid] = y;
+            dy = 2.0f * (y - tg) / (float)M;
         }
-#pragma unroll
-        for (int o = 16; o > 0; o >>= 1) dy += __shfl_xor(dy, o);
-        if (tid == 0) pt[4 * MLP_HID] = dy;
+        dys[tid] = B.dy[i0 + tid] = dy;
     }
     __syncthreads();
     float g[16];
     {
-        float u[16];
         const float w4 = w4s[j];
 #pragma unroll
         for (int v = 0; v < 16; v++) {
-            const float dy = dys[(v >> 2) * 8 + r4 + (v & 3)];
-            u[v] = dy * bf2f(h[v]);
-            g[v] = silu_back(dy * w4, z3[v]);
+            g[v] = silu_back(dys[(v >> 2) * 8 + r4 + (v & 3)] * w4, z3[v]);
             h[v] = f2bf(g[v]);
         }
-        const float su = tr_colsum(u), sg = tr_colsum(g);
-        if (l < 32) pt[3 * MLP_HID + j] = su, pt[2 * MLP_HID + j] = sg;
     }
-    tr_put(h, hb, dz3o, i0, j, l);
+    tr_rows(g, B.df3, i0, j, l);
+    tr_put(h, hb, B.dz3, i0, j, l);
     tr_weights(wc, wbt, MLP_HID, j, l);               /* W2 transposed */
     __syncthreads();
     z3 = tr_product(hb, GN_HLD, wa, f32x16{}, l);
@@ -409,11 +399,8 @@ k_train_rows(const float *__restrict__ X, const float *__restrict__ target, int 
         g[v] = silu_back(z3[v], z2[v]);
         h[v] = f2bf(g[v]);
     }
-    tr_put(h, ha, dz2o, i0, j, l);
-    {
-        const float sg = tr_colsum(g);
-        if (l < 32) pt[MLP_HID + j] = sg;
-    }
+    tr_put(h, ha, B.dz2, i0, j, l);
+    tr_rows(g, B.df2, i0, j, l);
     __syncthreads();
     z3 = tr_product(ha, GN_HLD, wc, f32x16{}, l);
 #pragma unroll
@@ -424,67 +411,127 @@ k_train_rows(const float *__restrict__ X, const float *__restrict__ target, int 
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const uint2 u = make_uint2(h[4 * q] | (unsigned)h[4 * q + 1] << 16, h[4 * q + 2] | (unsigned)h[4 * q + 3] << 16);
-        *reinterpret_cast<uint2 *>(dz1o + oct_at(i0 + 8 * q + r4, MLP_HID, j)) = u;
+        *reinterpret_cast<uint2 *>(B.dz1 + oct_at(i0 + 8 * q + r4, MLP_HID, j)) = u;
     }
-    const float sg = tr_colsum(g);
-    if (l < 32) pt[j] = sg;
+    tr_rows(g, B.df1, i0, j, l);
 }
 
-/* dW[o][i] = sum_m dZ[m][o] Hin[m][i] of the rows [y chunk, (y + 1) chunk)
- * into part y: a 64 x 64 tile (64 x 32 of W1) a wave, 2 x 2 matrix-core
- * tiles.  chunk is a multiple of 16.  A tile of 64 x 64 reads each operand 4
- * times instead of 8; 12.0 us at 4000 rows (15 parts, 540 waves), bound by the
- * loads' latency and the parts' 8.4 MB. */
-constexpr int DW_STEPS = 8;   /* matrix-core steps loaded at a time */
+/* dW[o][i] = sum_m dZ[m][o] Hin[m][i], a 32 x 32 tile a wave, all rows in
+ * one chain of matrix-core steps: the order of the sum is part of the result
+ * (parts added up afterwards give other last bits, which Adam's g / |g| turns
+ * into other weights).  The chain is 32 cycles a step, 3.4 us of 4000 rows;
+ * the loads are what takes longer, so a batch of DW_STEPS is in flight while
+ * the one before it is multiplied. */
+constexpr int DW_STEPS = 16;
 
-template <int NI>
+struct DwBatch {
+    bf16x8 a[DW_STEPS], b[DW_STEPS];
+};
+
+__device__ __forceinline__ void dw_load(DwBatch &t, const unsigned short *pa, const unsigned short *pb, int kin, int m,
+                                        int rows)
+{
+#pragma unroll
+    for (int q = 0; q < DW_STEPS; q++) {
+        const int64_t mm = min(m + 16 * q, rows - 16);
+        t.a[q] = *reinterpret_cast<const bf16x8 *>(pa + mm * MLP_HID);
+        t.b[q] = *reinterpret_cast<const bf16x8 *>(pb + mm * kin);
+    }
+}
+
 __device__ __forceinline__ void dw_tile(const unsigned short *__restrict__ dz, const unsigned short *__restrict__ hin,
-                                        int kin, int o0, int c0, int m0, int m1, float *__restrict__ out, int l)
+                                        int kin, int o0, int c0, int rows, float *__restrict__ out, int l)
 {
     const int r = l & 31, half = l >> 5;
-    const unsigned short *pa = dz + ((int64_t)(m0 / 8 + half) * MLP_HID + o0 + r) * 8;
-    const unsigned short *pb = hin + ((int64_t)(m0 / 8 + half) * kin + c0 + r) * 8;
-    f32x16 acc[2][NI] = {};
-    for (int m = m0; m < m1; m += 16 * DW_STEPS) {   /* a batch's loads in flight together */
-        bf16x8 a[DW_STEPS][2], b[DW_STEPS][NI];
+    const unsigned short *pa = dz + ((int64_t)half * MLP_HID + o0 + r) * 8;
+    const unsigned short *pb = hin + ((int64_t)half * kin + c0 + r) * 8;
+    f32x16 acc = {};
+    constexpr int BR = 16 * DW_STEPS;
+    DwBatch t, u;
+    dw_load(t, pa, pb, kin, 0, rows);
+    int m = 0;
+    for (; m + 2 * BR <= rows; m += 2 * BR) {
+        dw_load(u, pa, pb, kin, m + BR, rows);
 #pragma unroll
-        for (int q = 0; q < DW_STEPS; q++) {
-            const int mm = min(m + 16 * q, m1 - 16) - m0;
+        for (int q = 0; q < DW_STEPS; q++) acc = mfma16(t.a[q], t.b[q], acc);
+        dw_load(t, pa, pb, kin, m + 2 * BR, rows);
 #pragma unroll
-            for (int t = 0; t < 2; t++) a[q][t] = *reinterpret_cast<const bf16x8 *>(pa + (int64_t)mm * MLP_HID + 256 * t);
-#pragma unroll
-            for (int t = 0; t < NI; t++) b[q][t] = *reinterpret_cast<const bf16x8 *>(pb + (int64_t)mm * kin + 256 * t);
-        }
-#pragma unroll
-        for (int q = 0; q < DW_STEPS; q++)
-            if (m + 16 * q < m1) {
-#pragma unroll
-                for (int t = 0; t < 2; t++)
-#pragma unroll
-                    for (int u = 0; u < NI; u++) acc[t][u] = mfma16(a[q][t], b[q][u], acc[t][u]);
-            }
+        for (int q = 0; q < DW_STEPS; q++) acc = mfma16(u.a[q], u.b[q], acc);
     }
+    /* under two batches are left, the first in t */
+    if (m + BR < rows) dw_load(u, pa, pb, kin, m + BR, rows);
 #pragma unroll
-    for (int t = 0; t < 2; t++)
+    for (int q = 0; q < DW_STEPS; q++)
+        if (m + 16 * q < rows) acc = mfma16(t.a[q], t.b[q], acc);
+    m += BR;
 #pragma unroll
-        for (int u = 0; u < NI; u++)
+    for (int q = 0; q < DW_STEPS; q++)
+        if (m + 16 * q < rows) acc = mfma16(u.a[q], u.b[q], acc);
 #pragma unroll
-            for (int v = 0; v < 16; v++)
-                out[(int64_t)(o0 + 32 * t + (v >> 2) * 8 + half * 4 + (v & 3)) * kin + c0 + 32 * u + r] = acc[t][u][v];
+    for (int v = 0; v < 16; v++)
+        out[(int64_t)(o0 + (v >> 2) * 8 + half * 4 + (v & 3)) * kin + c0 + r] = acc[v];
 }
 
-__global__ void __launch_bounds__(64)
-k_train_dw(const unsigned short *__restrict__ xo, const unsigned short *__restrict__ h1o,
-           const unsigned short *__restrict__ h2o, const unsigned short *__restrict__ dz1o,
-           const unsigned short *__restrict__ dz2o, const unsigned short *__restrict__ dz3o, int rows, int chunk,
-           float *__restrict__ part)
+/* the sums of rows [i0, i1) of a column of x (times wt), four row lanes whose
+ * sums are added in order; the product is rounded before it is added */
+template <class X>
+__device__ __forceinline__ float col_part(int i0, int i1, X x)
 {
-    const int l = threadIdx.x, t = blockIdx.x, o0 = (t & 3) * 64, c0 = (t >> 2 & 3) * 64;
-    const int m0 = blockIdx.y * chunk, m1 = min(rows, m0 + chunk);
-    float *out = part + (int64_t)blockIdx.y * MLP_NPARAM;
-    if (t < 16) dw_tile<2>(dz2o, h1o, MLP_HID, o0, c0, m0, m1, out + MLP_OFF_W2, l);
-    else if (t < 32) dw_tile<2>(dz3o, h2o, MLP_HID, o0, c0, m0, m1, out + MLP_OFF_W3, l);
-    else dw_tile<1>(dz1o, xo, MLP_IN_PAD, o0, 0, m0, m1, out + MLP_OFF_W1, l);
+#pragma clang fp contract(off)
+    constexpr int U = 8;
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    int i = i0;
+    for (; i + 4 * U <= i1; i += 4 * U) {
+        float t[4 * U];
+#pragma unroll
+        for (int q = 0; q < 4 * U; q++) t[q] = x(i + q);
+#pragma unroll
+        for (int q = 0; q < 4 * U; q++) s[q & 3] += t[q];
+    }
+    for (; i < i1; i += 4)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (i + q < i1) s[q] += x(i + q);
+    return ((s[0] + s[1]) + s[2]) + s[3];
+}
+
+/* The weight gradients, a tile a workgroup of one wavefront, and beside them
+ * the column sums (bias gradients of the FP32 gradients, w4's and b4's), a
+ * part of the rows and 64 columns a workgroup, parts in cols.  14.5 us at
+ * 4000 rows. */
+constexpr int DW_W2 = (MLP_HID / 32) * (MLP_HID / 32), DW_TILES = 2 * DW_W2 + MLP_HID / 32;
+
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1)))
+k_train_dw(TrainBufs B, int rows, int parts, int chunk)
+{
+    const int l = threadIdx.x;
+    int t = blockIdx.x;
+    if (t < DW_TILES) {
+        const int o0 = (t & 7) * 32, c0 = (t >> 3 & 7) * 32;
+        if (t < DW_W2) dw_tile(B.dz2, B.h1, MLP_HID, o0, c0, rows, B.g + MLP_OFF_W2, l);
+        else if (t < 2 * DW_W2) dw_tile(B.dz3, B.h2, MLP_HID, o0, c0, rows, B.g + MLP_OFF_W3, l);
+        else dw_tile(B.dz1, B.x, MLP_IN_PAD, o0, 0, rows, B.g + MLP_OFF_W1, l);
+        return;
+    }
+    t -= DW_TILES;
+    const int p = t % parts, i0 = p * chunk, i1 = min(rows, i0 + chunk);
+    t /= parts;
+    const int k = t >> 2, j = (t & 3) * 64 + l;   /* vector, column */
+    float *out = B.cols + (int64_t)p * TR_PART;
+    if (k < 3) {
+        const float *__restrict__ f = (k == 0 ? B.df1 : k == 1 ? B.df2 : B.df3) + j;
+        out[k * MLP_HID + j] = col_part(i0, i1, [&](int i) { return f[(int64_t)i * MLP_HID]; });
+    } else if (k == 3) {
+        const float *__restrict__ dy = B.dy;
+        const unsigned short *__restrict__ h = B.h3 + j;
+        out[3 * MLP_HID + j] = col_part(i0, i1, [&](int i) {
+#pragma clang fp contract(off)
+            return dy[i] * bf2f(h[(int64_t)i * MLP_HID]);
+        });
+    } else if (l == 0) {
+        const float *__restrict__ dy = B.dy;
+        out[4 * MLP_HID] = col_part(i0, i1, [&](int i) { return dy[i]; });
+    }
 }
 
 /* Adam on an FP32 master weight */
@@ -498,69 +545,50 @@ __device__ __forceinline__ float adam(float *__restrict__ w, float *__restrict__
     return *w = *w - A.lr * (mi / A.c1) / (sqrtf(vi / A.c2) + A.eps);
 }
 
-/* The gradients from their parts, in order, and with lr > 0 an Adam step on
- * them, refreshing the BF16 copies.  A workgroup takes 16 x 16 weights (the
- * transposed copy written through LDS), or, after the weights, 16 of the
- * column-summed parameters with 16 threads each. */
+/* The column sums from their parts, in order, and with lr > 0 an Adam step on
+ * all gradients, refreshing the BF16 copies.  A workgroup takes 256 of the
+ * column-summed parameters, or 16 x 16 weights (the transposed copy written
+ * through LDS); the weights' are launched only with lr > 0.  5.1 us. */
 constexpr int TR_TILES_W1 = (int)(MLP_SZ_W1 / 256), TR_TILES_W2 = (int)(MLP_SZ_W2 / 256);
+constexpr int TR_WG_COLS = (TR_COLS + 255) / 256;
 __global__ void __launch_bounds__(256)
-k_train_apply(const float *__restrict__ dw, int S, const float *__restrict__ cols, int tiles, float *__restrict__ g,
-              float *__restrict__ w, unsigned short *__restrict__ wb, unsigned short *__restrict__ wbt,
-              float *__restrict__ m, float *__restrict__ v, AdamStep A)
+k_train_apply(TrainBufs B, int parts, AdamStep A)
 {
     const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
     int b = blockIdx.x;
-    if (b < TR_TILES_W1 + 2 * TR_TILES_W2) {
-        __shared__ unsigned short T[16][17];
-        int kin = MLP_IN_PAD;
-        int64_t off = MLP_OFF_W1, toff = -1;
-        if (b >= TR_TILES_W1) {
-            b -= TR_TILES_W1;
-            const bool w3 = b >= TR_TILES_W2;
-            kin = MLP_HID;
-            off = w3 ? MLP_OFF_W3 : MLP_OFF_W2;
-            toff = w3 ? MLP_SZ_W2 : 0;
-            if (w3) b -= TR_TILES_W2;
-        }
-        const int o0 = b / (kin / 16) * 16, c0 = b % (kin / 16) * 16;
-        const int64_t i = off + (int64_t)(o0 + ty) * kin + c0 + tx;
+    if (b < TR_WG_COLS) {
+        const int c = b * 256 + tid;
+        if (c >= TR_COLS) return;
         float s = 0.0f;
-        int p = 0;
-        for (; p + 8 <= S; p += 8) {
-            float t[8];
-#pragma unroll
-            for (int q = 0; q < 8; q++) t[q] = dw[(p + q) * MLP_NPARAM + i];
-#pragma unroll
-            for (int q = 0; q < 8; q++) s += t[q];
-        }
-        for (; p < S; p++) s += dw[p * MLP_NPARAM + i];
-        g[i] = s;
-        if (!(A.lr > 0)) return;
-        const unsigned short nb = f2bf(adam(w + i, m + i, v + i, s, A));
-        wb[i] = nb;
-        if (toff < 0) return;
-        T[ty][tx] = nb;
-        __syncthreads();
-        wbt[toff + (int64_t)(c0 + ty) * MLP_HID + o0 + tx] = T[tx][ty];
+#pragma unroll 16
+        for (int p = 0; p < parts; p++) s += B.cols[(int64_t)p * TR_PART + c];
+        const int k = c / MLP_HID;
+        const int64_t i = (k == 0 ? MLP_OFF_B1 : k == 1 ? MLP_OFF_B2 : k == 2 ? MLP_OFF_B3 : k == 3 ? MLP_OFF_W4 : MLP_OFF_B4) +
+                          c % MLP_HID;
+        B.g[i] = s;
+        if (A.lr > 0) B.wb[i] = f2bf(adam(B.w + i, B.m + i, B.v + i, s, A));
         return;
     }
-    b -= TR_TILES_W1 + 2 * TR_TILES_W2;
-    __shared__ float R[16][17];
-    const int c = b * 16 + tx;
-    float s = 0.0f;
-#pragma unroll 8
-    for (int p = ty; p < tiles; p += 16) s += cols[(int64_t)p * TR_PART + min(c, TR_COLS - 1)];
-    R[ty][tx] = s;
+    b -= TR_WG_COLS;
+    __shared__ unsigned short T[16][17];
+    int kin = MLP_IN_PAD;
+    int64_t off = MLP_OFF_W1, toff = -1;
+    if (b >= TR_TILES_W1) {
+        b -= TR_TILES_W1;
+        const bool w3 = b >= TR_TILES_W2;
+        kin = MLP_HID;
+        off = w3 ? MLP_OFF_W3 : MLP_OFF_W2;
+        toff = w3 ? MLP_SZ_W2 : 0;
+        if (w3) b -= TR_TILES_W2;
+    }
+    const int o0 = b / (kin / 16) * 16, c0 = b % (kin / 16) * 16;
+    const int64_t i = off + (int64_t)(o0 + ty) * kin + c0 + tx;
+    const unsigned short nb = f2bf(adam(B.w + i, B.m + i, B.v + i, B.g[i], A));
+    B.wb[i] = nb;
+    if (toff < 0) return;
+    T[ty][tx] = nb;
     __syncthreads();
-    if (ty != 0 || c >= TR_COLS) return;
-    s = 0.0f;
-#pragma unroll
-    for (int q = 0; q < 16; q++) s += R[q][tx];
-    const int k = c / MLP_HID;
-    const int64_t i = (k == 0 ? MLP_OFF_B1 : k == 1 ? MLP_OFF_B2 : k == 2 ? MLP_OFF_B3 : k == 3 ? MLP_OFF_W4 : MLP_OFF_B4) +
-                      c % MLP_HID;
-    g[i] = s;
-    if (A.lr > 0) wb[i] = f2bf(adam(w + i, m + i, v + i, s, A));
+    B.wbt[toff + (int64_t)(c0 + ty) * MLP_HID + o0 + tx] = T[tx][ty];
 }
 
 /* W2 and W3 of wb transposed into wbt */
@@ -573,17 +601,13 @@ __global__ void k_train_transpose(const unsigned short *__restrict__ wb, unsigne
 
 int launch_train_step(const TrainBufs &B, const float *X, const float *target, int M, const AdamStep &A, hipStream_t s)
 {
-    const int rows = (M + 31) / 32 * 32, tiles = rows / 32;
-    hipLaunchKernelGGL(k_train_rows, dim3((unsigned)tiles), dim3(GN_THREADS), 0, s, X, target, M, B.wb, B.wbt, B.w, B.y,
-                       B.x, B.h1, B.h2, B.dz1, B.dz2, B.dz3, B.cols);
+    const int rows = (M + 31) / 32 * 32, parts = train_parts(rows), chunk = (rows + parts - 1) / parts;
+    hipLaunchKernelGGL(k_train_rows, dim3((unsigned)(rows / 32)), dim3(GN_THREADS), 0, s, X, target, M, B);
     NGMI_HIP(hipGetLastError());
-    const int S = train_splits(rows), chunk = ((rows / 16 + S - 1) / S) * 16;
-    hipLaunchKernelGGL(k_train_dw, dim3(36, (unsigned)S), dim3(64), 0, s, B.x, B.h1, B.h2, B.dz1, B.dz2, B.dz3, rows,
-                       chunk, B.dw);
+    hipLaunchKernelGGL(k_train_dw, dim3((unsigned)(DW_TILES + (4 * 4 + 1) * parts)), dim3(64), 0, s, B, rows, parts, chunk);
     NGMI_HIP(hipGetLastError());
-    const unsigned apply = TR_TILES_W1 + 2 * TR_TILES_W2 + (TR_COLS + 15) / 16;
-    hipLaunchKernelGGL(k_train_apply, dim3(apply), dim3(256), 0, s, B.dw, S, B.cols, tiles, B.g, B.w, B.wb, B.wbt, B.m,
-                       B.v, A);
+    const unsigned apply = TR_WG_COLS + (A.lr > 0 ? TR_TILES_W1 + 2 * TR_TILES_W2 : 0);
+    hipLaunchKernelGGL(k_train_apply, dim3(apply), dim3(256), 0, s, B, parts, A);
     NGMI_HIP(hipGetLastError());
     return NGMI_OK;
 }

@@ -41,29 +41,29 @@ __device__ __forceinline__ unsigned short hidden_out(float z) { return f2bf(silu
 
 /* ---- training ---- */
 
-/* a row tile's column sums: b1, b2, b3, w4 (256 each), b4; padded to whole
- * 64-byte lines */
+/* one part of the rows' column sums: b1, b2, b3, w4 (256 each), b4; padded to
+ * whole 64-byte lines */
 constexpr int TR_COLS = 4 * MLP_HID + 1, TR_PART = (TR_COLS + 15) / 16 * 16;
 
-/* parts the weight gradients' rows are split in: 256 rows each, a chain of 16
- * matrix-core steps, until there are 32 parts (1152 waves; more would cost
- * more in writing and summing parts, 0.56 MB each, than a shorter chain
- * gains) */
-inline int train_splits(int rows) { return rows < 512 ? 1 : rows / 256 > 32 ? 32 : rows / 256; }
+/* parts the column sums' rows are split in: 128 rows each until there are 64.
+ * The split is part of the gradients' last bits. */
+constexpr int TR_PARTS = 64;
+inline int train_parts(int rows) { return rows > 128 * TR_PARTS ? TR_PARTS : (rows + 127) / 128; }
 
 struct AdamStep {
     float lr, b1, b2, eps, c1, c2;   /* lr <= 0: gradients only */
 };
 
 /* device buffers of a training step: parameters, their BF16 copy and W2, W3
- * transposed; outputs y; BF16 inputs, activations and gradients in octets of
- * rows; column sums by row tile; weight gradients by part */
+ * transposed; outputs y and their gradients dy; BF16 inputs, activations and
+ * gradients in octets of rows; by rows h3 and the gradients in FP32; column
+ * sums by part */
 struct TrainBufs {
     float *w, *g, *m, *v;
     unsigned short *wb, *wbt;
-    float *y;
-    unsigned short *x, *h1, *h2, *dz1, *dz2, *dz3;
-    float *cols, *dw;
+    float *y, *dy;
+    unsigned short *x, *h1, *h2, *dz1, *dz2, *dz3, *h3;
+    float *df1, *df2, *df3, *cols;
 };
 
 }  // namespace ngmi

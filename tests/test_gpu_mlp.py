@@ -8,6 +8,10 @@ order on the matrix cores and the BF16 rounding of the backward operands
 every gradient block within 2e-2 of its largest magnitude (BF16 has an
 8-bit mantissa, 2^-8 = 3.9e-3 relative).
 """
+import hashlib
+import json
+import os
+
 import numpy as np
 import pytest
 
@@ -93,10 +97,10 @@ def test_training_reduces_loss():
 
 @pytest.mark.parametrize('M', [1, 31, 32, 33, 511, 512, 545, 8240])
 def test_gradients_after_a_step(M):
-    """Row tiles' ends, one to 32 parts of the rows (8240: a last part with
-    none), and the weights' copies after Adam: the gradients of a second step
-    on the updated parameters.  Bar: the backward operands' BF16 rounding, as
-    above; a sum over rows split in parts only shortens its chains."""
+    """Row tiles' ends, batches of rows in the weight gradients' chain, one to
+    64 parts of the column sums, and the weights' copies after Adam: the
+    gradients of a second step on the updated parameters.  Bar: the backward
+    operands' BF16 rounding, as above."""
     print('case: guess network two steps M=%d' % M, flush=True)
     rng = np.random.default_rng(100 + M)
     net = ngmi.GuessNet(seed=9)
@@ -119,3 +123,26 @@ def test_gradients_after_a_step(M):
         err = np.abs(gg - gr).max() / max(np.abs(gr).max(), 1e-30)
         print('grad %-3s scaled err %.2e' % (name, err), flush=True)
         assert err < 2e-2, name
+
+
+with open(os.path.join(os.path.dirname(__file__), 'golden', 'guess_training_bits.json')) as f:
+    TRAINING_BITS = json.load(f)
+
+
+@pytest.mark.parametrize('M', [int(k) for k in TRAINING_BITS if k != '_'])
+def test_training_bits(M):
+    """A network trained again from the same rows is the same network: the
+    order of every sum over the rows is fixed, so parameters and gradients
+    are those of the recorded training bit for bit (and with them the
+    learned transient's starting values)."""
+    print('case: guess network training bits M=%d' % M, flush=True)
+    rng = np.random.default_rng(700 + M)
+    net = ngmi.GuessNet(seed=5)
+    X = rng.normal(size=(M, 16)).astype(np.float32)
+    T = rng.normal(scale=0.1, size=M).astype(np.float32)
+    dX, dT = torch.from_numpy(X).cuda(), torch.from_numpy(T).cuda()
+    for lr in (0.0, 1e-3, 1e-3, 1e-3):
+        net.train_step(dX.data_ptr(), dT.data_ptr(), M, lr, want_loss=False)
+    p, g = net.params(), net.params(grads=True)
+    assert hashlib.sha256(p.tobytes()).hexdigest() == TRAINING_BITS[str(M)]['params']
+    assert hashlib.sha256(g.tobytes()).hexdigest() == TRAINING_BITS[str(M)]['grads']
