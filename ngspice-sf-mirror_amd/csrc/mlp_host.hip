@@ -35,6 +35,32 @@ constexpr int H = MLP_HID;
 constexpr int64_t OFF_W1 = MLP_OFF_W1, OFF_B1 = MLP_OFF_B1, OFF_W2 = MLP_OFF_W2, OFF_B2 = MLP_OFF_B2,
                   OFF_W3 = MLP_OFF_W3, OFF_B3 = MLP_OFF_B3, OFF_W4 = MLP_OFF_W4, OFF_B4 = MLP_OFF_B4,
                   NPARAM = MLP_NPARAM;
+
+/* work buffers of the layer-by-layer inference: packed input and two
+ * activation buffers (ping-pong), BF16 */
+struct InferBufs {
+    int cap = 0;   /* rows */
+    unsigned short *xb = nullptr, *a = nullptr, *b = nullptr;
+    ~InferBufs() { release(); }
+    void release()
+    {
+        for (unsigned short **p : {&xb, &a, &b}) {
+            (void)hipFree(*p);
+            *p = nullptr;
+        }
+        cap = 0;
+    }
+    int ensure(int rows)
+    {
+        if (rows <= cap) return NGMI_OK;
+        release();
+        NGMI_HIP(hipMalloc(&xb, (size_t)rows * IN_PAD * 2));
+        NGMI_HIP(hipMalloc(&a, (size_t)rows * H * 2));
+        NGMI_HIP(hipMalloc(&b, (size_t)rows * H * 2));
+        cap = rows;
+        return NGMI_OK;
+    }
+};
 }  // namespace
 
 struct ngmi_mlp {
@@ -45,24 +71,13 @@ struct ngmi_mlp {
     unsigned short *dz1 = nullptr, *dz2 = nullptr, *dz3 = nullptr;
     float *df1 = nullptr, *df2 = nullptr, *df3 = nullptr, *y = nullptr, *dy = nullptr, *cols = nullptr;
     int64_t step = 0;
-    /* inference-only buffers (BF16 activations, ping-pong) */
-    int icap = 0;
-    unsigned short *ixb = nullptr, *ia = nullptr, *ib = nullptr;
+    /* ngmi_mlp_forward's and the transient's: a transient keeps the pointers
+     * in its captured passes, and may run beside a forward call */
+    InferBufs fwd, guess;
     ~ngmi_mlp()
     {
-        void *ps[] = {w, g, m, v, wb, wbt, xo, h1, h2, h3, dz1, dz2, dz3, df1, df2, df3, y, dy, cols, ixb, ia, ib};
+        void *ps[] = {w, g, m, v, wb, wbt, xo, h1, h2, h3, dz1, dz2, dz3, df1, df2, df3, y, dy, cols};
         for (void *p : ps) (void)hipFree(p);
-    }
-    int ensure_infer(int rows)
-    {
-        if (rows <= icap) return NGMI_OK;
-        void *ps[] = {ixb, ia, ib};
-        for (void *p : ps) (void)hipFree(p);
-        NGMI_HIP(hipMalloc(&ixb, (size_t)rows * 32 * 2));
-        NGMI_HIP(hipMalloc(&ia, (size_t)rows * MLP_HID * 2));
-        NGMI_HIP(hipMalloc(&ib, (size_t)rows * MLP_HID * 2));
-        icap = rows;
-        return NGMI_OK;
     }
     int ensure(int rows)   /* a multiple of 32 */
     {
@@ -184,9 +199,9 @@ int mlp_forward_rows(ngmi_mlp *n, const float *X, float *y, int maxRows, const i
                      hipStream_t s)
 {
     const int Mpad = (maxRows + 31) / 32 * 32;
-    int rc = n->ensure_infer(Mpad);
+    int rc = n->guess.ensure(Mpad);
     if (rc) return rc;
-    return forward_infer(n, X, y, maxRows, Mpad, n->ixb, n->ia, n->ib, dcount, s);
+    return forward_infer(n, X, y, maxRows, Mpad, n->guess.xb, n->guess.a, n->guess.b, dcount, s);
 }
 
 /* the fused inference of the transient's guess pass: rows from count[0]
@@ -263,9 +278,9 @@ int ngmi_mlp_forward(ngmi_mlp *n, const float *X, float *y, int M, void *stream)
     if (tune_get(TUNE_GUESS_FUSED))
         return launch_guess_net(n->wb, n->w, X, nullptr, M, nullptr, nullptr, nullptr, y, nullptr, s);
     const int Mpad = (M + 31) / 32 * 32;
-    const int rc = n->ensure_infer(Mpad);
+    const int rc = n->fwd.ensure(Mpad);
     if (rc) return rc;
-    return forward_infer(n, X, y, M, Mpad, n->ixb, n->ia, n->ib, nullptr, s);
+    return forward_infer(n, X, y, M, Mpad, n->fwd.xb, n->fwd.a, n->fwd.b, nullptr, s);
 }
 
 /* ngmi_mlp_forward without allocating: the work buffers are the library's

@@ -22,6 +22,7 @@ from engine_path import ngmi, workloads
 import guess
 import os
 import sys
+import threading
 
 sys.path.insert(0, os.path.join(os.path.dirname(__file__), '..', 'oracle'))
 import pyoracle as po  # noqa: E402
@@ -179,6 +180,50 @@ def test_features_match_the_engine_bit_for_bit():
         assert np.array_equal(act_dev[keep], A_host)
         checked += len(F_host)
     assert checked > 1000
+
+
+def test_forward_beside_a_layered_transient(trained):
+    """With the network run layer by layer (guess_fused 0), forward calls on
+    another stream and thread, of more rows than the transient's and of fewer
+    (so the forward's buffers grow while the transient replays its captured
+    passes), leave a learned transient's waveforms as they are, bit for bit,
+    and get their own outputs."""
+    net = trained[0]
+    print('case: ngmi_mlp_forward beside a layered learned transient, adder seeds 0..3', flush=True)
+    rng = np.random.default_rng(8)
+    keep = ngmi.get_tune('guess_fused')
+    try:
+        ngmi.tune('guess_fused', 0)
+        b, _ = run([0, 1, 2, 3], net=net)
+        n = b.info()['unknowns']
+        alone = [b.waveform(c, n) for c in range(4)]
+        X = torch.from_numpy(rng.normal(size=(40000, 16)).astype(np.float32)).cuda()
+        sizes = (64, 1000, 8192, 40000)
+        want, out = {}, {}
+        t = threading.Thread(target=lambda: out.update(b=run([0, 1, 2, 3], net=net)[0]))
+        t.start()
+        side = torch.cuda.Stream()
+        got, k = {}, 0
+        while t.is_alive() or k < len(sizes):
+            m = sizes[k % len(sizes)]
+            got[m] = torch.zeros(m, dtype=torch.float32, device='cuda')
+            torch.cuda.current_stream().synchronize()
+            net.forward(X.data_ptr(), got[m].data_ptr(), m, stream=side.cuda_stream)
+            side.synchronize()
+            k += 1
+        t.join()
+        for m in sizes:
+            want[m] = torch.zeros(m, dtype=torch.float32, device='cuda')
+            net.forward(X.data_ptr(), want[m].data_ptr(), m)
+        torch.cuda.synchronize()
+    finally:
+        ngmi.tune('guess_fused', keep)
+    print('%d forward calls beside the transient' % k, flush=True)
+    for m in sizes:
+        assert torch.equal(got[m], want[m]), m
+    for c in range(4):
+        te, xe = out['b'].waveform(c, n)
+        assert np.array_equal(te, alone[c][0]) and np.array_equal(xe, alone[c][1])
 
 
 @pytest.mark.parametrize('seed', [0, 1])
