@@ -65,6 +65,12 @@ __device__ __forceinline__ double rdlane(double v, int lane)
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+/* div_by gives num / d, a positive zero's included */
+__device__ __forceinline__ bool div_by_ok(double num, double d)
+{
+    return div_by_divisor(d) && (div_by_dividend(num) || __double_as_longlong(num) == 0);
+}
+
 /* v of lane N of each row of 16 lanes, to the row (one v_mov_b64_dpp; every
  * lane of the wave has to be active) */
 template <int N>
@@ -811,9 +817,10 @@ __global__ void __launch_bounds__(WG) k_sp_bwd_small(SpDev d, const int *__restr
         dg[q] = S[row[q] * ns + row[q]];
         di[q] = 1.0 / dg[q];
     }
-#pragma unroll
-    for (int s = SR - 1; s >= 0; s--) {
-        if (64 * s >= ns) continue;
+    /* 64 pivots, from the last; EXACT divides, else quotients come from the
+     * pivots' reciprocals.  num takes each lane's dividend. */
+    auto pivots = [&](auto sc, auto exact, double &num) {
+        constexpr int s = sc;
         const int ke = min(ns, 64 * s + 64);
         for (int k0 = ((ke - 1) & ~7); k0 >= 64 * s; k0 -= 8) {
             double u[8][SR];
@@ -825,17 +832,35 @@ __global__ void __launch_bounds__(WG) k_sp_bwd_small(SpDev d, const int *__restr
             for (int j = 7; j >= 0; j--) {
                 const int k = k0 + j;
                 if (k < ke) {
-                    const double xk = rdlane(div_by(v[s], dg[s], di[s]), k & 63);
+                    const double xk = rdlane(exact ? v[s] / dg[s] : div_by(v[s], dg[s], di[s]), k & 63);
 #pragma unroll
                     for (int q = 0; q <= s; q++) {
                         const int i = lane + 64 * q;
-                        if (i == k) v[q] = xk;
-                        else if (i < k) v[q] -= u[j][q] * xk;
+                        if (i == k) {
+                            num = v[q];
+                            v[q] = xk;
+                        } else if (i < k) {
+                            v[q] -= u[j][q] * xk;
+                        }
                     }
                 }
             }
         }
-    }
+    };
+    static_for<0, SR>([&](auto rc) {
+        constexpr int s = SR - 1 - rc;
+        if (64 * s >= ns) return;
+        double v0[s + 1], num = 1.0;
+#pragma unroll
+        for (int q = 0; q <= s; q++) v0[q] = v[q];
+        pivots(std::integral_constant<int, s>(), std::false_type(), num);
+        /* once more, dividing, where a quotient was out of div_by's range */
+        if (__any(lane + 64 * s < ns && !div_by_ok(num, dg[s]))) {
+#pragma unroll
+            for (int q = 0; q <= s; q++) v[q] = v0[q];
+            pivots(std::integral_constant<int, s>(), std::true_type(), num);
+        }
+    });
 #pragma unroll
     for (int q = 0; q < SR; q++)
         if (lane + 64 * q < ns) x[id[lane + 64 * q]] = v[q];
@@ -966,14 +991,26 @@ __global__ void __launch_bounds__(WG) k_sp_bwd_blk(SpDev d, const int *__restric
 #pragma unroll
         for (int k = 0; k < NB; k++) uv[k] = k < w ? Fr[(int64_t)(kb + k) * nf + kb + row] : 0.0;
         const double dg = Fr[(int64_t)(kb + row) * nf + kb + row], di = 1.0 / dg;
-        double v = tid < w ? wf[kb + row] : 0.0;
+        const double v0 = tid < w ? wf[kb + row] : 0.0;
+        double v = v0, num = 1.0;
+        auto pivots = [&](auto exact) {
 #pragma unroll
-        for (int k = NB - 1; k >= 0; k--) {
-            if (k < w) {
-                const double xk = div_by(rdlane(v, k), rdlane(dg, k), rdlane(di, k));
-                if (tid == k) v = xk;
-                else if (tid < k) v -= uv[k] * xk;
+            for (int k = NB - 1; k >= 0; k--) {
+                if (k < w) {
+                    const double xk = rdlane(exact ? v / dg : div_by(v, dg, di), k);
+                    if (tid == k) {
+                        num = v;
+                        v = xk;
+                    } else if (tid < k) {
+                        v -= uv[k] * xk;
+                    }
+                }
             }
+        };
+        pivots(std::false_type());
+        if (__any(tid < w && !div_by_ok(num, dg))) {   /* as k_sp_bwd_small */
+            v = v0;
+            pivots(std::true_type());
         }
         xb[tid] = tid < w ? v : 0.0;
         if (blockIdx.y == 0 && tid < w) x[d.idx[fr.idx + kb + tid]] = v;

@@ -1065,8 +1065,7 @@ __device__ __forceinline__ double lu_row_terms(double acc, const Prog &r, const 
  * leave the range of normal numbers */
 __device__ __forceinline__ double quotient(double acc, double piv, double inv)
 {
-    const double p = fabs(piv), a = fabs(acc);
-    if (p > 0x1p-400 && p < 0x1p400 && a > 0x1p-500 && a < 0x1p500) return div_by(acc, piv, inv);
+    if (div_by_divisor(piv) && div_by_dividend(acc)) return div_by(acc, piv, inv);
     return acc / piv;
 }
 

@@ -216,3 +216,67 @@ def test_front_sizes(leaves, chain, border, touch):
     ref = spla.spsolve(A, b)
     assert np.abs(x - ref).max() <= 12 * n * 2.0 ** -53 * na * np.abs(ref).max()   # |A^-1| <= 1
     assert np.array_equal(x, _gpu(s, A.data, b))
+
+
+# a front one workgroup solves and one that runs by 64-pivot panels
+@pytest.mark.parametrize('n', [1, 64, 140, 141, 200])
+def test_quotients_at_the_ends_of_the_range(n):
+    """A solve divides: the last pivot of a front may be any number the factor
+    accepts.  Overflow is infinite and not NaN, a subnormal pivot divides, a
+    quotient of or to a small number is rounded once, zeros keep their sign
+    (an upper triangle whose last unknown alone reaches the ends)."""
+    print('case: %d unknowns, last pivot and right-hand side at the ends of the range' % n, flush=True)
+    r, c = np.arange(n), np.arange(n)
+    if n > 1:   # a dense pattern of zeros: one front
+        r, c = np.repeat(r, n), np.tile(c, n)
+    A = sp.csc_matrix((np.ones(len(r)), (r, c)), shape=(n, n))
+    A.sort_indices()
+    s = ngmi.SparseLU(n, A.indptr.astype(np.int64), A.indices.astype(np.int32))
+    assert s.info()['fronts'] == 1
+    ns, nb, _, idx = s.front(0)
+    last = idx[ns - 1]
+    Ai = A.indices
+    cols = np.repeat(np.arange(n), np.diff(A.indptr))
+    tiny, sub = 2.0 ** -1022, 2.0 ** -1060
+    for piv, rhs in [(1e-200, 1e200), (-1e-200, 1e200), (sub, 3 * sub), (sub, 1.0), (sub, 0.0), (3 * sub, 5 * tiny),
+                     (1.7e308, 1e-3), (1.7e308, 1.7e308), (3.0, 7 * tiny), (7.0, 5e-324), (-3.0, 0.0), (3.0, -0.0),
+                     (3.0, np.inf), (1e308, 0.0), (0.7, 1e307), (1e-5, 1e305)]:
+        Ax = np.where((Ai == cols) & (cols == last), piv, np.where(Ai == cols, 1.0, 0.0))
+        b = np.zeros(n)
+        b[last] = rhs
+        x = _gpu(s, Ax, b)
+        with np.errstate(over='ignore'):
+            want = np.float64(rhs) / np.float64(piv)
+        assert x[last] == want and np.signbit(x[last]) == np.signbit(want), (piv, rhs, x[last], want)
+
+
+def test_reciprocals_and_quotients_are_rounded_once():
+    """Pairs [[p, 0], [1, 1]] with right-hand side (a, 0): the pivot's
+    reciprocal is the multiplier, and comes out as the second unknown for a =
+    1; the first is a / p.  Both equal the correctly rounded ones for random
+    mantissas, exponents to +-1000 for the reciprocals and +-350 for the
+    quotients."""
+    n = 1 << 17
+    print('case: %d reciprocals and quotients' % (n // 2), flush=True)
+    i = 2 * np.arange(n // 2)
+    A = sp.csc_matrix((np.ones(3 * len(i)), (np.concatenate([i, i + 1, i + 1]), np.concatenate([i, i, i + 1]))),
+                      shape=(n, n))
+    A.sort_indices()
+    s = ngmi.SparseLU(n, A.indptr.astype(np.int64), A.indices.astype(np.int32))
+    order = np.concatenate([idx[:ns] for ns, _, _, idx in map(s.front, range(s.info()['fronts']))])
+    at = np.argsort(order)
+    led = at[i] < at[i + 1]      # pairs whose reciprocal is a multiplier
+    assert led.sum() > n // 16
+    first = A.indptr[:-1][::2]   # entry (i, i) of each pair
+    g = workloads.rng(31, n)
+    for span, ones in ((1000, True), (350, False)):
+        p = g.uniform(0.5, 1.0, len(i)) * 2.0 ** g.integers(-span, span, len(i)) * g.choice([-1.0, 1.0], len(i))
+        a = np.ones(len(i)) if ones else g.uniform(0.5, 1.0, len(i)) * 2.0 ** g.integers(-span, span, len(i))
+        Ax = np.ones(A.nnz)
+        Ax[first] = p
+        b = np.zeros(n)
+        b[i] = a
+        x = _gpu(s, Ax, b)
+        assert np.array_equal(x[i], a / p)
+        if ones:
+            assert np.array_equal(x[i + 1], -1.0 / p)
