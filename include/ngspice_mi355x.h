@@ -128,6 +128,12 @@ double ngmi_bsim4_set_field(const ngmi_bsim4_set *s, int k, const char *field);
 /* number of per-instance / per-model table columns and table bytes on the device */
 int ngmi_bsim4_set_layout(const ngmi_bsim4_set *s, int *inst_cols, int *model_cols,
                           size_t *device_bytes);
+/* how ngmi_bsim4_eval reads the tables, and its workgroups (of up to 64
+ * instances): NGMI_FORM_COLUMNS a column per field, NGMI_FORM_WAVE a record
+ * per wavefront, NGMI_FORM_LANE a record per lane.  The forms give the same
+ * results bit for bit; the set's size and what its instances share decide. */
+enum { NGMI_FORM_COLUMNS = 0, NGMI_FORM_WAVE = 1, NGMI_FORM_LANE = 2 };
+int ngmi_bsim4_set_form(const ngmi_bsim4_set *s, int *form, int64_t *workgroups);
 
 /* Per-instance evaluation, BSIM4load (b4ld.c:69-5399) on isolated
  * instances: terminal voltages come from vterm (4 x n, rows d g s b, device
@@ -432,6 +438,8 @@ void ngmi_batch_free(ngmi_batch *b);
 int ngmi_batch_info(const ngmi_batch *b, int *n_unknowns, int *nslots, int *nterms, int *levels);
 /* number of topology groups */
 int ngmi_batch_groups(const ngmi_batch *b, int *ngroups);
+/* how the transient reads its MOSFETs' tables (NGMI_FORM_*) */
+int ngmi_batch_form(const ngmi_batch *b, int *form);
 /* circuit c's group, unknowns, recorded unknowns per point and L+U nonzeros */
 int ngmi_batch_circuit_info(const ngmi_batch *b, int c, int *group, int *n_unknowns, int *nprobe,
                             int *nslots);

@@ -463,6 +463,17 @@ int ngmi_bsim4_set_layout(const ngmi_bsim4_set *s, int *inst_cols, int *model_co
     return NGMI_OK;
 }
 
+int ngmi_bsim4_set_form(const ngmi_bsim4_set *s, int *form, int64_t *workgroups)
+{
+    static_assert(NGMI_FORM_COLUMNS == B4T_COLUMNS && NGMI_FORM_WAVE == B4T_UNIFORM && NGMI_FORM_LANE == B4T_LANES,
+                  "the header's forms");
+    if (!s || !s->final_) return NGMI_E_PANIC;
+    if (form) *form = s->tab.mode;
+    if (workgroups)
+        *workgroups = s->tab.mode == B4T_UNIFORM ? s->tab.nitems : (s->tab.n + B4_TILE - 1) / B4_TILE;
+    return NGMI_OK;
+}
+
 int ngmi_bsim4_eval(const ngmi_bsim4_set *s, const ngmi_ckt_scalars *c, const double *vterm,
                     double *const state[3], double *cache, double *stamp, double *rhs,
                     int *noncon, void *stream)

@@ -23,6 +23,7 @@
 
 #include <array>
 #include "bsim4_fields.h"
+#include "ngmi_internal.h"
 
 namespace ngmi {
 
@@ -53,6 +54,28 @@ constexpr std::array<signed char, B4F__COUNT> b4_icols()
 constexpr std::array<signed char, B4F__COUNT> B4_ICOL = b4_icols();
 
 #ifdef __HIPCC__
+
+/* the column form of a table (B4Tab's): the lane's instance is i0 + lane, with
+ * i0 the wave's.  Pointers and strides are held here: read through the
+ * descriptor, they are loaded again behind every store. */
+struct ColPrm {
+    const NGMI_CONST int *code;
+    const NGMI_GLOBAL double *col;   /* instance i0's first column */
+    const NGMI_GLOBAL double *mod;   /* the lane's model's row */
+    int64_t n;
+    unsigned lane;
+    __device__ __forceinline__ ColPrm(const B4Tab &t, int64_t i0, unsigned lane_)
+        : code((const NGMI_CONST int *)t.code), col((const NGMI_GLOBAL double *)t.itab + i0),
+          mod((const NGMI_GLOBAL double *)t.mtab + (int64_t)((const NGMI_GLOBAL int *)t.model_of + i0)[lane_] * t.mcols),
+          n(t.n), lane(lane_)
+    {
+    }
+    __device__ __forceinline__ double operator()(int f) const
+    {
+        const int c = code[f];
+        return c >= 0 ? (col + (int64_t)c * n)[lane] : mod[~c];
+    }
+};
 
 template <int NC, bool UNI>
 struct RecPrm;

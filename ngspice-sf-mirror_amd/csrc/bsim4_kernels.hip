@@ -13,17 +13,6 @@
 
 namespace ngmi {
 
-struct DevPrm {
-    const B4Tab &t;
-    int64_t i;
-    int mi;
-    __device__ __forceinline__ double operator()(int f) const
-    {
-        const int c = t.code[f];
-        return c >= 0 ? t.itab[(int64_t)c * t.n + i] : t.mtab[(int64_t)mi * t.mcols + (~c)];
-    }
-};
-
 /* states: level l row k of the wave's lane at lv[l][k * n + lane] */
 struct DevState {
     NGMI_GLOBAL double *lv[3];
@@ -70,19 +59,19 @@ __device__ __forceinline__ void eval_one(const P &p, const B4Ckt &ck, const Eval
 }
 
 /* Column form.  WAVES = wavefronts per SIMD the register allocation aims
- * for. */
-template <int WAVES>
+ * for; FL >= 0: the selector word every instance shares, compiled as a
+ * constant. */
+template <int WAVES, int FL>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES)))
 k_bsim4_eval_cols(B4Tab tab, B4Ckt ck, EvalIO io)
 {
     const int64_t i0 = (int64_t)blockIdx.x * 64;
     const unsigned lane = threadIdx.x;
     if (i0 + lane >= tab.n) return;
-    eval_one<-1>(DevPrm{tab, i0 + lane, tab.model_of[i0 + lane]}, ck, io, tab.n, i0, lane);
+    eval_one<FL>(ColPrm(tab, i0, lane), ck, io, tab.n, i0, lane);
 }
 
-/* Record form.  WAVES as above; FL >= 0: the selector word every instance
- * shares, compiled as a constant.  UNI: a workgroup per item (tile of 64
+/* Record form.  WAVES and FL as above.  UNI: a workgroup per item (tile of 64
  * instances, record): the tile's lanes of that record run, reading it with
  * scalar loads; a tile whose instances have several records has as many
  * items.  Else a workgroup per tile, each lane reading its own record. */
@@ -122,16 +111,21 @@ int launch_bsim4_eval(const B4Tab &tab, const B4Ckt &ck, const double *vterm,
     EvalIO io{vterm, state[0], state[1], state[2], cache, stamp, rhs, noncon};
     const dim3 nb((unsigned)((tab.n + 63) / 64));
     const bool dflt = tab.flags == B4FL_DEFAULT && tune_get(TUNE_SPECIALISE);
+    const unsigned wgs = tab.mode == B4T_UNIFORM ? (unsigned)tab.nitems : nb.x;
     const int waves = waves_for(TUNE_EVAL_WAVES, tab.n);
-#define NGMI_EVAL(...) hipLaunchKernelGGL((k_bsim4_eval<__VA_ARGS__>), dim3(tab.mode == B4T_UNIFORM ? (unsigned)tab.nitems : nb.x), dim3(64), 0, stream, tab, ck, io)
+#define NGMI_EVAL(...) hipLaunchKernelGGL((k_bsim4_eval<__VA_ARGS__>), dim3(wgs), dim3(64), 0, stream, tab, ck, io)
 #define NGMI_EVAL_W(...) \
     do { \
         if (waves == 1) NGMI_EVAL(1, __VA_ARGS__); \
         else NGMI_EVAL(2, __VA_ARGS__); \
     } while (0)
     if (tab.mode == B4T_COLUMNS) {
-        if (waves == 1) hipLaunchKernelGGL(k_bsim4_eval_cols<1>, nb, dim3(64), 0, stream, tab, ck, io);
-        else hipLaunchKernelGGL(k_bsim4_eval_cols<2>, nb, dim3(64), 0, stream, tab, ck, io);
+#define NGMI_COLS(W, F) hipLaunchKernelGGL((k_bsim4_eval_cols<W, F>), nb, dim3(64), 0, stream, tab, ck, io)
+        if (dflt && waves == 1) NGMI_COLS(1, B4FL_DEFAULT);
+        else if (dflt) NGMI_COLS(2, B4FL_DEFAULT);
+        else if (waves == 1) NGMI_COLS(1, -1);
+        else NGMI_COLS(2, -1);
+#undef NGMI_COLS
     } else if (tab.mode == B4T_LANES) {
         if (dflt) NGMI_EVAL_W(B4FL_DEFAULT, B4_NC_GEOM, false);
         else NGMI_EVAL_W(-1, B4_NC_GEOM, false);

@@ -1452,6 +1452,13 @@ int ngmi_batch_groups(const ngmi_batch *b, int *ngroups)
     return NGMI_OK;
 }
 
+int ngmi_batch_form(const ngmi_batch *b, int *form)
+{
+    if (!b || !form) return NGMI_E_PANIC;
+    *form = b->mos.mode;
+    return NGMI_OK;
+}
+
 int ngmi_batch_circuit_info(const ngmi_batch *b, int c, int *group, int *n_unknowns, int *nprobe,
                             int *nslots)
 {

@@ -36,17 +36,6 @@ __device__ __forceinline__ int lvl(int rb, int l) { return (rb + l) & (NLEV - 1)
 
 /* ---------------- MOSFET evaluation ---------------- */
 
-struct TranPrm {
-    const B4Tab &t;
-    int64_t i;
-    int mi;
-    __device__ __forceinline__ double operator()(int f) const
-    {
-        const int c = t.code[f];
-        return c >= 0 ? t.itab[(int64_t)c * t.n + i] : t.mtab[(int64_t)mi * t.mcols + (~c)];
-    }
-};
-
 static_assert(MOS_ROWS == B4X__COUNT, "state rows of the MOSFET storage");
 
 /* the states and caches of one tile; lane = place within it */
@@ -170,7 +159,7 @@ __device__ __forceinline__ void tran_mos_dense(const MosArgs &A, const B4Tab &ta
     if (K->phase >= PH_DONE || K->pvhold) return;
     int nc;
     if constexpr (COLS) {
-        TranPrm p{tab, i, tab.model_of[i]};
+        ColPrm p(tab, tile * MOS_TILE, lane);
         nc = tran_mos_one<FL>(p, A, K, c, j, tile, lane);
     } else {
         RecPrm<B4_NC_GEOM, false> p{(const NGMI_GLOBAL double *)A.rec +
@@ -2536,7 +2525,8 @@ int launch_tran_pass(const MosLaunch &M, const TranDev *D0, int c_begin, int c_e
         if (waves == 1) MACRO(1, __VA_ARGS__); \
         else MACRO(2, __VA_ARGS__); \
     } while (0)
-        if (M.mode == B4T_COLUMNS) NGMI_W(NGMI_MOS_DENSE, -1, true);
+        if (M.mode == B4T_COLUMNS && dflt) NGMI_W(NGMI_MOS_DENSE, B4FL_DEFAULT, true);
+        else if (M.mode == B4T_COLUMNS) NGMI_W(NGMI_MOS_DENSE, -1, true);
         else if (M.mode == B4T_LANES && dflt) NGMI_W(NGMI_MOS_DENSE, B4FL_DEFAULT, false);
         else if (M.mode == B4T_LANES) NGMI_W(NGMI_MOS_DENSE, -1, false);
         else if (!dflt) NGMI_W(NGMI_MOS, -1, B4_NC_GEOM);

@@ -22,6 +22,9 @@ OK = 0
 E_BADPARM = 7
 E_UNSUPP = 10
 E_SINGULAR = 102
+# how the BSIM4 kernels read their tables: a column per field, a record per
+# wavefront, a record per lane
+FORM_COLUMNS, FORM_WAVE, FORM_LANE = 0, 1, 2
 E_ITERLIM = 103
 E_TIMESTEP = 106
 E_DEVICE = 120
@@ -92,6 +95,7 @@ def lib():
         L.ngmi_bsim4_set_field.restype = d
         L.ngmi_bsim4_set_layout.argtypes = [vp, ctypes.POINTER(i), ctypes.POINTER(i),
                                             ctypes.POINTER(sz)]
+        L.ngmi_bsim4_set_form.argtypes = [vp, ctypes.POINTER(i), ctypes.POINTER(i64)]
         L.ngmi_bsim4_eval.argtypes = [vp, ctypes.POINTER(_Scalars), vp, ctypes.POINTER(vp),
                                       vp, vp, vp, vp, vp]
         L.ngmi_csc_from_elements.argtypes = [i, i64, vp, vp, vp, vp, vp, ctypes.POINTER(i64)]
@@ -200,6 +204,12 @@ class InstanceSet:
         check(lib().ngmi_bsim4_set_layout(self.h, ctypes.byref(a), ctypes.byref(b),
                                           ctypes.byref(c)), 'layout')
         return a.value, b.value, c.value
+
+    def form(self):
+        """(FORM_*, workgroups) of an evaluation"""
+        f, w = ctypes.c_int(), ctypes.c_int64()
+        check(lib().ngmi_bsim4_set_form(self.h, ctypes.byref(f), ctypes.byref(w)), 'form')
+        return f.value, w.value
 
     def eval(self, mode, vterm, states, cache, stamp, rhs, noncon, ag=(0.0,) * 7, order=1,
              method=1, xfact=0.0, gmin=1e-12, reltol=1e-3, abstol=1e-12, stream=0):
@@ -380,6 +390,7 @@ def _tran_protos(L):
                                               ctypes.POINTER(i), i, i, ctypes.POINTER(cp),
                                               ctypes.POINTER(d)]
     L.ngmi_batch_groups.argtypes = [vp, ctypes.POINTER(i)]
+    L.ngmi_batch_form.argtypes = [vp, ctypes.POINTER(i)]
     L.ngmi_batch_write_raw.argtypes = [vp, i, cp, cp, ctypes.POINTER(cp), i]
     L.ngmi_netlist_parse.argtypes = [cp, ctypes.c_uint64]
     L.ngmi_netlist_parse.restype = vp
@@ -829,6 +840,12 @@ class Batch:
         g = ctypes.c_int()
         check(lib().ngmi_batch_groups(self.h, ctypes.byref(g)), 'groups')
         return g.value
+
+    def form(self):
+        """FORM_* of the MOSFETs' tables"""
+        f = ctypes.c_int()
+        check(lib().ngmi_batch_form(self.h, ctypes.byref(f)), 'form')
+        return f.value
 
     def circuit_info(self, c):
         g, n, p, s = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_int()

@@ -181,7 +181,7 @@ def test_gather_assembly_matches_ordered_sum():
 # a lane (many tiles, each with every record), a column per field (no two
 # devices alike)
 @pytest.mark.parametrize('n,geometries,spread', [(1, 1, False), (65, 1, False), (777, 7, True), (777, 7, False),
-                                                 (25601, 8, True), (129, 129, True)])
+                                                 (25601, 8, True), (129, 129, True), (4161, 4161, True)])
 def test_table_forms(n, geometries, spread):
     print('case: %d devices of %d geometries, %s' % (n, geometries, 'interleaved' if spread else 'in runs'), flush=True)
     rng = np.random.default_rng(n + geometries)
@@ -193,6 +193,9 @@ def test_table_forms(n, geometries, spread):
               'delvto': rng.normal(0, 0.03, n)}
     models = [workloads.BASE_NMOS, workloads.BASE_PMOS]
     g, o = GpuEval(models, model_idx, params), OracleBatch(models, model_idx, params)
+    form = g.s.form()
+    print('form %d, %d workgroups' % form, flush=True)
+    assert n != 4161 or form[0] == ngmi.FORM_COLUMNS
     sign = np.where(model_idx == 0, 1.0, -1.0)
     vterm = sign * np.array([rng.uniform(0, 1.2, n), rng.uniform(0, 1.2, n), np.zeros(n), rng.uniform(-0.4, 0, n)])
     gst = [np.zeros((29, n)) for _ in range(3)]

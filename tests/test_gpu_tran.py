@@ -293,3 +293,38 @@ def test_step_widths(name, count, klu):
     assert len(alone[0]) > 5
     for t, x in run(count):
         assert np.array_equal(t, alone[0]) and np.array_equal(x, alone[1])
+
+
+@pytest.mark.parametrize('mobmod', [None, 1])
+def test_column_tables(mobmod):
+    """A batch whose MOSFETs share too few records for record tables (every
+    device its own drain and source areas) reads a column per field; the
+    waveforms are those of its circuits alone, which have records, bit for
+    bit.  With the default selectors and with others."""
+    count, bits, tstop = 30, 5, 1.05e-9
+    print('case: %d adders of %d bits, every ad and as its own, mobmod %s' % (count, bits, mobmod), flush=True)
+    g = workloads.rng(41, bits)
+    descs = []
+    for k in range(count):
+        d = workloads.mc_adder(50 + k, bits=bits)
+        d['mos'] = [m[:5] + (dict(m[5], **{'ad': float(a), 'as': float(s)}),)
+                    for m, a, s in zip(d['mos'], g.uniform(1e-14, 1e-13, len(d['mos'])),
+                                       g.uniform(1e-14, 1e-13, len(d['mos'])))]
+        if mobmod is not None:
+            d['models'] = {key: dict(card, mobmod=mobmod) for key, card in d['models'].items()}
+        descs.append(d)
+
+    def run(ds):
+        b = ngmi.Batch([ngmi.Circuit(d) for d in ds], max_points=4096)
+        rc, _ = b.tran(ds[0]['tstep'], tstop)
+        assert rc == 0, ngmi.last_error()
+        return b, b.info()['unknowns']
+
+    b, n = run(descs)
+    assert b.form() == ngmi.FORM_COLUMNS
+    for c in (0, 13, count - 1):
+        one, _ = run([descs[c]])
+        assert one.form() != ngmi.FORM_COLUMNS
+        t, x = b.waveform(c, n)
+        ta, xa = one.waveform(0, n)
+        assert len(t) > 5 and np.array_equal(t, ta) and np.array_equal(x, xa)
