@@ -428,10 +428,16 @@ int ngmi_bsim4_set_finalize(ngmi_bsim4_set *s)
     for (size_t k = 0; k < at.size(); k++) at[k] = (int)k;
     build_items(R.rec_of, items);
     const size_t ntile = (at.size() + B4_TILE - 1) / B4_TILE, nit = items.size() / 2;
-    /* scalar records run a tile once per record in it: worth it up to a
-     * third more workgroups, or while they all fit two to a SIMD (one of
-     * 1024 SIMDs each) */
-    s->tab.mode = nit <= std::max(ntile + ntile / 3, (size_t)2048) ? B4T_UNIFORM : B4T_LANES;
+    /* Scalar records run a tile once per record in it; a record a lane runs
+     * it once, with slower loads.  Worth it up to a third more workgroups
+     * (524288 devices in runs of one record, 8192 tiles: 9196 items 237 us
+     * against 280, 12235 items 297 against 281), and not for another round
+     * of workgroups, one or two of which each of the 1024 SIMDs takes at a
+     * time (40000 devices, 625 tiles: 688 items 44 us against 45, 1250 55
+     * against 44; 131072, 2048 tiles: 2051 items 76 against 67). */
+    constexpr size_t SIMDS = 1024;
+    const size_t round = ntile <= SIMDS ? SIMDS : ntile <= 2 * SIMDS ? 2 * SIMDS : nit;
+    s->tab.mode = nit <= std::min(ntile + ntile / 3, round) ? B4T_UNIFORM : B4T_LANES;
     s->tab.nc = R.nc;
     s->tab.nitems = (int)nit;
     std::vector<double> tiles;

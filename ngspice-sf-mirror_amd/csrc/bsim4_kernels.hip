@@ -112,7 +112,7 @@ int launch_bsim4_eval(const B4Tab &tab, const B4Ckt &ck, const double *vterm,
     const dim3 nb((unsigned)((tab.n + 63) / 64));
     const bool dflt = tab.flags == B4FL_DEFAULT && tune_get(TUNE_SPECIALISE);
     const unsigned wgs = tab.mode == B4T_UNIFORM ? (unsigned)tab.nitems : nb.x;
-    const int waves = waves_for(TUNE_EVAL_WAVES, tab.n);
+    const int waves = waves_for(TUNE_EVAL_WAVES, (int64_t)wgs * 64);
 #define NGMI_EVAL(...) hipLaunchKernelGGL((k_bsim4_eval<__VA_ARGS__>), dim3(wgs), dim3(64), 0, stream, tab, ck, io)
 #define NGMI_EVAL_W(...) \
     do { \

@@ -176,13 +176,18 @@ def test_gather_assembly_matches_ordered_sum():
     assert np.array_equal(d_ax.cpu().numpy(), ref)
 
 
-# the three forms of the device table: tiles run once per record in them
-# (one record; a few in the same tiles; a last tile of one device), a record
-# a lane (many tiles, each with every record), a column per field (no two
-# devices alike)
-@pytest.mark.parametrize('n,geometries,spread', [(1, 1, False), (65, 1, False), (777, 7, True), (777, 7, False),
-                                                 (25601, 8, True), (129, 129, True), (4161, 4161, True)])
-def test_table_forms(n, geometries, spread):
+# the three forms of the device table: a record a wavefront, tiles run once per
+# record in them (one record; a few, some tiles with two; a last tile of one
+# device), a record a lane (tiles with every record, few tiles and many), a
+# column per field (no two devices alike, and more of them than records are
+# kept for)
+W, L, C = ngmi.FORM_WAVE, ngmi.FORM_LANE, ngmi.FORM_COLUMNS
+
+
+@pytest.mark.parametrize('n,geometries,spread,form', [
+    (1, 1, False, W), (65, 1, False, W), (1400, 7, False, W), (777, 7, True, L), (777, 7, False, L),
+    (25601, 8, True, L), (129, 129, True, L), (4161, 4161, True, C)])
+def test_table_forms(n, geometries, spread, form):
     print('case: %d devices of %d geometries, %s' % (n, geometries, 'interleaved' if spread else 'in runs'), flush=True)
     rng = np.random.default_rng(n + geometries)
     rec = np.arange(n) % geometries if spread else np.arange(n) * geometries // n
@@ -193,9 +198,8 @@ def test_table_forms(n, geometries, spread):
               'delvto': rng.normal(0, 0.03, n)}
     models = [workloads.BASE_NMOS, workloads.BASE_PMOS]
     g, o = GpuEval(models, model_idx, params), OracleBatch(models, model_idx, params)
-    form = g.s.form()
-    print('form %d, %d workgroups' % form, flush=True)
-    assert n != 4161 or form[0] == ngmi.FORM_COLUMNS
+    print('form %d, %d workgroups' % g.s.form(), flush=True)
+    assert g.s.form()[0] == form
     sign = np.where(model_idx == 0, 1.0, -1.0)
     vterm = sign * np.array([rng.uniform(0, 1.2, n), rng.uniform(0, 1.2, n), np.zeros(n), rng.uniform(-0.4, 0, n)])
     gst = [np.zeros((29, n)) for _ in range(3)]
@@ -206,3 +210,45 @@ def test_table_forms(n, geometries, spread):
         gout = g.load(mode, vterm, gst, **kw)
         os_, or_, onc = o.load(mode, vterm, ost, **kw)
         _check_all(gout, gst, o, o.cache, os_, or_, onc, ost)
+
+
+# what decides: tiles of 64, (tile, record) items, and rounds of 1024 or 2048
+# workgroups
+@pytest.mark.parametrize('n,order,form,workgroups', [
+    (40000, 'split', W, 626), (40000, 'mixed', L, 625), (65536, 'split', W, 1024), (65536, 'mixed', L, 1024),
+    (131072, 'split', W, 2048), (131072 - 64, 'split', W, 2048), (131072, 'mixed', L, 2048), (200000, 'split', W, 3126),
+    (5000, 'eight', L, 79), (5000, 'split', W, 80)])
+def test_form_rule(n, order, form, workgroups):
+    """The same devices in the order of their records and mixed: the form
+    follows the order, each device's results do not, bit for bit."""
+    print('case: %d devices, records %s' % (n, order), flush=True)
+    g = np.random.default_rng(n)
+    rec = g.integers(0, 8 if order == 'eight' else 2, n)
+    params = {'l': np.exp(g.uniform(np.log(45e-9), np.log(1e-6), n)),
+              'w': np.exp(g.uniform(np.log(1e-7), np.log(1e-5), n)), 'delvto': g.normal(0, 0.03, n),
+              'ad': 1e-14 * (rec // 2)}
+    mi = (rec % 2).astype(np.int32)
+    at = np.argsort(rec, kind='stable')
+    if order == 'split' and n % 128 == 0:   # whole tiles a record
+        rec = (np.arange(n) >= n // 2).astype(int)
+        mi, at = rec.astype(np.int32), np.arange(n)
+        mixed = g.permutation(n)
+    else:
+        mixed = np.arange(n)
+    sign = np.where(mi == 0, 1.0, -1.0)
+    vterm = sign * np.array([g.uniform(0, 1.2, n), g.uniform(0, 1.2, n), np.zeros(n), g.uniform(-0.4, 0, n)])
+    models = [workloads.BASE_NMOS, workloads.BASE_PMOS]
+
+    def run(ix):
+        e = GpuEval(models, mi[ix], {k: v[ix] for k, v in params.items()})
+        st = [np.zeros((29, n)) for _ in range(3)]
+        h = workloads.H_STEP
+        out = e.load(ngmi.MODETRAN | ngmi.MODEINITFLOAT, vterm[:, ix], st, ag=(1 / h, -1 / h, 0, 0, 0, 0, 0), order=1)
+        back = np.argsort(ix)
+        return e.s.form(), [a[..., back] for a in out] + [a[:, back] for a in st]
+
+    f, a = run(at if order == 'split' else mixed)
+    assert f == (form, workgroups)
+    _, b = run(mixed if order == 'split' else at)
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)
