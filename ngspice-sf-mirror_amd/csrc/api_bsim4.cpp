@@ -141,7 +141,8 @@ static void build_records(const std::vector<double> &rows, const std::vector<int
         by_content.emplace(h, r);
         return r;
     };
-    /* more records than this are no cheaper to read than columns */
+    /* records are not built for sets with more of them than this: 1.9 KB each,
+     * a fraction of the columns' room */
     const size_t most = std::max<size_t>(4096, n / 8);
     for (size_t k = 0; k < n; k++) {
         int r = -1;
@@ -419,15 +420,23 @@ int ngmi_bsim4_set_finalize(ngmi_bsim4_set *s)
     if (rc) return rc;
     s->final_ = false;   /* until its tables are on the device */
     const SetRecords &R = s->recs;
-    if (!R.ok) {
+    std::vector<int> items, at(s->inst.size());
+    for (size_t k = 0; k < at.size(); k++) at[k] = (int)k;
+    if (R.ok) build_items(R.rec_of, items);
+    const size_t ntile = (at.size() + B4_TILE - 1) / B4_TILE, nit = items.size() / 2;
+    constexpr size_t SIMDS = 1024;
+    /* Lanes of one wavefront each with another of many records read 64 lines
+     * where a column is a few; below two rounds of workgroups latency hides
+     * that (65536 devices, 28397 records mixed, 57 us against columns' 61),
+     * and in runs the lines are shared. 524288 devices mixed: 128 records 303
+     * us against 324, 1024 records 337, 8192 records 366; 16385 in runs, 3
+     * a tile, 289. */
+    const bool scattered = ntile > SIMDS && R.rec.size() > (size_t)512 * B4F__COUNT && nit > 16 * ntile;
+    if (!R.ok || scattered) {
         if ((rc = set_upload_columns(s))) return rc;
         s->final_ = true;
         return NGMI_OK;
     }
-    std::vector<int> items, at(s->inst.size());
-    for (size_t k = 0; k < at.size(); k++) at[k] = (int)k;
-    build_items(R.rec_of, items);
-    const size_t ntile = (at.size() + B4_TILE - 1) / B4_TILE, nit = items.size() / 2;
     /* Scalar records run a tile once per record in it; a record a lane runs
      * it once, with slower loads.  Worth it up to a third more workgroups
      * (524288 devices in runs of one record, 8192 tiles: 9196 items 237 us
@@ -435,7 +444,6 @@ int ngmi_bsim4_set_finalize(ngmi_bsim4_set *s)
      * of workgroups, one or two of which each of the 1024 SIMDs takes at a
      * time (40000 devices, 625 tiles: 688 items 44 us against 45, 1250 55
      * against 44; 131072, 2048 tiles: 2051 items 76 against 67). */
-    constexpr size_t SIMDS = 1024;
     const size_t round = ntile <= SIMDS ? SIMDS : ntile <= 2 * SIMDS ? 2 * SIMDS : nit;
     s->tab.mode = nit <= std::min(ntile + ntile / 3, round) ? B4T_UNIFORM : B4T_LANES;
     s->tab.nc = R.nc;

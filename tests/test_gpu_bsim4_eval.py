@@ -217,18 +217,20 @@ def test_table_forms(n, geometries, spread, form):
 @pytest.mark.parametrize('n,order,form,workgroups', [
     (40000, 'split', W, 626), (40000, 'mixed', L, 625), (65536, 'split', W, 1024), (65536, 'mixed', L, 1024),
     (131072, 'split', W, 2048), (131072 - 64, 'split', W, 2048), (131072, 'mixed', L, 2048), (200000, 'split', W, 3126),
-    (5000, 'eight', L, 79), (5000, 'split', W, 80)])
+    (5000, 'eight', L, 79), (5000, 'split', W, 80), (65536, 'scattered', L, 1024), (65537, 'scattered', C, 1025),
+    (65600, 'scattered_few', L, 1025), (65600, 'runs', L, 1025)])
 def test_form_rule(n, order, form, workgroups):
     """The same devices in the order of their records and mixed: the form
     follows the order, each device's results do not, bit for bit."""
     print('case: %d devices, records %s' % (n, order), flush=True)
     g = np.random.default_rng(n)
-    rec = g.integers(0, 8 if order == 'eight' else 2, n)
+    rec = g.integers(0, {'eight': 8, 'scattered': 600, 'scattered_few': 400, 'runs': 1200}.get(order, 2), n)
     params = {'l': np.exp(g.uniform(np.log(45e-9), np.log(1e-6), n)),
               'w': np.exp(g.uniform(np.log(1e-7), np.log(1e-5), n)), 'delvto': g.normal(0, 0.03, n),
               'ad': 1e-14 * (rec // 2)}
     mi = (rec % 2).astype(np.int32)
     at = np.argsort(rec, kind='stable')
+    sorted_ = order in ('split', 'runs')
     if order == 'split' and n % 128 == 0:   # whole tiles a record
         rec = (np.arange(n) >= n // 2).astype(int)
         mi, at = rec.astype(np.int32), np.arange(n)
@@ -247,8 +249,8 @@ def test_form_rule(n, order, form, workgroups):
         back = np.argsort(ix)
         return e.s.form(), [a[..., back] for a in out] + [a[:, back] for a in st]
 
-    f, a = run(at if order == 'split' else mixed)
+    f, a = run(at if sorted_ else mixed)
     assert f == (form, workgroups)
-    _, b = run(mixed if order == 'split' else at)
+    _, b = run(mixed if sorted_ else at)
     for x, y in zip(a, b):
         assert np.array_equal(x, y)
