@@ -1376,9 +1376,13 @@ ngmi_batch *ngmi_batch_new(ngmi_circuit *const *ckts, int C, const int *probe, i
         return bail(nullptr);
     /* the BSIM4 instances of every group, then how the batch stores and
      * reads them: padded storage (a wavefront has one circuit and one record,
-     * read with scalar loads) unless its holes cost more than a third more
-     * wavefronts than dense storage takes and the wavefronts no longer fit
-     * two to a SIMD of the 1024 (small circuits in large batches) */
+     * read with scalar loads) unless its holes cost more than three quarters
+     * more wavefronts than dense storage takes.  ms of a .tran, padded /
+     * dense, by that ratio: 1.27 (1000 rings of 101 stages) 29.7 / 35.8; 1.52
+     * (1500 3-bit adders) 76.0 / 80.3; 1.71 (512 rings of 75) 21.0 / 24.1;
+     * 1.83 (200 5-bit adders) 53.7 / 50.6; 4.6 (256 1-bit adders) 47.7 / 37.0;
+     * 21 (1000 rings of 3) 22.6 / 14.9; 64 (a 16-bit adder whose devices all
+     * differ) 95 / 38 */
     int64_t wp = 0, wd = 0;
     bool records = true, pad = true;
     std::vector<std::vector<const ngmi_circuit *>> cs(members.size());
@@ -1397,7 +1401,7 @@ ngmi_batch *ngmi_batch_new(ngmi_circuit *const *ckts, int C, const int *probe, i
         wp += (int64_t)G->C * (int64_t)(G->place.size() / MOS_TILE);
         wd += ((int64_t)G->C * G->NM + MOS_TILE - 1) / MOS_TILE;
     }
-    b->mos.mode = !records ? B4T_COLUMNS : pad && wp <= std::max<int64_t>(wd + wd / 3, 2048) ? B4T_UNIFORM : B4T_LANES;
+    b->mos.mode = !records ? B4T_COLUMNS : pad && wp <= wd + 3 * wd / 4 ? B4T_UNIFORM : B4T_LANES;
     std::vector<TranDev> Ds;
     std::vector<B4Tab> tabs;
     std::vector<int2> sb;

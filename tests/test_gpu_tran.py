@@ -328,3 +328,40 @@ def test_column_tables(mobmod):
         t, x = b.waveform(c, n)
         ta, xa = one.waveform(0, n)
         assert len(t) > 5 and np.array_equal(t, ta) and np.array_equal(x, xa)
+
+
+@pytest.mark.parametrize('name,count,areas,form', [
+    ('ring3', 40, 1, ngmi.FORM_LANE), ('ring45', 40, 1, ngmi.FORM_WAVE), ('ring75', 2, 1, ngmi.FORM_WAVE),
+    ('adder1', 40, 1, ngmi.FORM_LANE), ('adder5', 3, 1, ngmi.FORM_WAVE), ('adder5', 8, 1, ngmi.FORM_LANE), ('adder5', 1, 1, ngmi.FORM_WAVE),
+    ('adder5', 1, 140, ngmi.FORM_LANE), ('adder5', 7, 140, ngmi.FORM_LANE), ('adder16', 1, 1, ngmi.FORM_WAVE)])
+def test_storage_rule(name, count, areas, form):
+    """Padded storage (a record a wavefront) while its holes add at most three
+    quarters of the wavefronts, dense (a record a lane) else; a circuit's
+    waveform is the same in either, bit for bit (in a batch of rings or
+    adders of its size, beside one of 101 stages, and alone)."""
+    print('case: %s x %d, %d drain areas' % (name, count, areas), flush=True)
+    size = int(name.lstrip('ringade'))
+    descs = [workloads.ring_oscillator(stages=size) if name.startswith('ring') else workloads.mc_adder(3, bits=size)
+             for _ in range(count)]
+    for d in descs:
+        if areas > 1:
+            d['mos'] = [m[:5] + (dict(m[5], ad=1e-14 * (1 + k % areas)),) for k, m in enumerate(d['mos'])]
+    tstop = 0.15e-9 if name.startswith('ring') else 1.05e-9
+
+    def run(ds):
+        b = ngmi.Batch([ngmi.Circuit(d) for d in ds], max_points=4096)
+        rc, _ = b.tran(descs[0]['tstep'], tstop)
+        assert rc == 0, ngmi.last_error()
+        return b
+
+    b = run(descs)
+    assert b.form() == form
+    n = b.info()['unknowns']
+    first = b.waveform(0, n)
+    assert len(first[0]) > 5
+    big = workloads.ring_oscillator(stages=301)
+    mixed = run([descs[0]] + [big] * (4 * count))   # padded for the large ring's sake where the small is few
+    for o, c in ((run(descs[:1]), 0), (b, count - 1), (mixed, 0)):
+        t, x = o.waveform(c, n)
+        assert np.array_equal(t, first[0]) and np.array_equal(x, first[1]), o.form()
+    print('forms: batch %d, alone %d, mixed %d' % (b.form(), run(descs[:1]).form(), mixed.form()), flush=True)
