@@ -730,9 +730,9 @@ __device__ __forceinline__ double circuit_terr(const TranDev &D, const CktCtl *K
         const double c1 = Q[((int64_t)lvl(rb, 1) * 2 + 1) * cnc];
         m = fmin(m, terr_one(q0, q1, q2, q3, c0, c1, K, D));
     }
-    /* qb, qg and qd of each MOSFET (holes hold zeros, whose bound is that of a
-     * constant charge) */
+    /* qb, qg and qd of each MOSFET (holes hold zeros, and bound nothing) */
     for (int j = threadIdx.x; j < D.NS; j += blockDim.x) {
+        const int drain = ((const NGMI_GLOBAL int *)D.mos_nodes)[j];
         const NGMI_GLOBAL double *Q =
             (const NGMI_GLOBAL double *)D.mstate + mos_at((int64_t)c * D.NS + j, 0, B4X_qb);
         constexpr int lv = MOS_ROWS * MOS_TILE;
@@ -749,7 +749,10 @@ __device__ __forceinline__ double circuit_terr(const TranDev &D, const CktCtl *K
             c1[r] = Q[l1 + k + MOS_TILE];
         }
 #pragma unroll
-        for (int r = 0; r < 3; r++) m = fmin(m, terr_one(q0[r], q1[r], q2[r], q3[r], c0[r], c1[r], K, D));
+        for (int r = 0; r < 3; r++) {
+            const double t = terr_one(q0[r], q1[r], q2[r], q3[r], c0[r], c1[r], K, D);
+            if (drain >= 0) m = fmin(m, t);
+        }
     }
     return group_min(m);
 }

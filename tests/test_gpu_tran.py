@@ -365,3 +365,34 @@ def test_storage_rule(name, count, areas, form):
         t, x = o.waveform(c, n)
         assert np.array_equal(t, first[0]) and np.array_equal(x, first[1]), o.form()
     print('forms: batch %d, alone %d, mixed %d' % (b.form(), run(descs[:1]).form(), mixed.form()), flush=True)
+
+
+@pytest.mark.parametrize('order', [1, 2])
+def test_slow_transient_storage(order):
+    """Steps of seconds, where the truncation error's absolute tolerance binds:
+    the empty places of padded storage bound no step, so time points and
+    waveforms are those of dense storage, bit for bit.  65 MOSFETs of one
+    record (63 empty places), gate and drain ramping for 1000 s, alone (padded)
+    and beside smaller ones (dense)."""
+    print('case: slow ramp, maxord %d' % order, flush=True)
+    d = {'nnodes': 2, 'models': {'n': dict(workloads.BASE_NMOS)},
+         'mos': [('n', 2, 1, 0, 0, {'w': 1e-4, 'l': 1e-6, 'delvto': 1e-3 * k}) for k in range(65)],
+         'caps': [(1, 2, 1e-3)], 'res': [], 'vsrc': [(1, 0, 0.0, (0.0, 1.0, 10.0, 1000.0, 1000.0, 500.0, 4000.0)),
+                                                     (2, 0, 1.0, (1.0, 0.7, 10.0, 700.0, 1000.0, 500.0, 4000.0))],
+         'ic': {}, 'options': {'maxord': order}}
+
+    def run(ds):
+        b = ngmi.Batch([ngmi.Circuit(x) for x in ds], max_points=8192)
+        rc, _ = b.tran(50.0, 2000.0, max_passes=200000)
+        assert rc == 0, ngmi.last_error()
+        return b
+
+    one = run([d])
+    assert one.form() == ngmi.FORM_WAVE
+    n = one.info()['unknowns']
+    ta, xa = one.waveform(0, n)
+    print('%d points, largest step %.3f s' % (len(ta), np.diff(ta).max()), flush=True)
+    dense = run([d] + [dict(d, mos=d['mos'][:6]) for _ in range(64)])
+    assert dense.form() == ngmi.FORM_LANE
+    tb, xb = dense.waveform(0, n)
+    assert np.diff(ta).max() > 2.6 and np.array_equal(ta, tb) and np.array_equal(xa, xb)
