@@ -468,7 +468,8 @@ int splu_analyze(int n, const int64_t *Ap, const int *Ai, SpluSym &S)
                 S.ent_src[q] = tmp[q - b].second;
             }
             in.clear();
-            for (int k = S.kid_ptr[f]; k < S.kid_ptr[f + 1]; k++) {
+            const bool many = S.kid_ptr[f + 1] - S.kid_ptr[f] > SPLU_KIDS;
+            for (int k = S.kid_ptr[f]; k < S.kid_ptr[f + 1] && !many; k++) {
                 const int c = S.kids[k];
                 const int *rl = S.rel.data() + S.idx_off[c] + S.ns[c];   /* ascending */
                 for (int i = 0; i < S.nb[c]; i++)
@@ -489,28 +490,52 @@ int splu_analyze(int n, const int64_t *Ap, const int *Ai, SpluSym &S)
             }
         }
     }
-    /* inverse of the children's relative indices; the fronts' records */
+    /* inverse of the children's relative indices, by child or by unknown; the
+     * fronts' records */
     S.inv_off.assign(nfr, 0);
+    auto by_child = [&](int f) {
+        return S.kid_ptr[f + 1] - S.kid_ptr[f] <= SPLU_KIDS || S.ns[f] + S.nb[f] <= SPLU_SMALL;
+    };
     {
         size_t all = 0;
-        for (int f = 0; f < nfr; f++) all += (size_t)(S.kid_ptr[f + 1] - S.kid_ptr[f]) * (S.ns[f] + S.nb[f]);
+        for (int f = 0; f < nfr; f++)
+            if (by_child(f)) all += (size_t)(S.kid_ptr[f + 1] - S.kid_ptr[f]) * (S.ns[f] + S.nb[f]);
         S.inv.reserve(all);
         S.front.reserve(nfr);
         S.kid.reserve(S.kids.size());
     }
     for (int f = 0; f < nfr; f++) {
-        const int nf = S.ns[f] + S.nb[f], nk = S.kid_ptr[f + 1] - S.kid_ptr[f];
+        const int nf = S.ns[f] + S.nb[f], k0 = S.kid_ptr[f], nk = S.kid_ptr[f + 1] - k0;
         S.inv_off[f] = (int64_t)S.inv.size();
         S.front.push_back({S.ns[f], nf, nk, (int)(S.ent_ptr[f + 1] - S.ent_ptr[f]), S.off[f], S.idx_off[f],
-                           S.ent_ptr[f], S.inv_off[f], S.kid_ptr[f], S.cg_off[f], S.gk_off[f]});
-        for (int k = S.kid_ptr[f]; k < S.kid_ptr[f + 1]; k++) {
+                           S.ent_ptr[f], S.inv_off[f], S.kid_ptr[f], S.cg_off[f], S.gk_off[f], -1, 0});
+        for (int k = k0; k < k0 + nk; k++) {
             const int c = S.kids[k];
-            const size_t at = S.inv.size();
-            S.inv.resize(at + nf, -1);
-            const int *rl = S.rel.data() + S.idx_off[c] + S.ns[c];
-            for (int i = 0; i < S.nb[c]; i++) S.inv[at + rl[i]] = i;
             const int nfc = S.ns[c] + S.nb[c];
-            S.kid.push_back({S.off[c] + (int64_t)S.ns[c] * nfc + S.ns[c], S.idx_off[c] + S.ns[c], nfc, 0});
+            if (by_child(f)) {
+                const size_t at = S.inv.size();
+                S.inv.resize(at + nf, -1);
+                const int *rl = S.rel.data() + S.idx_off[c] + S.ns[c];
+                for (int i = 0; i < S.nb[c]; i++) S.inv[at + rl[i]] = i;
+            }
+            S.kid.push_back({S.off[c] + (int64_t)S.ns[c] * nfc + S.ns[c], S.idx_off[c] + S.ns[c], nfc, S.nb[c]});
+        }
+        if (nk <= SPLU_KIDS) continue;
+        S.front[f].up = (int64_t)S.up_ptr.size();
+        S.front[f].upe = (int64_t)S.up_ent.size();
+        std::vector<int> at(nf + 1, 0);
+        for (int k = k0; k < k0 + nk; k++) {
+            const int c = S.kids[k];
+            const int *rl = S.rel.data() + S.idx_off[c] + S.ns[c];
+            for (int i = 0; i < S.nb[c]; i++) at[rl[i] + 1]++;
+        }
+        for (int r = 0; r < nf; r++) at[r + 1] += at[r];
+        S.up_ptr.insert(S.up_ptr.end(), at.begin(), at.end());
+        S.up_ent.resize(S.up_ent.size() + at[nf]);
+        for (int k = k0; k < k0 + nk; k++) {
+            const int c = S.kids[k];
+            const int *rl = S.rel.data() + S.idx_off[c] + S.ns[c];
+            for (int i = 0; i < S.nb[c]; i++) S.up_ent[S.front[f].upe + at[rl[i]]++] = {k - k0, i};
         }
     }
 

@@ -16,20 +16,29 @@ constexpr int SPLU_LEAF = 64;          /* nested dissection stops at this many v
 constexpr int SPLU_SMALL = 140;
 constexpr int SPLU_NB = 64;            /* panel width of the larger fronts */
 constexpr int SPLU_CG = 16;            /* columns a workgroup assembles of a larger front */
-constexpr int SPLU_MAX_FRONT = 8000;   /* a front's right-hand side and the solve kernels'
-                                          static LDS fit 64 KB */
+/* a front with more children than this lists, for each of its unknowns, the
+ * children whose boundary holds it; one with fewer lists, for each child, where
+ * the child's boundary holds each unknown (children x unknowns, read side by
+ * side; the few children of a mesh's fronts) */
+constexpr int SPLU_KIDS = 16;
+constexpr int SPLU_MAX_FRONT = 8000;   /* a column of a front fits 64 KB of LDS */
 
 /* what the numeric kernels need of a front, in one record, and of each of
  * its children (kid0 on): where the Schur complement starts in the store, its
- * leading dimension, where its boundary's part of the solves' work vector
- * starts */
+ * leading dimension and size, where its boundary's part of the solves' work
+ * vector, and of the indices in the parent, starts */
 struct SpluFront {
     int ns, nf, nkid, nent;
     int64_t off, idx, ent, inv, kid0, cg, gk;
+    int64_t up, upe;   /* up: -1 without lists by unknown */
 };
 struct SpluKid {
     int64_t schur, wk;
-    int ld, pad;
+    int ld, nb;
+};
+/* child q (from kid0) holds an unknown at its boundary index i */
+struct SpluUp {
+    int q, i;
 };
 
 struct SpluSym {
@@ -54,9 +63,13 @@ struct SpluSym {
     std::vector<SpluKid> kid;
     std::vector<uint32_t> ent_rc;
     /* at inv_off[f] + q nf + r the boundary index in child q of the front's
-     * local unknown r, or -1 */
+     * local unknown r, or -1; kept where f has few children, or is small */
     std::vector<int64_t> inv_off;
     std::vector<int> inv;
+    /* where f has many: local unknown r is held by up_ent[front[f].upe + k],
+     * k from up_ptr[front[f].up + r] to the next, children in order */
+    std::vector<int> up_ptr;
+    std::vector<SpluUp> up_ent;
     int H = 0;                           /* largest height */
     std::vector<int> lev_ptr, lev;       /* fronts by height, by size within one */
     int max_front = 0;

@@ -195,10 +195,13 @@ def _bordered(leaves, chain, border, touch, seed):
 
 # one front (leaves 0) around the 16-pivot steps, the 64-pivot panels, the
 # edges of 64-row chunks and the 140 unknowns one workgroup takes; trees whose
-# root gathers from many children, in LDS and 16 columns a workgroup
+# root gathers from many children, in LDS and a column a wavefront, from 16 and
+# 17 of them, with boundaries under and over 64 unknowns
 @pytest.mark.parametrize('leaves,chain,border,touch', [
     (0, 1, n, 0) for n in (1, 2, 15, 16, 17, 33, 63, 64, 65, 129, 139, 140, 141, 142, 192, 193, 257, 391)
-] + [(200, 4, 8, 2), (900, 3, 60, 3), (1000, 4, 130, 6), (1000, 4, 300, 6), (5000, 3, 100, 3), (64, 1, 65, 1)])
+] + [(200, 4, 8, 2), (900, 3, 60, 3), (1000, 4, 130, 6), (1000, 4, 300, 6), (5000, 3, 100, 3), (64, 1, 65, 1),
+     (310, 3, 150, 3), (336, 3, 150, 3), (300, 3, 100, 3), (318, 3, 100, 3), (1200, 1, 200, 40), (1260, 1, 200, 40),
+     (60, 20, 200, 100)])
 def test_front_sizes(leaves, chain, border, touch):
     print('case: %d leaves of %d, %d of a border of %d each' % (leaves, chain, touch, border), flush=True)
     A = _bordered(leaves, chain, border, touch, 11) if leaves else _bordered(1, 1, max(border - 1, 1), 1, 11)
