@@ -931,24 +931,14 @@ __global__ void __launch_bounds__(WG) k_sp_bwd_small(SpDev d, const int *__restr
         if (lane + 64 * q < ns) x[id[lane + 64 * q]] = v[q];
 }
 
-constexpr int SWG = 512;
-
-/* larger fronts, forward: the right-hand side gathered into wk */
-__global__ void __launch_bounds__(SWG) k_sp_fwd_init(SpDev d, const int *__restrict__ list,
-                                                     const double *__restrict__ bp, double *__restrict__ wk)
-{
-    const SpluFront fr = d.front[list[blockIdx.x]];
-    const int k = blockIdx.y * SWG + threadIdx.x;
-    if (k < fr.nf) wk[fr.idx + k] = gather_rhs(d, fr, k, bp, wk);
-}
-
 /* Panel p forward: the 64 pivots solved by wave 0 of every workgroup (one
  * row a lane, the solved pivot broadcast), then each of the workgroup's 256
  * rows below takes its 64 products.  Its loads need nothing of the triangle
- * and are issued before it. */
+ * and are issued before it.  Panel 0 gathers the rows (a launch of its own
+ * for that cost 6 us a height), the others find them in wk. */
 __global__ void __launch_bounds__(WG) k_sp_fwd_blk(SpDev d, const int *__restrict__ list, int p,
-                                                   const double *__restrict__ F, double *__restrict__ wk,
-                                                   double *__restrict__ y)
+                                                   const double *__restrict__ F, const double *__restrict__ bp,
+                                                   double *wk, double *__restrict__ y)
 {
     const SpluFront fr = d.front[list[blockIdx.x]];
     const int nsf = fr.ns, nf = fr.nf;
@@ -964,13 +954,14 @@ __global__ void __launch_bounds__(WG) k_sp_fwd_blk(SpDev d, const int *__restric
     double l[NB];
 #pragma unroll
     for (int k = 0; k < NB; k++) l[k] = k < w ? Fr[(int64_t)(kb + k) * nf + ic] : 0.0;
-    double ri = wf[ic];
+    double ri = p == 0 ? gather_rhs(d, fr, ic, bp, wk) : wf[ic];
     if (tid < 64) {
         double lv[NB];
         const int row = kb + min(tid, w - 1);
 #pragma unroll
         for (int k = 0; k < NB; k++) lv[k] = k < w ? Fr[(int64_t)(kb + k) * nf + row] : 0.0;
-        double v = tid < w ? wf[row] : 0.0;
+        double v = p == 0 ? gather_rhs(d, fr, row, bp, wk) : wf[row];
+        if (tid >= w) v = 0.0;
 #pragma unroll
         for (int k = 0; k < NB; k++) {
             const double yk = rdlane(v, k);
@@ -1030,10 +1021,11 @@ __global__ void __launch_bounds__(OFF_WG) k_sp_bwd_off(SpDev d, const int *__res
 }
 
 /* panel p backward, as k_sp_fwd_blk: the 64 pivots from the last, then 256
- * rows above per workgroup */
+ * rows above per workgroup.  A front without a boundary starts from y, the
+ * others from what k_sp_bwd_off left in wk. */
 __global__ void __launch_bounds__(WG) k_sp_bwd_blk(SpDev d, const int *__restrict__ list, int p,
-                                                   const double *__restrict__ F, double *__restrict__ wk,
-                                                   double *__restrict__ x)
+                                                   const double *__restrict__ F, const double *__restrict__ y,
+                                                   double *__restrict__ wk, double *__restrict__ x)
 {
     const SpluFront fr = d.front[list[blockIdx.x]];
     const int nsf = fr.ns, nf = fr.nf;
@@ -1049,14 +1041,16 @@ __global__ void __launch_bounds__(WG) k_sp_bwd_blk(SpDev d, const int *__restric
     double u[NB];
 #pragma unroll
     for (int k = 0; k < NB; k++) u[k] = k < w ? Fr[(int64_t)(kb + k) * nf + ic] : 0.0;
-    double ri = wf[ic];
+    const bool fresh = nf == nsf && kb + NB >= nsf;
+    const int *id = d.idx + fr.idx;
+    double ri = fresh ? y[id[ic]] : wf[ic];
     if (tid < 64) {
         double uv[NB];
         const int row = min(tid, w - 1);
 #pragma unroll
         for (int k = 0; k < NB; k++) uv[k] = k < w ? Fr[(int64_t)(kb + k) * nf + kb + row] : 0.0;
         const double dg = Fr[(int64_t)(kb + row) * nf + kb + row], di = 1.0 / dg;
-        const double v0 = tid < w ? wf[kb + row] : 0.0;
+        const double v0 = tid < w ? (fresh ? y[id[kb + row]] : wf[kb + row]) : 0.0;
         double v = v0, num = 1.0;
         auto pivots = [&](auto exact) {
 #pragma unroll
@@ -1078,7 +1072,7 @@ __global__ void __launch_bounds__(WG) k_sp_bwd_blk(SpDev d, const int *__restric
             pivots(std::true_type());
         }
         xb[tid] = tid < w ? v : 0.0;
-        if (blockIdx.y == 0 && tid < w) x[d.idx[fr.idx + kb + tid]] = v;
+        if (blockIdx.y == 0 && tid < w) x[id[kb + tid]] = v;
     }
     __syncthreads();
     double s = 0.0;
@@ -1088,7 +1082,7 @@ __global__ void __launch_bounds__(WG) k_sp_bwd_blk(SpDev d, const int *__restric
     if (i < kb) wf[i] = ri;
 }
 
-enum { L_SMALL, L_ASM, L_ASM_MANY, L_PANEL, L_UPDATE, L_FWD_SMALL, L_FWD_INIT, L_FWD_DBK, L_BWD_SMALL, L_BWD_OFF, L_BWD_DBK };
+enum { L_SMALL, L_ASM, L_ASM_MANY, L_PANEL, L_UPDATE, L_FWD_SMALL, L_FWD_DBK, L_BWD_SMALL, L_BWD_OFF, L_BWD_DBK };
 /* a launch: fronts lev[first ..+gx) (L_ASM_MANY: of the list of those with many
  * children), panel p, gy workgroups a front, dynamic LDS */
 struct Step {
@@ -1220,10 +1214,11 @@ static int splu_device_alloc(ngmi_splu *s)
         if (big == e) continue;
         const unsigned nl = (unsigned)(e - big);
         most = std::max(most, e - big);
-        int maxns = 0, manynf = 0;
+        int maxns = 0, maxnb = 0, manynf = 0;
         const int many0 = (int)many.size();
         for (int q = big; q < e; q++) {
             maxns = std::max(maxns, S.ns[S.lev[q]]);
+            maxnb = std::max(maxnb, S.nb[S.lev[q]]);
             if (S.front[S.lev[q]].up < 0) continue;
             many.push_back(S.lev[q]);
             manynf = std::max(manynf, size(q));
@@ -1233,7 +1228,6 @@ static int splu_device_alloc(ngmi_splu *s)
         if (manynf)
             s->factor.push_back({L_ASM_MANY, many0, 0, (unsigned)many.size() - many0, (unsigned)manynf,
                                  manynf * sizeof(double)});
-        s->fwd.push_back({L_FWD_INIT, big, 0, nl, (unsigned)((maxnf + SWG - 1) / SWG), 0});
         std::vector<Step> bb;
         for (int p = 0; p * NB < maxns; p++) {
             int64_t chunks = 1, tiles = 1, below = 1;
@@ -1256,7 +1250,7 @@ static int splu_device_alloc(ngmi_splu *s)
             bb.push_back({L_BWD_DBK, big, p, nl, (unsigned)std::max(1, (p * NB + WG - 1) / WG), 0});
         }
         back.insert(back.end(), bb.begin(), bb.end());
-        back.push_back({L_BWD_OFF, big, 0, nl, (unsigned)((maxns + OFF_ROWS - 1) / OFF_ROWS), 0});
+        if (maxnb) back.push_back({L_BWD_OFF, big, 0, nl, (unsigned)((maxns + OFF_ROWS - 1) / OFF_ROWS), 0});
     }
     s->bwd.assign(back.rbegin(), back.rend());
     DO(put(s->d_many, many));
@@ -1394,9 +1388,7 @@ int ngmi_splu_solve(ngmi_splu *s, double *b, void *stream)
         const dim3 g(p.gx, p.gy);
         if (p.kind == L_FWD_SMALL)
             hipLaunchKernelGGL(k_sp_fwd_small, g, dim3(WG), p.lds, st, s->d, list, s->F, s->vb, s->wk, s->vy);
-        else if (p.kind == L_FWD_INIT)
-            hipLaunchKernelGGL(k_sp_fwd_init, g, dim3(SWG), 0, st, s->d, list, s->vb, s->wk);
-        else hipLaunchKernelGGL(k_sp_fwd_blk, g, dim3(WG), 0, st, s->d, list, p.p, s->F, s->wk, s->vy);
+        else hipLaunchKernelGGL(k_sp_fwd_blk, g, dim3(WG), 0, st, s->d, list, p.p, s->F, s->vb, s->wk, s->vy);
     }
     for (const Step &p : s->bwd) {
         const int *list = s->d_lev + p.first;
@@ -1405,7 +1397,7 @@ int ngmi_splu_solve(ngmi_splu *s, double *b, void *stream)
             hipLaunchKernelGGL(k_sp_bwd_small, g, dim3(WG), p.lds, st, s->d, list, s->F, s->vy, s->vx);
         else if (p.kind == L_BWD_OFF)
             hipLaunchKernelGGL(k_sp_bwd_off, g, dim3(OFF_WG), 0, st, s->d, list, s->F, s->vy, s->vx, s->wk);
-        else hipLaunchKernelGGL(k_sp_bwd_blk, g, dim3(WG), 0, st, s->d, list, p.p, s->F, s->wk, s->vx);
+        else hipLaunchKernelGGL(k_sp_bwd_blk, g, dim3(WG), 0, st, s->d, list, p.p, s->F, s->vy, s->wk, s->vx);
     }
     NGMI_HIP(hipGetLastError());
     NGMI_HIP(hipMemcpyAsync(b, s->vx, (size_t)S.n * sizeof(double), hipMemcpyDeviceToDevice, st));
