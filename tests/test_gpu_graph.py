@@ -91,6 +91,8 @@ def test_autotune_and_cache():
             print(rep, flush=True)
             chosen = {k: ngmi.get_tune(k) for k in before}
             assert 'chosen' in rep and os.path.exists(path)
+            # values that run another's kernel are not tried
+            assert 'mos_waves=1:' in rep and 'mos_waves=3:' not in rep and 'mos_waves=4:' not in rep
             for k, v in before.items():
                 ngmi.tune(k, v)
             assert ngmi.autotune_load(circ, path)
