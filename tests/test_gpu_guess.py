@@ -182,6 +182,50 @@ def test_features_match_the_engine_bit_for_bit():
     assert checked > 1000
 
 
+def _fixed_net(seed):
+    """a network of fixed parameters, no training in between"""
+    g = np.random.default_rng(seed)
+    net = ngmi.GuessNet(seed=1)
+    p = net.params()
+    p += (0.02 * g.standard_normal(len(p)) * (p != 0)).astype(np.float32)
+    net.set_params(p)
+    return net
+
+
+@pytest.mark.parametrize('bits,count', [(1, 513), (2, 520)])
+def test_learned_step_widths(bits, count):
+    """A learned transient at fixed parameters: the circuits' feature rows,
+    starting values and waveforms do not depend on whether a step takes four
+    wavefronts (up to 512 circuits a launch) or one, nor on which circuits
+    are beside, bit for bit."""
+    print('case: learned guess of fixed parameters, %d-bit adders alone and %d in a launch' % (bits, count), flush=True)
+    net = _fixed_net(17)
+    tstop, seeds = 1.2e-9, (0, 1, 2)
+
+    def run(ds):
+        b = ngmi.Batch([ngmi.Circuit(d) for d in ds], max_points=2048)
+        b.set_guess(net)
+        rc, _ = b.tran(workloads.ADDER_TSTEP, tstop)
+        assert rc == 0, ngmi.last_error()
+        return b
+
+    ds = [workloads.mc_adder(s, bits=bits) for s in seeds]
+    keep = ngmi.get_tune('streams')
+    try:
+        ngmi.tune('streams', 1)
+        b = run([ds[k % 3] for k in range(count)])
+    finally:
+        ngmi.tune('streams', keep)
+    for k, d in enumerate(ds):
+        one = run([d])
+        t1, x1 = one.waveform(0)
+        assert one.guess_stats(0)['guessed'] > 10
+        for c in (k, k + 3 * ((count - 1 - k) // 3)):
+            t, x = b.waveform(c)
+            assert np.array_equal(t, t1) and np.array_equal(x, x1)
+            assert b.guess_stats(c) == one.guess_stats(0) and b.stats(c) == one.stats(0)
+
+
 def test_forward_beside_a_layered_transient(trained):
     """With the network run layer by layer (guess_fused 0), forward calls on
     another stream and thread, of more rows than the transient's and of fewer

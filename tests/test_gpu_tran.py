@@ -267,11 +267,20 @@ def test_operating_point_stepping():
             _compare('%s-%s' % (tag, how), eng, ora, d['nnodes'])
 
 
+@pytest.fixture
+def one_stream():
+    """a batch's circuits in one launch, not in halves on two streams"""
+    keep = ngmi.get_tune('streams')
+    ngmi.tune('streams', 1)
+    yield
+    ngmi.tune('streams', keep)
+
+
 @pytest.mark.parametrize('name,count,klu', [('ring3', 513, False), ('ring45', 1040, False), ('adder1', 1025, False),
                                             ('adder5', 513, True)])
-def test_step_widths(name, count, klu):
+def test_step_widths(name, count, klu, one_stream):
     """A circuit alone (its step by four wavefronts) and as one of more than
-    two to a compute unit (by one): the same sums in the same order, so the
+    512 in a launch (by one): the same sums in the same order, so the
     waveforms are equal bit for bit.  adder5 on KLU's order, whose solve runs
     block by block; its supply rows are partial sums and combines."""
     print('case: %s alone and %d times, klu order %s' % (name, count, klu), flush=True)
@@ -293,6 +302,32 @@ def test_step_widths(name, count, klu):
     assert len(alone[0]) > 5
     for t, x in run(count):
         assert np.array_equal(t, alone[0]) and np.array_equal(x, alone[1])
+
+
+@pytest.mark.parametrize('count', [512, 513, 700])
+def test_step_widths_of_mixed_topologies(count):
+    """Rings of two sizes and adders in one launch, up to 512 circuits by four
+    wavefronts each and more by one: each as it is alone, bit for bit."""
+    print('case: %d circuits of three topologies' % count, flush=True)
+    kinds = [workloads.ring_oscillator(stages=5), workloads.ring_oscillator(stages=45), workloads.mc_adder(5, bits=2)]
+    for d in kinds:
+        d['tstep'] = 5e-12
+    tstop = 0.15e-9
+
+    def run(ds):
+        b = ngmi.Batch([ngmi.Circuit(d) for d in ds], max_points=2048)
+        rc, _ = b.tran(5e-12, tstop)
+        assert rc == 0, ngmi.last_error()
+        return b
+
+    b = run([kinds[k % 3] for k in range(count)])
+    assert b.groups() == 3
+    for k, d in enumerate(kinds):
+        one = run([d]).waveform(0)
+        assert len(one[0]) > 5
+        for c in (k, k + 3 * ((count - 1 - k) // 3)):
+            t, x = b.waveform(c)
+            assert np.array_equal(t, one[0]) and np.array_equal(x, one[1])
 
 
 @pytest.mark.parametrize('mobmod', [None, 1])
