@@ -2543,11 +2543,15 @@ int launch_tran_pass(const MosLaunch &M, const TranDev *D0, int c_begin, int c_e
     }
     if (ev) NGMI_HIP(hipEventRecord(ev[1], s));
     const int ns = D0 ? c_end - c_begin : n_step_blk;
-    /* four wavefronts a circuit while they are all resident (two such
-     * workgroups fit a compute unit's registers: 2 x 256), else one, of which
-     * eight fit.  Adders of 16 bits, ms with one / four: 64 circuits 127 / 97,
-     * 512 231 / 204; halves of 300 189 / 171, of 600 317 / 313, of 768 390 /
-     * 406, of 1024 615 / 660; a 101-stage ring alone 32.0 / 25.6 */
+    /* four wavefronts a circuit in launches of up to 512, else one.  Measured
+     * by the launch, of which a batch on two streams has two side by side (it
+     * is no bound on what is resident).  16-bit adders, ms with one / four:
+     * 64 circuits 127 / 97, 512 231 / 204; halves of 300 189 / 171, of 600 317
+     * / 313, of 768 390 / 406, of 1024 615 / 660.  Small circuits cross
+     * earlier: halves of 500 rings of 3 stages 13.7 / 14.9, of 11 17.1 / 18.7,
+     * of 1-bit adders 53.0 / 55.0, 500 of 3 bits 62.0 / 67.9, but 101 stages
+     * 32.8 / 29.7; halves of 256 are faster by four for all of them (3 stages
+     * 12.3 / 11.8, 1 bit 43.8 / 37.5).  A 101-stage ring alone 32.0 / 25.6. */
     const bool wide = ns <= 512;
     const dim3 g((unsigned)ns), wg(wide ? STEP_WIDE : ONE_WAVE);
     if (D0 && wide) hipLaunchKernelGGL(k_tran_step<true>, g, wg, lds_bytes, s, *D0, c_begin);
