@@ -1382,7 +1382,9 @@ ngmi_batch *ngmi_batch_new(ngmi_circuit *const *ckts, int C, const int *probe, i
      * (1500 3-bit adders) 76.0 / 80.3; 1.71 (512 rings of 75) 21.0 / 24.1;
      * 1.83 (200 5-bit adders) 53.7 / 50.6; 4.6 (256 1-bit adders) 47.7 / 37.0;
      * 21 (1000 rings of 3) 22.6 / 14.9; 64 (a 16-bit adder whose devices all
-     * differ) 95 / 38 */
+     * differ) 95 / 38.  Nor where the tiles (states, caches, columns, saved
+     * states) would take more than half of the device's free memory: a batch
+     * that fits without holes is not refused for them. */
     int64_t wp = 0, wd = 0;
     bool records = true, pad = true;
     std::vector<std::vector<const ngmi_circuit *>> cs(members.size());
@@ -1401,6 +1403,10 @@ ngmi_batch *ngmi_batch_new(ngmi_circuit *const *ckts, int C, const int *probe, i
         wp += (int64_t)G->C * (int64_t)(G->place.size() / MOS_TILE);
         wd += ((int64_t)G->C * G->NM + MOS_TILE - 1) / MOS_TILE;
     }
+    constexpr size_t TILE_BYTES = (size_t)MOS_TILE * 8 * ((NLEV + 1) * MOS_ROWS + B4C__COUNT + B4_NC_GEOM);
+    size_t room = 0, total = 0;
+    if (hipMemGetInfo(&room, &total) != hipSuccess) return bail("no device memory information");
+    pad = pad && (size_t)wp * TILE_BYTES <= room / 2;
     b->mos.mode = !records ? B4T_COLUMNS : pad && wp <= wd + 3 * wd / 4 ? B4T_UNIFORM : B4T_LANES;
     std::vector<TranDev> Ds;
     std::vector<B4Tab> tabs;
