@@ -944,6 +944,8 @@ int build_group(ngmi_batch *b, TopoGroup *G, const std::vector<const ngmi_circui
         vs_nodes(3 * (size_t)NVS), ic_nodes(NN + 1);
     for (int j = 0; j < NS; j++)
         for (int r = 0; r < 4 && at[j] >= 0; r++) mos_nodes[(size_t)r * NS + j] = c0.mos[at[j]].node[r];
+    std::vector<int> tile_n((NS + MOS_TILE - 1) / MOS_TILE, 0);
+    for (int j = 0; j < NS; j++) tile_n[j / MOS_TILE] += at[j] >= 0;
     for (int k = 0; k < NCAP; k++) {
         cap_nodes[k] = (int)c0.caps[k][0];
         cap_nodes[NCAP + k] = (int)c0.caps[k][1];
@@ -988,6 +990,7 @@ int build_group(ngmi_batch *b, TopoGroup *G, const std::vector<const ngmi_circui
     int4 *i4;
 #define UP(vec, field, T, tmp) do { if (upload<T>(b, vec, &tmp) != NGMI_OK) return fail(nullptr); D.field = tmp; } while (0)
     UP(mos_nodes, mos_nodes, int, ip);
+    UP(tile_n, tile_n, int, ip);
     UP(cap_nodes, cap_nodes, int, ip);
     UP(res_nodes, res_nodes, int, ip);
     UP(vs_nodes, vs_nodes, int, ip);

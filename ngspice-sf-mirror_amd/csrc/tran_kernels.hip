@@ -732,7 +732,8 @@ __device__ __forceinline__ double circuit_terr(const TranDev &D, const CktCtl *K
     }
     /* qb, qg and qd of each MOSFET (holes hold zeros, and bound nothing) */
     for (int j = threadIdx.x; j < D.NS; j += blockDim.x) {
-        const int drain = ((const NGMI_GLOBAL int *)D.mos_nodes)[j];
+        /* a wavefront has one tile */
+        const int live = D.W ? ((const NGMI_CONST int *)D.tile_n)[__builtin_amdgcn_readfirstlane(j / MOS_TILE)] : MOS_TILE;
         const NGMI_GLOBAL double *Q =
             (const NGMI_GLOBAL double *)D.mstate + mos_at((int64_t)c * D.NS + j, 0, B4X_qb);
         constexpr int lv = MOS_ROWS * MOS_TILE;
@@ -751,7 +752,7 @@ __device__ __forceinline__ double circuit_terr(const TranDev &D, const CktCtl *K
 #pragma unroll
         for (int r = 0; r < 3; r++) {
             const double t = terr_one(q0[r], q1[r], q2[r], q3[r], c0[r], c1[r], K, D);
-            if (drain >= 0) m = fmin(m, t);
+            if (j % MOS_TILE < live) m = fmin(m, t);
         }
     }
     return group_min(m);

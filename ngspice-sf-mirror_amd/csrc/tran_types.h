@@ -131,6 +131,7 @@ struct TranDev {
     double *bak_s;            /* [C][29 NS + 2 NCAP] CKTop's saved CKTstate0 */
     /* topology (shared) */
     const int *mos_nodes;     /* [4][NS] d g s b, -1 at a hole */
+    const int *tile_n;        /* [W] MOSFETs in each tile of a circuit, padded storage (its holes are last) */
     const int *cap_nodes;     /* [2][NCAP] */
     const int *res_nodes;     /* [2][NRES] */
     const int *vs_nodes;      /* [3][NVS] p n branch */
