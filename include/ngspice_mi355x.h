@@ -55,8 +55,8 @@ const char *ngmi_last_error(void);
  * "mos_waves" (0..4) set the occupancy the BSIM4 kernels' register
  * allocation targets for ngmi_bsim4_eval and the batched transient;
  * 3 and 4 run the 2-wave variant (more waves spilled); 0 (the default of
- * both) takes 2, or 1 for a launch whose instances fit
- * one wave per SIMD (a single small circuit: no spills, shorter latency);
+ * both) takes 2, or 1 for a launch whose workgroups (of up to 64 instances)
+ * fit one wave per SIMD (a single small circuit: no spills, shorter latency);
  * "streams" (1..4, default 2): with 2, a single-topology transient (with
  * the learned guess only when its network runs fused) alternates the two
  * halves of its circuits on two streams so one half's step kernel overlaps
